@@ -475,15 +475,14 @@ static int upload_transform(Engine<R>* ctx, int nx, int ny, double dx, Transform
 
 // ---- kernel dispatch over the compile-time column count ------------------------------------
 // Launch variants ("tile shapes") the autotuner chooses among, per kernel class: the pressure
-// solve of 2D 64-column CRMs has five (0: one instance per 4-wave workgroup, two workgroups per
-// CU, the gradient pass reading its inputs again; 1: one instance on 8 waves with every level's
-// inputs of the gradient pass kept in registers, one workgroup per CU; 2 and 3: variant 0 with
-// two or four levels of each pass unrolled together; 4: variant 0 with the Thomas factors in
-// registers, so that the workgroup needs only the slab of LDS), MPDATA six (0, 1: the default
-// or the other number of levels per trip; 2, 3: the same with registers bounded for three
-// waves per SIMD; 4, 5: the default sweep with each scalar on its own waves, registers
-// unbounded or bounded for three waves per SIMD).  Results are bitwise the same in every
-// variant of a class.
+// solve of 2D 64-column CRMs has five (0: chosen by the batch's size; 1: one instance on 8 waves
+// with every level's inputs of the gradient pass kept in registers, one workgroup per CU; 2 and
+// 3: one instance per 4-wave workgroup, two workgroups per CU, two or four levels of each pass
+// unrolled together; 4: the same, one level at a time, with the Thomas factors in registers, so
+// that the workgroup needs only the slab of LDS), MPDATA six (0: chosen by the batch's size; 1:
+// the other number of levels per trip; 2, 3: as the default and 1 with registers bounded for
+// three waves per SIMD; 4: the default number of levels, registers unbounded; 5: as 2).  Results
+// are bitwise the same in every variant of a class.
 static int variants_of(int kid, int nx, bool y3) {
   if (kid == CRM_K_PRESS) return (nx == 64 && !y3) ? 5 : 1;
   if (kid == CRM_K_MPDATA) return 6;
@@ -498,6 +497,10 @@ static void launch_press(int nzm, dim3 g, dim3 b, size_t sh, hipStream_t s, cons
   const bool z28 = nzm == 28, z58 = nzm == 58;
   const dim3 gi((unsigned)d.ncrms);
   if constexpr (NX == 64 && !G::Y3) {  // matrix-core transforms
+    // variant 0: the factors in registers once more instances wait than two workgroups per CU
+    // hold (4096 x 64 x 58: 590 -> 535 us FP64, 390 -> 345 mixed), else the 0 below (500 x 64 x
+    // 58: 75 against 78 us)
+    if (variant == 0 && d.ncrms > 512) variant = 4;
     if (!z28 && !z58) {
       k_press64<0, R, G><<<gi, b, press64_lds_bytes<0>(), s>>>(d, na, nb, nc);
     } else if (variant == 0) {  // one instance per 4-wave block
@@ -550,35 +553,119 @@ static void launch_press(int nzm, dim3 g, dim3 b, size_t sh, hipStream_t s, cons
   }
 }
 
+// o: where the advected fields go (their own buffers, or the hand-over buffers of split sweeps)
 template <int NX, typename R, typename G>
-static void launch_mpdata(dim3 g, dim3 b, hipStream_t s, const DevT<R>& d, int variant) {
+static void launch_mpdata(dim3 g, dim3 b, hipStream_t s, const DevT<R>& d, const Scalars<R>& o, bool split,
+                          int variant) {
   constexpr bool PAIR = (NX == 64 && !G::Y3);
-  if (variant == 1)
-    k_mpdata<NX, R, G, !PAIR><<<g, b, 0, s>>>(d);
-  else if (variant == 2)
-    k_mpdata_w3<NX, R, G, PAIR><<<g, b, 0, s>>>(d);
-  else if (variant == 3)
-    k_mpdata_w3<NX, R, G, !PAIR><<<g, b, 0, s>>>(d);
-  else if (variant == 4)
-    k_mpdata_split<NX, R, G, PAIR, false><<<dim3(g.x * 3), b, 0, s>>>(d, (int)g.x);
-  else if (variant == 5)
-    k_mpdata_split<NX, R, G, PAIR, true><<<dim3(g.x * 3), b, 0, s>>>(d, (int)g.x);
+  const bool other = variant == 1 || variant == 3;
+  const int nb = (int)g.x;
+  const bool many = PAIR && (size_t)nb * b.x >= (size_t)64 * 2048;
+  const bool w3 = variant == 0 ? many : variant == 2 || variant == 3 || variant == 5;
+  g.x *= 3;  // a grid per scalar
+  if (split)
+    k_mpdata<NX, R, G, PAIR, false, true><<<g, b, 0, s>>>(d, nb, o);
+  else if (w3 && other)
+    k_mpdata<NX, R, G, !PAIR, true, false><<<g, b, 0, s>>>(d, nb, o);
+  else if (w3)
+    k_mpdata<NX, R, G, PAIR, true, false><<<g, b, 0, s>>>(d, nb, o);
+  else if (other)
+    k_mpdata<NX, R, G, !PAIR, false, false><<<g, b, 0, s>>>(d, nb, o);
   else
-    k_mpdata<NX, R, G, PAIR><<<g, b, 0, s>>>(d);
+    k_mpdata<NX, R, G, PAIR, false, false><<<g, b, 0, s>>>(d, nb, o);
 }
 
 struct Launcher {
   int nx, nzm, ncrms;
   hipStream_t s;
   const int* block;  // threads per workgroup of each kernel class
+  bool split;        // the scalars are handed on through other buffers (mpdata, precip, diffuse)
   dim3 grid_inst(int b) const { return dim3((unsigned)((ncrms + b - 1) / b)); }
+  int waves() const { return (int)(((size_t)ncrms * nx + 63) / 64); }
+  // Chunks of levels of segment-kernel class kid (level_chunk, crm_kernels.hpp).  One sweep over
+  // all levels is a serial chain of nzm levels on a wave per 64 columns, so a batch that does not
+  // fill the device waits for that chain (16 x 32 x 28: 630 us of kernels a substep in 8 waves).
+  // A chunk adds a warm-up of 0 (k_pre, k_micro, k_stats), 1 (k_sgs, k_mom, k_diffuse), 5
+  // (k_precip) or 8 (k_mpdata) steps, so the sweeps are cut only as far as the chunks still find
+  // idle wave slots: to about `fill` waves in all, measured at 16 to 866 x 32 x 28, 256 x 128 x
+  // 58, 500 x 64 x 58, 1024 x 4 x 4 x 28 and 333 x 8 x 8 x 40 for fills of 1024 to 16384.
+  // k_micro's levels are independent and uneven (a cloudy level takes a Newton iteration and
+  // powers), so smaller pieces also balance a full device: 4096 x 64 x 58 FP64 568 us in one
+  // piece, 462 in two, 442 in four (mixed 293, 271, 243).
+  int chunks(int kid) const {
+    int fill, least;  // waves aimed at, fewest levels per chunk
+    switch (kid) {
+      case CRM_K_KURANT: fill = 4096, least = 2; break;
+      case CRM_K_PRE: fill = 2048, least = 2; break;
+      case CRM_K_SGS: fill = 2048, least = 2; break;
+      case CRM_K_MOM: fill = 3072, least = 2; break;
+      case CRM_K_MPDATA: fill = 1024, least = 4; break;  // waves per scalar
+      case CRM_K_PRECIP: fill = 2048, least = 4; break;
+      case CRM_K_DIFFUSE: fill = 4096, least = 2; break;
+      case CRM_K_MICRO: fill = std::max(8192, 4 * waves()), least = 1; break;
+      case CRM_K_STATS: fill = 2048, least = 2; break;
+      default: return 1;
+    }
+    if (!split && (kid == CRM_K_MPDATA || kid == CRM_K_PRECIP || kid == CRM_K_DIFFUSE)) return 1;
+    int n = std::max(1, std::min(fill / waves(), nzm / least));
+    // the chunks of k_precip are waves of one workgroup (of 512 threads at most)
+    if (kid == CRM_K_PRECIP && nx != 128) n = std::min(n, 8);
+    return n;
+  }
+  // From 1024 waves on, MPDATA and the sedimentation are not cut (chunks), and the scalars are
+  // updated in place (k_diffuse at 4096 x 64 x 58: 181 us from one buffer to another, 169 in place)
+  static bool split_batch(int ncrms, int columns) { return (size_t)ncrms * columns < (size_t)64 * 1024; }
   // threads per workgroup of segment-kernel class kid: 128-column instances span two waves
-  // whose exchanges are workgroup barriers, so they run one instance per workgroup
-  int bs(int kid) const { return nx == 128 ? 128 : block[kid]; }
+  // whose exchanges are workgroup barriers, so they run one instance per workgroup; a batch
+  // of fewer waves than the device has SIMDs is spread one wave per workgroup
+  int bs(int kid) const { return nx == 128 ? 128 : waves() < 1024 ? 64 : block[kid]; }
   // grid and workgroup of segment-kernel class kid
-  dim3 g(int kid) const { return dim3((unsigned)(((size_t)ncrms * nx + bs(kid) - 1) / bs(kid))); }
+  dim3 g(int kid) const {
+    return dim3((unsigned)(((size_t)ncrms * nx + bs(kid) - 1) / bs(kid)), (unsigned)chunks(kid));
+  }
   dim3 b(int kid) const { return dim3((unsigned)bs(kid)); }
 };
+
+template <int NX, typename R>
+static void launch_precip(const Launcher& L, const DevT<R>& d, R* tt, const R* qsrc, R* qdst, R* qx) {
+  const int n = L.chunks(CRM_K_PRECIP);
+  if constexpr (NX <= 64) {
+    if (n > 1) {
+      k_precip_wg<NX, R><<<dim3((unsigned)L.waves()), dim3(64 * n), 0, L.s>>>(d, tt, qsrc, qdst, qx);
+      return;
+    }
+  }
+  k_precip<NX, R><<<L.g(CRM_K_PRECIP), L.b(CRM_K_PRECIP), 0, L.s>>>(d, tt, qsrc, qdst, qx);
+}
+
+template <int NX, typename R>
+static void launch_pre(const Launcher& L, const DevT<R>& d, int na, const double* qrad) {
+  const dim3 g = L.g(CRM_K_PRE), b = L.b(CRM_K_PRE);
+  if (g.y == 1)
+    k_pre<NX, R, false><<<g, b, 0, L.s>>>(d, na, qrad);
+  else
+    k_pre<NX, R, true><<<g, b, 0, L.s>>>(d, na, qrad);
+}
+
+template <int NX, typename R, typename G>
+static void launch_diffuse(const Launcher& L, const DevT<R>& d, const Scalars<R>& src) {
+  const dim3 g = L.g(CRM_K_DIFFUSE), b = L.b(CRM_K_DIFFUSE);
+  if (L.split)
+    k_diffuse<NX, R, G, true><<<g, b, 0, L.s>>>(d, src);
+  else
+    k_diffuse<NX, R, G, false><<<g, b, 0, L.s>>>(d, src);
+}
+
+template <int NX, typename R>
+static void launch_stats(const Launcher& L, const DevT<R>& d) {
+  dim3 g = L.g(CRM_K_STATS);
+  if (g.y == 1) {
+    k_stats<NX, R, true><<<g, L.b(CRM_K_STATS), 0, L.s>>>(d);
+  } else {  // one more workgroup row for the water paths
+    g.y++;
+    k_stats<NX, R, false><<<g, L.b(CRM_K_STATS), 0, L.s>>>(d);
+  }
+}
 
 // NXV: columns per instance; GEO: the lane geometry (a 2D row of NXV columns, or the 8 x 8
 // or 4 x 4 columns of a 3D CRM; nx here counts nx*ny).
@@ -748,7 +835,11 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
   d.gmax = gmax;
   d.docoriolis = ctx->coriolis;
   host_constants(d);
-  Launcher L{nx, nzm, ncrms, s, ctx->block};
+  // a debug run that stops inside a substep reads the fields in their own buffers
+  Launcher L{nx, nzm, ncrms, s, ctx->block, phase_stop == 0 && Launcher::split_batch(ncrms, nx)};
+  // the advected scalars after MPDATA and after the sedimentation (Scalars, crm_kernels.hpp)
+  auto after_mpdata = [&]() { return L.split ? Scalars<R>{d.qcl, d.qci, d.qpl} : Scalars<R>{d.t, d.qt, d.qp}; };
+  auto after_precip = [&]() { return L.split ? Scalars<R>{d.qcl, d.qci, d.qpi} : Scalars<R>{d.t, d.qt, d.qp}; };
   const dim3 b256(256);
   ctx->last_ok = false;
   ctx->stats = crm_hip_stats{};
@@ -907,19 +998,19 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
           k_decide<<<1, 64, 0, s>>>(gmax, n, ctx->debug_stop);
           k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_FLAGS, d.stop);
           k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d);
-          NX_DISPATCH(nx, (k_pre<NXV, R><<<L.g(CRM_K_PRE), L.b(CRM_K_PRE), 0, s>>>(d, na, qrad)));
+          NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad)));
           NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
           NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
           NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, gpress, b256, press_lds, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
           k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
-          NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, ctx->variant[CRM_K_MPDATA])));
-          NX_DISPATCH(nx, (k_precip<NXV, R><<<L.g(CRM_K_PRECIP), L.b(CRM_K_PRECIP), 0, s>>>(d)));
+          NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA])));
+          NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp)));
         }
         std::swap(d.u, d.dudt[nc]);
         std::swap(d.w, d.dwdt[nc]);
         if (y3) std::swap(d.v, d.dvdt[nc]);
         if (launch) {
-          NX_DISPATCH(nx, (k_diffuse<NXV, R, GEO><<<L.g(CRM_K_DIFFUSE), L.b(CRM_K_DIFFUSE), 0, s>>>(d)));
+          NX_DISPATCH(nx, (launch_diffuse<NXV, R, GEO>(L, d, after_precip())));
           NX_DISPATCH(nx, (k_micro<NXV, R, true><<<L.g(CRM_K_MICRO), L.b(CRM_K_MICRO), 0, s>>>(d, 0)));
         }
         int nn = na;
@@ -927,7 +1018,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
         nc = nb;
         nb = nn;
         if (launch) {
-          NX_DISPATCH(nx, (k_stats<NXV, R><<<L.g(CRM_K_STATS), L.b(CRM_K_STATS), 0, s>>>(d)));
+          NX_DISPATCH(nx, (launch_stats<NXV, R>(L, d)));
         }
       }
     };
@@ -1018,23 +1109,23 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       const double* qrad = qrad_buf;
       auto body = [&]() {
         k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d);
-        NX_DISPATCH(nx, (k_pre<NXV, R><<<L.g(CRM_K_PRE), L.b(CRM_K_PRE), 0, s>>>(d, na, qrad)));
+        NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad)));
         NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
         NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
         NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, gpress, b256, press_lds, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
         k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
-        NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, ctx->variant[CRM_K_MPDATA])));
-        NX_DISPATCH(nx, (k_precip<NXV, R><<<L.g(CRM_K_PRECIP), L.b(CRM_K_PRECIP), 0, s>>>(d)));
+        NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA])));
+        NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp)));
         std::swap(d.u, d.dudt[nc]);
         std::swap(d.w, d.dwdt[nc]);
         if (y3) std::swap(d.v, d.dvdt[nc]);
-        NX_DISPATCH(nx, (k_diffuse<NXV, R, GEO><<<L.g(CRM_K_DIFFUSE), L.b(CRM_K_DIFFUSE), 0, s>>>(d)));
+        NX_DISPATCH(nx, (launch_diffuse<NXV, R, GEO>(L, d, after_precip())));
         NX_DISPATCH(nx, (k_micro<NXV, R><<<L.g(CRM_K_MICRO), L.b(CRM_K_MICRO), 0, s>>>(d, 0)));
         int nn = na;
         na = nc;
         nc = nb;
         nb = nn;
-        NX_DISPATCH(nx, (k_stats<NXV, R><<<L.g(CRM_K_STATS), L.b(CRM_K_STATS), 0, s>>>(d)));
+        NX_DISPATCH(nx, (launch_stats<NXV, R>(L, d)));
       };
       DevT<R> dk;  // the key: every kernel argument of the substep
       std::memcpy(&dk, &d, sizeof(d));
@@ -1082,7 +1173,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
         TIMED(CRM_K_PRECIP_INIT,
               (k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d)));
       const double* qrad = qrad_buf;
-      TIMED(CRM_K_PRE, NX_DISPATCH(nx, (k_pre<NXV, R><<<L.g(CRM_K_PRE), L.b(CRM_K_PRE), 0, s>>>(d, na, qrad))));
+      TIMED(CRM_K_PRE, NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad))));
       if (last && phase_stop == 7) goto stopped;
       TIMED(CRM_K_SGS, NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d))));
       if (last && phase_stop == 9) goto stopped;
@@ -1091,14 +1182,14 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       TIMED(CRM_K_PRESS, NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, gpress, b256, press_lds, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS]))));
       if (last && phase_stop == 13) goto stopped;
       k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
-      TIMED(CRM_K_MPDATA, NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, ctx->variant[CRM_K_MPDATA]))));
-      TIMED(CRM_K_PRECIP, NX_DISPATCH(nx, (k_precip<NXV, R><<<L.g(CRM_K_PRECIP), L.b(CRM_K_PRECIP), 0, s>>>(d))));
+      TIMED(CRM_K_MPDATA, NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA]))));
+      TIMED(CRM_K_PRECIP, NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp))));
       if (last && phase_stop == 15) goto stopped;
       std::swap(d.u, d.dudt[nc]);
       std::swap(d.w, d.dwdt[nc]);
       if (y3) std::swap(d.v, d.dvdt[nc]);
       if (last && phase_stop == 17) goto stopped;
-      TIMED(CRM_K_DIFFUSE, NX_DISPATCH(nx, (k_diffuse<NXV, R, GEO><<<L.g(CRM_K_DIFFUSE), L.b(CRM_K_DIFFUSE), 0, s>>>(d))));
+      TIMED(CRM_K_DIFFUSE, NX_DISPATCH(nx, (launch_diffuse<NXV, R, GEO>(L, d, after_precip()))));
       if (last && phase_stop == 18) goto stopped;
       {
         const int accel = (acc && !ceased) ? 1 : 0;
@@ -1116,7 +1207,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       nc = nb;
       nb = nn;
     }
-    TIMED(CRM_K_STATS, NX_DISPATCH(nx, (k_stats<NXV, R><<<L.g(CRM_K_STATS), L.b(CRM_K_STATS), 0, s>>>(d))));
+    TIMED(CRM_K_STATS, NX_DISPATCH(nx, (launch_stats<NXV, R>(L, d))));
     HIPCHECK(hipGetLastError());
   }
   ctx->stats.nstop = nstop;

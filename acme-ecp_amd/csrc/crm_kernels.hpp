@@ -27,6 +27,18 @@ namespace CRM_NS {
 #define CRM_STOP_CHECK(d) \
   if ((d).stop && *(const volatile unsigned long long*)(d).stop) return
 
+// A sweep's levels are dealt to the gridDim.y workgroups of its instances in contiguous chunks:
+// level_chunk gives the chunk [k0, k1) of n levels that this workgroup computes and stores.  A
+// chunk that does not start at level 0 first runs the few levels below it that its carried
+// values come from, without storing them, so every level's arithmetic (and its bits) is that of
+// one sweep over all levels.
+struct LevelChunk {
+  int k0, k1;
+};
+__device__ __forceinline__ LevelChunk level_chunk(int n) {
+  return {(int)((unsigned)n * blockIdx.y / gridDim.y), (int)((unsigned)n * (blockIdx.y + 1) / gridDim.y)};
+}
+
 // Clears KURANT_SLOTS slots of the batch-global maxima (a kernel rather than a memset, so that
 // it can sit in a captured graph); launched with at least KURANT_SLOTS threads.
 __global__ void k_clear_u64(unsigned long long* p, const unsigned long long* stop) {
@@ -434,8 +446,9 @@ __global__ void CRM_LB k_kurant(DevT<R> d) {
   auto U = [&](int k) { return (double)d.u[((size_t)c * nzm + k) * NX + i]; };
   auto V = [&](int k) { return y3 ? (double)d.v[((size_t)c * nzm + k) * NX + i] : 0.0; };
   auto T = [&](int k) { return (double)d.tkh[((size_t)c * nzm + k) * NX + i]; };
+  const LevelChunk ch = level_chunk(nzm);
 #pragma unroll 4
-  for (int k = 0; k < nzm; k++) {
+  for (int k = ch.k0; k < ch.k1; k++) {
     const double uu = U(k), vv = V(k), tkh = T(k);
     // the lid's w counts as zero (the reference's loop stops below it)
     const double wm = fabs(W(k)), wm_up = k + 1 < nzm ? fabs(W(k + 1)) : 0.0;
@@ -454,7 +467,9 @@ __global__ void CRM_LB k_kurant(DevT<R> d) {
 // zero.F90:8-25, buoyancy.F90:7-38, forcing.F90:7-79, crm_module.F90:766-777,
 // damping.F90:9-117, ice_fall.F90:6-173.  Writes dudt(na), dwdt(na) from scratch.
 // ------------------------------------------------------------------------------------------
-template <int NX, typename R>
+// CHUNKS: the levels dealt to gridDim.y chunks; with a run-time range the one sweep of a large
+// batch measured 5% slower (4096 x 64 x 58: 389 -> 410 us)
+template <int NX, typename R, bool CHUNKS>
 __global__ void CRM_LB k_pre(DevT<R> d, int na, const double* qrad) {
   CRM_STOP_CHECK(d);
   SegFor<NX> s;
@@ -502,12 +517,15 @@ __global__ void CRM_LB k_pre(DevT<R> d, int na, const double* qrad) {
   // one the flux uses): the flux icefz(k+1) needs all three, so they are read at least one
   // level ahead, and level k+3 is read at the top of level k.  Vector loads complete in issue
   // order, so a read of this level issued after the prefetch of the next would wait for it.
-  R qi0 = F(d.qci, 0), qi1 = F(d.qci, ::min(1, nzm - 1)), qi2 = F(d.qci, ::min(2, nzm - 1));
+  const LevelChunk ch = CHUNKS ? level_chunk(nzm) : LevelChunk{0, nzm};
+  const int k0 = ch.k0, k1 = ch.k1, kb0 = ::max(k0 - 1, 0);
+  R qi0 = F(d.qci, k0), qi1 = F(d.qci, ::min(k0 + 1, nzm - 1)), qi2 = F(d.qci, ::min(k0 + 2, nzm - 1));
   // the surface precipitation the ice flux adds to at level 0, read before the sweep's loads
   const double psfc0 = d.precsfc[(size_t)c * NX + i], pssfc0 = d.precssfc[(size_t)c * NX + i];
-  R fz_k = icefz(0, qi0, qi0, qi1);
-  // level k-1 thermodynamics for the buoyancy average
-  R pb_tabs = 0, pb_qv = 0, pb_qcl = 0, pb_qci = 0, pb_qpl = 0, pb_qpi = 0;
+  // level k-1 thermodynamics for the buoyancy average (not used at level 0)
+  R pb_tabs = F(d.tabs, kb0), pb_qv = F(d.qv, kb0), pb_qcl = F(d.qcl, kb0), pb_qci = F(d.qci, kb0);
+  R pb_qpl = F(d.qpl, kb0), pb_qpi = F(d.qpi, kb0);
+  R fz_k = icefz(k0, pb_qci, qi0, qi1);
   // the fields of one level, read one level ahead of their use
   struct Lvl {
     R tabs, qv, qcl, qpl, qpi, u, w, t, qt, v;
@@ -528,7 +546,7 @@ __global__ void CRM_LB k_pre(DevT<R> d, int na, const double* qrad) {
     L.qr = qrad[((size_t)c * nzm + k) * nxr + ir];  // [instance][level][radiation column]
   };
   Lvl nxt;
-  load(0, nxt);
+  load(k0, nxt);
   // the results of a level are stored at the top of the next one, before its reads: vector
   // memory operations complete in issue order, so the wait for the reads at the end of a
   // level then never includes stores issued after them
@@ -541,9 +559,9 @@ __global__ void CRM_LB k_pre(DevT<R> d, int na, const double* qrad) {
     if (y3) d.dvdt[na][o] = st_dv;
     dwdt[((size_t)c * nz + k) * NX + i] = st_dw;
   };
-  for (int k = 0; k < nzm; k++) {
+  for (int k = k0; k < k1; k++) {
     const Lvl L = nxt;
-    if (k > 0 && live) store_level(k - 1);
+    if (k > k0 && live) store_level(k - 1);
     // clamped at the top, where the record is not used again: an unconditional load needs no
     // copy that waits for earlier loads
     load(::min(k + 1, nzm - 1), nxt);
@@ -623,8 +641,8 @@ __global__ void CRM_LB k_pre(DevT<R> d, int na, const double* qrad) {
     st_dw = dw;
   }
   if (live) {
-    store_level(nzm - 1);
-    dwdt[((size_t)c * nz + nzm) * NX + i] = R(0.0);
+    store_level(k1 - 1);
+    if (k1 == nzm) dwdt[((size_t)c * nz + nzm) * NX + i] = R(0.0);
   }
 }
 
@@ -698,24 +716,29 @@ __global__ void CRM_LB k_sgs(DevT<R> d) {
   const R Ce = Ck * Ck * Ck / (Cs * Cs * Cs * Cs);
   auto F = [&](const R* p, int k) { return p[((size_t)c * nzm + k) * NX + i]; };
   auto W = [&](int k) { return d.w[((size_t)c * nz + k) * NX + i]; };
+  // a chunk above the surface starts one level below it, for the buoyancy flux bsv_prev
+  const LevelChunk ch = level_chunk(nzm - 1);
+  const int ks = ::max(ch.k0 - 1, 0), km = ::max(ks - 1, 0);
   // window: u (and v in 3D) at k-1,k,k+1 and w at k,k+1
-  R um = 0, u = F(d.u, 0), up = F(d.u, 1);
+  R um = F(d.u, km), u = F(d.u, ks), up = F(d.u, ks + 1);
   R vm = 0, v = 0, vp = 0;
   const cprof<R> v0 = profc(d, P_V0, c);
   if constexpr (G::Y3) {
-    v = F(d.v, 0);
-    vp = F(d.v, 1);
+    vm = F(d.v, km);
+    v = F(d.v, ks);
+    vp = F(d.v, ks + 1);
   }
-  R w0 = W(0), w1 = W(1);
+  R w0 = W(ks), w1 = W(ks + 1);
   R bsv_prev = R(0.0);
   // thermodynamics at k (carried) and k+1; level k+2 and tk at k+1 are read one iteration
   // ahead of their use
-  R th_tabs = F(d.tabs, 0), th_qcl = F(d.qcl, 0), th_qci = F(d.qci, 0), th_qv = F(d.qv, 0);
-  R th_qpl = F(d.qpl, 0), th_qpi = F(d.qpi, 0), th_t = F(d.t, 0);
-  R nx_tabs = F(d.tabs, 1), nx_qcl = F(d.qcl, 1), nx_qci = F(d.qci, 1), nx_qv = F(d.qv, 1);
-  R nx_qpl = F(d.qpl, 1), nx_qpi = F(d.qpi, 1), nx_t = F(d.t, 1);
-  R tk_cur = F(d.tk, 0);
-  for (int k = 0; k < nzm - 1; k++) {
+  const int kn0 = ks + 1;
+  R th_tabs = F(d.tabs, ks), th_qcl = F(d.qcl, ks), th_qci = F(d.qci, ks), th_qv = F(d.qv, ks);
+  R th_qpl = F(d.qpl, ks), th_qpi = F(d.qpi, ks), th_t = F(d.t, ks);
+  R nx_tabs = F(d.tabs, kn0), nx_qcl = F(d.qcl, kn0), nx_qci = F(d.qci, kn0), nx_qv = F(d.qv, kn0);
+  R nx_qpl = F(d.qpl, kn0), nx_qpi = F(d.qpi, kn0), nx_t = F(d.t, kn0);
+  R tk_cur = F(d.tk, ks);
+  for (int k = ks; k < ch.k1; k++) {
     int kc = k + 1, kb = k - 1;
     const R n_tabs = nx_tabs, n_qcl = nx_qcl, n_qci = nx_qci, n_qv = nx_qv, n_qpl = nx_qpl, n_qpi = nx_qpi;
     const R n_t = nx_t, tk_k = tk_cur;
@@ -810,7 +833,7 @@ __global__ void CRM_LB k_sgs(DevT<R> d) {
       R tk = sqrt(Ck * Ck * Ck / Cee * fmax(R(0.0), def2 - Pr * buoy)) * (smix * smix);
       R tt = tk / (Ck * smix);
       tk = fmin(tk, tkmax);
-      if (live) {
+      if (live && k >= ch.k0) {
         d.tke[o] = tt * tt;
         d.tk[o] = tk;
         d.tkh[o] = Pr * tk;
@@ -859,9 +882,13 @@ __device__ __forceinline__ void mom2(const DevT<R>& d, int na) {
   const R rdz = R(1.) / dz, dzx = dz / dx;
   auto F = [&](const R* p, int k) { return p[((size_t)c * nzm + k) * NX + i]; };
   auto W = [&](int k) { return d.w[((size_t)c * nz + k) * NX + i]; };
-  R u_k = F(d.u, 0), u_n = F(d.u, 1);
-  R w_k = W(0), w_n = W(1);
-  R tk_k = F(d.tk, 0), tk_n = F(d.tk, 1);
+  // a chunk above the surface starts one level below it, for the fluxes at its bottom and the
+  // horizontal contributions to its first w level
+  const LevelChunk ch = level_chunk(nzm);
+  const int ks = ::max(ch.k0 - 1, 0);
+  R u_k = F(d.u, ks), u_n = F(d.u, ks + 1);
+  R w_k = W(ks), w_n = W(ks + 1);
+  R tk_k = F(d.tk, ks), tk_n = F(d.tk, ks + 1);
   R fuz_k = R(0.0);    // fuz at level k (0 at the surface)
   R fwz_prev = R(0.0); // fwz(k-1)
   R fuv_k = R(0.0);    // vertical SGS u flux at the bottom of level k
@@ -869,9 +896,10 @@ __device__ __forceinline__ void mom2(const DevT<R>& d, int na) {
   R pend_adv = R(0.0), pend_dif = R(0.0);  // horizontal contributions for w level k
   R uwsb_sum = R(0.0);
   // tendencies of the next level, read one iteration ahead
-  R du_pre = dudt[((size_t)c * nzm) * NX + i];
-  R dw_pre = dwdt[((size_t)c * nz + 1) * NX + i];
-  for (int k = 0; k < nzm; k++) {
+  R du_pre = dudt[((size_t)c * nzm + ks) * NX + i];
+  R dw_pre = dwdt[((size_t)c * nz + ::max(ks, 1)) * NX + i];
+  for (int k = ks; k < ch.k1; k++) {
+    const bool store = live && k >= ch.k0;
     int kn = k + 1;
     bool has_n = kn < nzm;
     int kcu = has_n ? kn : k;
@@ -919,18 +947,22 @@ __device__ __forceinline__ void mom2(const DevT<R>& d, int na) {
       tkz = rdz25 * (tk_k + tk_m + tk_n + tkn_m);
       fuv_n = -tkz * ((u_n - u_k) * iadzw + (w_n - wn_m) * dzx) * rhow[kn];
       uwsb_sum = s.sum(fuv_n);
-      if (live && i == 0) prof(d, P_UWSB, c)[kn] = uwsb_sum;
+      if (store && i == 0) prof(d, P_UWSB, c)[kn] = uwsb_sum;
     } else {
       R rdz2 = rdz * rdz * R(1.0);
       R tkz = rdz2 * R(1.0) * tk_k;
       fwv_n = -R(2.) * tkz * (w_n - w_k) / adz[k] * rho[k];
     }
     du = du - (fuv_n - fuv_k) * rhoi_k;
-    if (live) dudt[o] = du;
+    if (store) dudt[o] = du;
     R fuz_sum = s.sum(fuz_n);
-    if (has_n && live && i == 0) prof(d, P_UWLE, c)[kn] = fuz_sum;
+    if (has_n && store && i == 0) prof(d, P_UWLE, c)[kn] = fuz_sum;
     // ---- dwdt(k) for w levels 1..nzm-1
-    R fwz_k = dz25 * (w_n * rhow[kn] + w_k * rhow[k]) * (w_n + w_k);
+    // which of the two products is rounded by itself is spelled out (the other one joins the
+    // addition), so that the bits do not hang on how the compiler arranges the sweep
+    constexpr bool KEEP_N = NX == 128 || (sizeof(R) == 4 && NX != 32);
+    const R wr = KEEP_N ? fma(w_k, (R)rhow[k], w_n * rhow[kn]) : fma(w_n, (R)rhow[kn], w_k * rhow[k]);
+    R fwz_k = dz25 * wr * (w_n + w_k);
     if (k >= 1) {
       size_t ow = ((size_t)c * nz + k) * NX + i;
       R dw = dw_k;
@@ -939,7 +971,7 @@ __device__ __forceinline__ void mom2(const DevT<R>& d, int na) {
       dw = dw - (fwz_k - fwz_prev) * rhoiw;
       dw = dw - pend_dif;
       dw = dw - (fwv_n - fwv_k) * rhoiw;
-      if (live) dwdt[ow] = dw;
+      if (store) dwdt[ow] = dw;
     }
     // ---- horizontal contributions to w level k+1 (applied next iteration)
     {
@@ -965,16 +997,16 @@ __device__ __forceinline__ void mom2(const DevT<R>& d, int na) {
     tk_n = tk_nn;
   }
   // lid (w level nzm): horizontal contributions only
-  if (live) {
+  if (live && ch.k1 == nzm) {
     size_t ow = ((size_t)c * nz + nzm) * NX + i;
     R dw = dwdt[ow];
     dw = dw - pend_adv;
     dw = dw - pend_dif;
     dwdt[ow] = dw;
-    if (i == 0) {
-      prof(d, P_UWLE, c)[0] = R(0.0);
-      prof(d, P_UWSB, c)[0] = R(0.0);
-    }
+  }
+  if (live && ch.k0 == 0 && i == 0) {
+    prof(d, P_UWLE, c)[0] = R(0.0);
+    prof(d, P_UWSB, c)[0] = R(0.0);
   }
 }
 
@@ -1002,19 +1034,22 @@ __device__ __forceinline__ void mom3(const DevT<R>& d, int na) {
   const R rdz = R(1.) / dz, dzx = dz / dx, dxy = dx / dx;
   auto F = [&](const R* p, int k) { return p[((size_t)c * nzm + k) * NX + i]; };
   auto W = [&](int k) { return d.w[((size_t)c * nz + k) * NX + i]; };
-  R u_k = F(d.u, 0), u_n = F(d.u, 1);
-  R v_k = F(d.v, 0), v_n = F(d.v, 1);
-  R w_k = W(0), w_n = W(1);
-  R tk_k = F(d.tk, 0), tk_n = F(d.tk, 1);
+  const LevelChunk ch = level_chunk(nzm);  // as in mom2
+  const int ks = ::max(ch.k0 - 1, 0);
+  R u_k = F(d.u, ks), u_n = F(d.u, ks + 1);
+  R v_k = F(d.v, ks), v_n = F(d.v, ks + 1);
+  R w_k = W(ks), w_n = W(ks + 1);
+  R tk_k = F(d.tk, ks), tk_n = F(d.tk, ks + 1);
   R fuz_k = R(0.0), fvz_k = R(0.0);  // vertical advective fluxes at the bottom of level k
   R fwz_prev = R(0.0);
   R fuv_k = R(0.0), fvv_k = R(0.0);  // vertical SGS fluxes at the bottom of level k
   R fwv_k = R(0.0);
   R pax = R(0.0), pay = R(0.0), pdx = R(0.0), pdy = R(0.0);  // horizontal terms for w level k
   // tendencies of the next level, read one iteration ahead
-  R du_pre = dudt[((size_t)c * nzm) * NX + i], dv_pre = dvdt[((size_t)c * nzm) * NX + i];
-  R dw_pre = dwdt[((size_t)c * nz + 1) * NX + i];
-  for (int k = 0; k < nzm; k++) {
+  R du_pre = dudt[((size_t)c * nzm + ks) * NX + i], dv_pre = dvdt[((size_t)c * nzm + ks) * NX + i];
+  R dw_pre = dwdt[((size_t)c * nz + ::max(ks, 1)) * NX + i];
+  for (int k = ks; k < ch.k1; k++) {
+    const bool store = live && k >= ch.k0;
     const int kn = k + 1;
     const bool has_n = kn < nzm;
     const int kcu = has_n ? kn : k;
@@ -1057,7 +1092,7 @@ __device__ __forceinline__ void mom3(const DevT<R>& d, int na) {
       tkz = rdz25 * (tk_k + tk_jm + tk_n + tkn_jm);
       fvv_n = -tkz * ((v_n - v_k) * iadzw + (w_n - wn_jm) * dzx) * rhow[kn];
       R s_uwle = s.sum(fuz_n), s_vwle = s.sum(fvz_n), s_uwsb = s.sum(fuv_n), s_vwsb = s.sum(fvv_n);
-      if (live && i == 0) {
+      if (store && i == 0) {
         prof(d, P_UWLE, c)[kn] = s_uwle;
         prof(d, P_VWLE, c)[kn] = s_vwle;
         prof(d, P_UWSB, c)[kn] = s_uwsb;
@@ -1112,7 +1147,7 @@ __device__ __forceinline__ void mom3(const DevT<R>& d, int na) {
       const R u_av = R(0.25) * (u_k + u_p + u_jm + u_p_jm);
       dv = dv - R(0.5) * (fcor + fcor) * (u_av - (R)prof(d, P_UG0, c)[k]);
     }
-    if (live) {
+    if (store) {
       dudt[o] = du;
       dvdt[o] = dv;
     }
@@ -1128,7 +1163,7 @@ __device__ __forceinline__ void mom3(const DevT<R>& d, int na) {
       dw = dw - pdx;
       dw = dw - pdy;
       dw = dw - (fwv_n - fwv_k) * rhoiw;
-      if (live) dwdt[ow] = dw;
+      if (store) dwdt[ow] = dw;
     }
     // ---- horizontal terms of w level k+1 (applied next iteration)
     {
@@ -1163,7 +1198,7 @@ __device__ __forceinline__ void mom3(const DevT<R>& d, int na) {
     tk_n = tk_nn;
   }
   // lid (w level nzm): horizontal terms only
-  if (live) {
+  if (live && ch.k1 == nzm) {
     size_t ow = ((size_t)c * nz + nzm) * NX + i;
     R dw = dwdt[ow];
     dw = dw - pax;
@@ -1171,12 +1206,12 @@ __device__ __forceinline__ void mom3(const DevT<R>& d, int na) {
     dw = dw - pdx;
     dw = dw - pdy;
     dwdt[ow] = dw;
-    if (i == 0) {
-      prof(d, P_UWLE, c)[0] = R(0.0);
-      prof(d, P_UWSB, c)[0] = R(0.0);
-      prof(d, P_VWLE, c)[0] = R(0.0);
-      prof(d, P_VWSB, c)[0] = R(0.0);
-    }
+  }
+  if (live && ch.k0 == 0 && i == 0) {
+    prof(d, P_UWLE, c)[0] = R(0.0);
+    prof(d, P_UWSB, c)[0] = R(0.0);
+    prof(d, P_VWLE, c)[0] = R(0.0);
+    prof(d, P_VWSB, c)[0] = R(0.0);
   }
 }
 
@@ -2040,16 +2075,29 @@ __device__ __forceinline__ float term_vel_bound(const TermVel& tv, double q, dou
   return v;
 }
 
-// One scalar of MPDATA, software-pipelined over levels.  At iteration K stage s works on
+// Where the advected scalars t, qt and qp are kept between MPDATA and the SGS diffusion.  A sweep
+// whose levels are dealt to several workgroups cannot update a field in place (a neighbouring
+// chunk may still read the old value), so the three sweeps then hand the fields on through the
+// buffers of qcl, qci, qpl, qpi and qv, which hold nothing there: they are last read by k_sgs and
+// rewritten by k_micro.
+template <typename R>
+struct Scalars {
+  R *t, *qt, *qp;
+};
+
+// One scalar of MPDATA, software-pipelined over levels, from f to fout (the same buffer, or one
+// no chunk reads).  At iteration K stage s works on
 // level K-s; ring variables are named by how far behind the front they are at the top of the
 // iteration.  Statistics: fadv (advect_scalar.F90:62-72) and the vertical flux of
 // advect_scalar2D.F90:113-118,204-206.  With want_cfl, also the precipitation Courant number
 // of precip_fall (microphysics.F90:596-611) on the advected field.
 // PAIR: the steady state advances two levels per trip (the launch variant the autotuner may
 // choose; the default for the 2D 64-column segment)
-template <int NX, typename R, typename G, bool PAIR>
-__device__ void mpdata_one(const DevT<R>& d, const G& s, int c, bool live, R* f, double* fadv,
-                           double* flux, bool want_cfl) {
+// CHUNKS: the levels dealt to gridDim.y chunks, the result in another buffer (else in place)
+template <int NX, typename R, typename G, bool PAIR, bool CHUNKS>
+__device__ __forceinline__ void mpdata_one(const DevT<R>& d, const G& s, int c, bool live, R* f, R* to, double* fadv,
+                                           double* flux, bool want_cfl) {
+  R* const fout = CHUNKS ? to : f;
   constexpr bool Y3 = G::Y3;  // 3D: advect_scalar3D.F90:8-349 (dy == dx)
   const int nzm = d.nzm, nz = d.nz, i = s.i;
   const cprof<R> adz = profc(d, P_ADZ, c);
@@ -2065,13 +2113,18 @@ __device__ void mpdata_one(const DevT<R>& d, const G& s, int c, bool live, R* f,
   const R dz = inst(d, I_DZ, c);
   R pcfl = R(0.0);
   R f_0 = 0, f_1 = 0, f_2 = 0, f_3 = 0, f_4 = 0, f_5 = 0;
+  // the new value of a level depends on the field up to three levels away: a chunk above the
+  // surface starts three levels below it, and what the stages make of the levels below that
+  // (from the rings' zeros) reaches none of the levels it stores
+  const LevelChunk ch = CHUNKS ? level_chunk(nzm) : LevelChunk{0, nzm};
+  const int k0 = ch.k0, k1 = ch.k1, ks = ::max(k0 - 3, 0);
   // inputs of the next two levels, loaded two iterations before use
-  R nf1 = F(f, 0), nu1 = F(d.u, 0), nw1 = Wv(0);
-  R nf2 = F(f, 1), nu2 = F(d.u, 1), nw2 = Wv(1);
+  R nf1 = F(f, ks), nu1 = F(d.u, ks), nw1 = Wv(ks);
+  R nf2 = F(f, ks + 1), nu2 = F(d.u, ks + 1), nw2 = Wv(ks + 1);
   R nv1 = 0, nv2 = 0;
   if constexpr (Y3) {
-    nv1 = F(d.v, 0);
-    nv2 = F(d.v, 1);
+    nv1 = F(d.v, ks);
+    nv2 = F(d.v, ks + 1);
   }
   R V_0 = 0, V_1 = 0, V_2 = 0, V_3 = 0;
   R vv1_0 = 0, vv1_1 = 0, vv2_a = 0, vv2_b = 0, vv3_a = 0;
@@ -2091,9 +2144,12 @@ __device__ void mpdata_one(const DevT<R>& d, const G& s, int c, bool live, R* f,
   // prefetch issued before it: vector loads complete in issue order)
   R s1_a = 0, s1_b = 0, s1_c = 0;
   // One pipeline step; ST: steady state (5 <= K < nzm), where every stage is active and every
-  // boundary case is the interior one, so the guards and level selects fold away.
-  auto step = [&](const int K, auto steady) {
-    constexpr bool ST = decltype(steady)::value;
+  // boundary case is the interior one, so the guards and level selects fold away.  MODE 2 is the
+  // steady state of the levels below an upper chunk, whose last stage has nothing to store.
+  // (inlined at every call: as a function, its rings would live in memory)
+  auto step = [&](const int K, auto mode) __attribute__((always_inline)) {
+    constexpr int MODE = decltype(mode)::value;
+    constexpr bool ST = MODE != 0;
     const R cf = nf1, cu = nu1, cw = nw1, cv = nv1;
     nf1 = nf2;
     nu1 = nu2;
@@ -2223,12 +2279,12 @@ __device__ void mpdata_one(const DevT<R>& d, const G& s, int c, bool live, R* f,
       }
       if (flux) {
         R s3 = s.sum(ww3_new);
-        if (live && i == 0) flux[L4] = (double)s1_c + s3;
+        if (live && i == 0 && (!CHUNKS || (L4 >= k0 && L4 < k1))) flux[L4] = (double)s1_c + s3;
       }
     }
     // stage 5: corrected update at level K-5
     const int L5 = K - 5;
-    if (ST || (L5 >= 0 && L5 < nzm)) {
+    if (MODE == 1 || (MODE == 0 && L5 >= k0 && L5 < nzm)) {
       R ww3up = (ST || L5 + 1 < nzm) ? ww3_new : R(0.0);
       R fn;
       if constexpr (Y3)
@@ -2238,7 +2294,7 @@ __device__ void mpdata_one(const DevT<R>& d, const G& s, int c, bool live, R* f,
       size_t o = ((size_t)c * nzm + L5) * NX + i;
       R adv = s.sum(fn - f_5);
       if (live) {
-        f[o] = fn;
+        fout[o] = fn;
         if (fadv && i == 0) fadv[L5] = adv;
       }
       if (want_cfl) {
@@ -2303,61 +2359,46 @@ __device__ void mpdata_one(const DevT<R>& d, const G& s, int c, bool live, R* f,
     s1_b = s1_a;
     s1_a = s1_new;
   };
-  int K = 0;
+  int K = ks;
+  const int kend = k1 + 4, kst = CHUNKS ? ::min(nzm, k1 + 5) : nzm;  // last step; end of the steady state
   // Peeled into fill, steady state and drain.  FP64 issues every instruction it keeps
   // (measured 27% faster peeled).  The FP32 sweep was measured faster as one loop until the
   // prefetch became unconditional; peeled since (2D 64-column 18% faster, the uneven classes
   // 4%).
-  for (; K < 5 && K <= nzm + 4; K++) step(K, std::false_type{});
+  using Edge = std::integral_constant<int, 0>;
+  using Steady = std::integral_constant<int, 1>;
+  using Below = std::integral_constant<int, 2>;
+  for (; K < 5 && K <= kend; K++) step(K, Edge{});
+  if constexpr (CHUNKS)
+    for (; K < k0 + 5 && K < kst; K++) step(K, Below{});
   // two levels per trip: fewer of the prefetched values are copied along the ring before
   // their use (a copy waits for its load); with the unconditional prefetch, measured 8%
   // faster at 64 x 58.  The other shapes hold more per lane and spilled more with it (the
   // uneven classes measured slower), so there it is the alternative variant
   if constexpr (PAIR) {
-    for (; K + 1 < nzm; K += 2) {
-      step(K, std::true_type{});
-      step(K + 1, std::true_type{});
+    for (; K + 1 < kst; K += 2) {
+      step(K, Steady{});
+      step(K + 1, Steady{});
     }
   }
-  for (; K < nzm; K++) step(K, std::true_type{});
-  for (; K <= nzm + 4; K++) step(K, std::false_type{});
+  for (; K < kst; K++) step(K, Steady{});
+  for (; K <= kend; K++) step(K, Edge{});
   if (want_cfl) {
     pcfl = s.max(pcfl);
     if (live && i == 0) atomic_max_nonneg(&d.gmax[GMAX_PCFL + (c % KURANT_SLOTS) * KURANT_STRIDE], pcfl);
   }
 }
 
-// advect_all_scalars.F90:7-94: t, then the two microphysics fields.
-template <int NX, typename R, typename G, bool PAIR>
-__device__ __forceinline__ void mpdata_all(const DevT<R>& d) {
-  G s;
-  int c;
-  bool live = seg_instance<NX>(d.ncrms, c);
-  mpdata_one<NX, R, G, PAIR>(d, s, c, live, d.t, nullptr, nullptr, false);
-  mpdata_one<NX, R, G, PAIR>(d, s, c, live, d.qt, prof(d, P_MKADV1, c), prof(d, P_MKWLE1, c), false);
-  mpdata_one<NX, R, G, PAIR>(d, s, c, live, d.qp, prof(d, P_MKADV2, c), prof(d, P_MKWLE2, c), true);
-}
-template <int NX, typename R, typename G = SegFor<NX>, bool PAIR = (NX == 64 && !G::Y3)>
-__global__ void CRM_LB k_mpdata(DevT<R> d) {
-  CRM_STOP_CHECK(d);
-  mpdata_all<NX, R, G, PAIR>(d);
-}
-// The same sweep with its registers bounded for three waves per SIMD (168 VGPRs; what does not
-// fit is spilled): more waves to hide latency at the cost of the spills (launch variants)
-template <int NX, typename R, typename G = SegFor<NX>, bool PAIR = (NX == 64 && !G::Y3)>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_mpdata_w3(DevT<R> d) {
-  CRM_STOP_CHECK(d);
-  mpdata_all<NX, R, G, PAIR>(d);
-}
-// The three scalars on separate waves (launch variants): the grid is three copies of the
-// one-scalar grid of nb blocks, qp (the longest sweep, with its Courant number) first, then
-// qt, then t.  The scalars are independent (each writes only its own field and statistics),
-// so the results are those of the sequential sweep; the GPU holds three times as many sweeps,
-// and a SIMD whose registers admit fewer waves than it has instances no longer ends with one
-// wave running its three sweeps alone.
-template <int NX, typename R, typename G = SegFor<NX>, bool PAIR = (NX == 64 && !G::Y3), bool W3 = false>
+// advect_all_scalars.F90:7-94: t and the two microphysics fields, each scalar on its own waves:
+// the grid's x dimension is three copies of the one-scalar grid of nb blocks, qp (the longest
+// sweep, with its Courant number) first, then qt, then t.  The scalars are independent (each
+// writes only its own field and statistics).
+// PAIR: two levels per trip of the steady state; W3: the registers bounded for three waves per
+// SIMD (168 VGPRs; what does not fit is spilled), more waves to hide latency at the cost of the
+// spills.
+template <int NX, typename R, typename G, bool PAIR, bool W3, bool CHUNKS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W3 ? 3 : CRM_WAVES_PER_EU)))
-k_mpdata_split(DevT<R> d, int nb) {
+k_mpdata(DevT<R> d, int nb, Scalars<R> o) {
   CRM_STOP_CHECK(d);
   G s;
   const int scalar = (int)blockIdx.x / nb, bl = (int)blockIdx.x % nb;
@@ -2366,11 +2407,11 @@ k_mpdata_split(DevT<R> d, int nb) {
   const int c = g < d.ncrms ? g : d.ncrms - 1;
   const bool live = g < d.ncrms;
   if (scalar == 0)
-    mpdata_one<NX, R, G, PAIR>(d, s, c, live, d.qp, prof(d, P_MKADV2, c), prof(d, P_MKWLE2, c), true);
+    mpdata_one<NX, R, G, PAIR, CHUNKS>(d, s, c, live, d.qp, o.qp, prof(d, P_MKADV2, c), prof(d, P_MKWLE2, c), true);
   else if (scalar == 1)
-    mpdata_one<NX, R, G, PAIR>(d, s, c, live, d.qt, prof(d, P_MKADV1, c), prof(d, P_MKWLE1, c), false);
+    mpdata_one<NX, R, G, PAIR, CHUNKS>(d, s, c, live, d.qt, o.qt, prof(d, P_MKADV1, c), prof(d, P_MKWLE1, c), false);
   else
-    mpdata_one<NX, R, G, PAIR>(d, s, c, live, d.t, nullptr, nullptr, false);
+    mpdata_one<NX, R, G, PAIR, CHUNKS>(d, s, c, live, d.t, o.t, nullptr, nullptr, false);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2378,13 +2419,30 @@ k_mpdata_split(DevT<R> d, int nb) {
 // sub-step count nprec read from the maximum Courant number gathered in k_mpdata.
 // Per column, one pipelined sweep per sub-step.
 // ------------------------------------------------------------------------------------------
-template <int NX, typename R>
-__global__ void CRM_LB k_precip(DevT<R> d) {
-  CRM_STOP_CHECK(d);
+// Sub-step j of nprec reads qp from qsrc (j = 1) or the previous sub-step's buffer and writes it
+// to qdst or qx, alternately, so that the last one writes qdst (one buffer for all: in place); t
+// is read and written at the same level only, in place in tt.
+// WG false: a wave's instances per wave, all levels (128 columns: gridDim.y chunks of levels while
+// nprec is 1, as sub-steps of different workgroups cannot wait for each other).  WG true: the
+// waves of a workgroup share one wave's instances, a chunk of levels each, and meet between
+// sub-steps.
+template <int NX, typename R, bool WG>
+__device__ __forceinline__ void precip_fall(const DevT<R>& d, R* tt, const R* qsrc, R* qdst, R* qx) {
   SegFor<NX> s;
   int c;
-  bool live = seg_instance<NX>(d.ncrms, c);
+  bool live;
+  LevelChunk ch = level_chunk(d.nzm);
   const int nzm = d.nzm, i = s.i;
+  if constexpr (WG) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), nw = (int)blockDim.x >> 6;
+    const int g = (int)blockIdx.x * (64 / NX) + s.lane / NX;
+    c = g < d.ncrms ? g : d.ncrms - 1;
+    if constexpr (NX == 64) c = __builtin_amdgcn_readfirstlane(c);
+    live = g < d.ncrms;
+    ch = LevelChunk{nzm * wave / nw, nzm * (wave + 1) / nw};
+  } else {
+    live = seg_instance<NX>(d.ncrms, c);
+  }
   const R dz = inst(d, I_DZ, c), dtn = d.dtn;
   const cprof<R> adz = profc(d, P_ADZ, c);
   const cprof<R> rho = profc(d, P_RHO, c);
@@ -2411,19 +2469,29 @@ __global__ void CRM_LB k_precip(DevT<R> d) {
   // instance keeps it (launches are stream-ordered)
   if (live && c == 0 && i == 0 && (unsigned long long)nprec > d.gmax[GMAX_NPREC])
     d.gmax[GMAX_NPREC] = (unsigned long long)nprec;
+  if (!WG && nprec > 1 && gridDim.y > 1) {
+    if (blockIdx.y > 0) return;
+    ch = LevelChunk{0, nzm};
+  }
+  const int k0 = ch.k0, k1 = ch.k1;
+  // qp's new value depends on the levels two below to three above: a chunk above the surface
+  // starts two levels below it
+  const int ks = ::max(k0 - 2, 0), kend = k1 + 2, kst = ::min(nzm, k1 + 3);
   const R rnprec = (R)nprec;
-  auto Q = [&](R* p, int k) -> R& { return p[((size_t)c * nzm + k) * NX + i]; };
+  auto Q = [&](const R* p, int k) { return p[((size_t)c * nzm + k) * NX + i]; };
+  const R* qin = qsrc;
   auto lfac_of = [&](R tabs) {
     R om = fmax(R(0.0), fmin(R(1.0), (tabs - TPRMIN) * a_pr));
     return FAC_COND + (1 - om) * FAC_FUS;
   };
   const R omega0 = fmax(R(0.0), fmin(R(1.0), (Q(d.tabs, 0) - TPRMIN) * a_pr));
   for (int iprec = 1; iprec <= nprec; iprec++) {
+    R* const qout = ((nprec - iprec) & 1) ? qx : qdst;
     R tq_0 = 0, tq_1 = 0, tq_2 = 0, tq_3 = 0;
     R ta_0 = 0, ta_1 = 0, ta_2 = 0, ta_3 = 0;  // tabs ring
     R tt_a = 0, tt_b = 0;                       // t of level K-2, K-3
     // qp and tabs of the next two levels, loaded two iterations before use
-    R nq1 = Q(d.qp, 0), na1 = Q(d.tabs, 0), nq2 = Q(d.qp, 1), na2 = Q(d.tabs, 1);
+    R nq1 = Q(qin, ks), na1 = Q(d.tabs, ks), nq2 = Q(qin, ks + 1), na2 = Q(d.tabs, ks + 1);
     R wp_0 = 0, wp_1 = 0, wp_2 = 0;
     R fz0_0 = 0, fz0_1 = 0, fz0_2 = 0;
     R tq1_a = 0, tq1_b = 0;
@@ -2432,9 +2500,10 @@ __global__ void CRM_LB k_precip(DevT<R> d) {
     R mx_a = 0, mn_a = 0;
     R fz_a = 0;
     // one level step; ST: steady state (4 <= K < nzm), where every stage is active and every
-    // boundary select is the interior one, so the guards fold away (as in MPDATA)
-    auto step = [&](const int K, auto steady) {
-      constexpr bool ST = decltype(steady)::value;
+    // boundary select is the interior one, so the guards fold away; modes as in MPDATA
+    auto step = [&](const int K, auto mode) __attribute__((always_inline)) {
+      constexpr int MODE = decltype(mode)::value;
+      constexpr bool ST = MODE != 0;
       const R cq = nq1, ca = na1;
       nq1 = nq2;
       na1 = na2;
@@ -2443,10 +2512,10 @@ __global__ void CRM_LB k_precip(DevT<R> d) {
          // directly (a conditional one is preceded by a copy that waits for earlier loads).
          // Level nzm-1 is written only at step nzm+2, after the last of these reads.
         const int kn = ::min(K + 2, nzm - 1);
-        nq2 = Q(d.qp, kn);
+        nq2 = Q(qin, kn);
         na2 = Q(d.tabs, kn);
       }
-      const R tt_new = (ST || (K >= 1 && K - 1 < nzm)) ? Q(d.t, K - 1) : R(0.0);
+      const R tt_new = (ST || (K >= 1 && K - 1 < nzm)) ? Q(tt, K - 1) : R(0.0);
       // a: level K, upwind flux
       if (ST || K < nzm) {
         tq_0 = cq;
@@ -2485,7 +2554,7 @@ __global__ void CRM_LB k_precip(DevT<R> d) {
       }
       // f: level K-3, update of qp and t, statistics
       const int Fl = K - 3;
-      if (ST || (Fl >= 0 && Fl < nzm)) {
+      if (MODE == 1 || (MODE == 0 && Fl >= k0 && Fl < nzm)) {
         R irhoadz = irhoadz_p[Fl];
         R fzF = fz_a, fzF1 = (ST || Fl + 1 < nzm) ? fz_new : R(0.0);
         R lf = lfac_of(ta_3), lf1 = (ST || Fl + 1 < nzm) ? lfac_of(ta_2) : R(0.0);
@@ -2494,8 +2563,9 @@ __global__ void CRM_LB k_precip(DevT<R> d) {
         R sfall = s.sum(dq * R(1.));
         R sflux = s.sum(fzF * R(1.));
         if (live) {
-          Q(d.qp, Fl) = tq_3 - (fzF1 - fzF) * irhoadz;
-          Q(d.t, Fl) = tt_b - lat_heat;
+          const size_t of = ((size_t)c * nzm + Fl) * NX + i;
+          qout[of] = tq_3 - (fzF1 - fzF) * irhoadz;
+          tt[of] = tt_b - lat_heat;
           if (i == 0) {
             accum(&qpfall[Fl], sfall);
             accum(&precflux[Fl], -sflux);
@@ -2527,11 +2597,29 @@ __global__ void CRM_LB k_precip(DevT<R> d) {
       mn_a = mn_new;
       fz_a = fz_new;
     };
-    int K = 0;
-    for (; K < 4 && K <= nzm + 2; K++) step(K, std::false_type{});
-    for (; K < nzm; K++) step(K, std::true_type{});
-    for (; K <= nzm + 2; K++) step(K, std::false_type{});
+    using Edge = std::integral_constant<int, 0>;
+    using Steady = std::integral_constant<int, 1>;
+    using Below = std::integral_constant<int, 2>;
+    int K = ks;
+    for (; K < 4 && K <= kend; K++) step(K, Edge{});
+    for (; K < k0 + 3 && K < kst; K++) step(K, Below{});
+    for (; K < kst; K++) step(K, Steady{});
+    for (; K <= kend; K++) step(K, Edge{});
+    qin = qout;
+    if constexpr (WG) {
+      if (iprec < nprec) __syncthreads();
+    }
   }
+}
+template <int NX, typename R>
+__global__ void CRM_LB k_precip(DevT<R> d, R* tt, const R* qsrc, R* qdst, R* qx) {
+  CRM_STOP_CHECK(d);
+  precip_fall<NX, R, false>(d, tt, qsrc, qdst, qx);
+}
+template <int NX, typename R>
+__global__ void __launch_bounds__(512) k_precip_wg(DevT<R> d, R* tt, const R* qsrc, R* qdst, R* qx) {
+  CRM_STOP_CHECK(d);
+  precip_fall<NX, R, true>(d, tt, qsrc, qdst, qx);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2542,14 +2630,16 @@ __global__ void CRM_LB k_precip(DevT<R> d) {
 // all three: tkh and the level profiles are read once per level instead of once per field, and
 // the three fields' chains interleave.  Each field's arithmetic is the one-field sweep's, so
 // the results are the same bits.
-template <int NX, typename R, typename G = SegFor<NX>>
-__global__ void CRM_LB k_diffuse(DevT<R> d) {
+// CHUNKS: the levels dealt to gridDim.y chunks, from src to the fields' own buffers (else in place)
+template <int NX, typename R, typename G, bool CHUNKS>
+__global__ void CRM_LB k_diffuse(DevT<R> d, Scalars<R> src) {
   CRM_STOP_CHECK(d);
   G s;
   int c;
   const bool live = seg_instance<NX>(d.ncrms, c);
   constexpr int NF = 3;
-  R* const fs[NF] = {d.t, d.qt, d.qp};
+  R* const fo[NF] = {d.t, d.qt, d.qp};
+  const R* const fs[NF] = {CHUNKS ? src.t : d.t, CHUNKS ? src.qt : d.qt, CHUNKS ? src.qp : d.qp};
   double* const fdiffs[NF] = {nullptr, prof(d, P_MKDIFF1, c), prof(d, P_MKDIFF2, c)};
   double* const fluxes[NF] = {nullptr, prof(d, P_MKWSB1, c), prof(d, P_MKWSB2, c)};
   const int nzm = d.nzm, i = s.i;
@@ -2561,15 +2651,19 @@ __global__ void CRM_LB k_diffuse(DevT<R> d) {
   const cprof<R> drhoi = profc(d, P_DRHOI, c);
   const R rdx2 = (R)(R(1.) / (d.dx * d.dx)), rdz2 = (R)1. / (dz * dz);
   auto Q = [&](const R* p, int k) { return p[((size_t)c * nzm + k) * NX + i]; };
+  // a chunk above the surface starts one level below it, for the flux at its bottom
+  const LevelChunk ch = CHUNKS ? level_chunk(nzm) : LevelChunk{0, nzm};
+  const int ks = ::max(ch.k0 - 1, 0);
   R f_k[NF], f_n[NF], flx_prev[NF];
 #pragma unroll
   for (int q = 0; q < NF; q++) {
-    f_k[q] = Q(fs[q], 0);
-    f_n[q] = Q(fs[q], 1);
+    f_k[q] = Q(fs[q], ks);
+    f_n[q] = Q(fs[q], ks + 1);
     flx_prev[q] = R(0.0) * (R(1.) / dz) * rhow[0];
   }
-  R tkh_k = Q(d.tkh, 0), tkh_n = Q(d.tkh, 1);
-  for (int k = 0; k < nzm; k++) {
+  R tkh_k = Q(d.tkh, ks), tkh_n = Q(d.tkh, ks + 1);
+  for (int k = ks; k < ch.k1; k++) {
+    const bool store = live && (!CHUNKS || k >= ch.k0);
     // level k+2, clamped at the top: a value read past it is never used (level k+1's values
     // enter only inner levels, k+1 <= nzm-2), and a load that always issues needs no copy
     // that would wait for earlier loads
@@ -2609,7 +2703,7 @@ __global__ void CRM_LB k_diffuse(DevT<R> d) {
         flxv = R(0.0) * (R(1.) / dz) * (R(1.) / adzw[nzm]) * rhow[nzm];
       const R dfdt = dtn * (dfh - (flxv - flx_prev[q]) * rhoi);
       const R fnew = fk + dfdt;
-      if (live) fs[q][((size_t)c * nzm + k) * NX + i] = fnew;
+      if (store) fo[q][((size_t)c * nzm + k) * NX + i] = fnew;
       if (q > 0) {
         if constexpr (std::is_same<R, double>::value) {  // reduced together below
           red[2 * (q - 1)] = flxv;
@@ -2617,10 +2711,10 @@ __global__ void CRM_LB k_diffuse(DevT<R> d) {
         } else {  // FP32: one DPP reduction each, in place (measured faster than batched)
           if (inner) {
             const R sv = s.sum(flxv);
-            if (live && i == 0) fluxes[q][k + 1] = sv;
+            if (store && i == 0) fluxes[q][k + 1] = sv;
           }
           const R sd = s.sum(fnew - fk);
-          if (live && i == 0) fdiffs[q][k] = sd;
+          if (store && i == 0) fdiffs[q][k] = sd;
         }
       }
       flx_prev[q] = flxv;
@@ -2629,7 +2723,7 @@ __global__ void CRM_LB k_diffuse(DevT<R> d) {
     }
     if constexpr (std::is_same<R, double>::value) {
       s.sums(red);
-      if (live) {
+      if (store) {
 #pragma unroll
         for (int q = 1; q < NF; q++) {
           if (inner && s.template sum_owner<R>(2 * (q - 1))) fluxes[q][k + 1] = red[2 * (q - 1)];
@@ -2642,7 +2736,12 @@ __global__ void CRM_LB k_diffuse(DevT<R> d) {
   }
 #pragma unroll
   for (int q = 0; q < NF; q++)
-    if (fluxes[q] && live && i == 0) fluxes[q][0] = R(0.0);
+    if (fluxes[q] && live && ch.k0 == 0 && i == 0) fluxes[q][0] = R(0.0);
+  // the cloud-ice level range that the chunks of k_micro extend (k_pre has read the last one)
+  if (live && ch.k0 == 0 && i == 0) {
+    inst(d, I_KMIN, c) = nzm;
+    inst(d, I_KMAX, c) = -1;
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2802,6 +2901,20 @@ __device__ __forceinline__ void diagnose_level(const DevT<R>& d, const S_& s, in
   }
 }
 
+// The instance's cloud-ice level range from this workgroup's levels.  The chunks of an instance
+// extend the range that k_diffuse emptied: kmin is not negative, so it orders as its bits, and so
+// does kmax >= -1 as signed bits.
+template <typename R>
+__device__ __forceinline__ void ice_range(const DevT<R>& d, int c, int kmin, int kmax) {
+  if (gridDim.y == 1) {
+    inst(d, I_KMIN, c) = kmin;
+    inst(d, I_KMAX, c) = kmax;
+  } else {
+    atomicMin((unsigned long long*)&inst(d, I_KMIN, c), (unsigned long long)__double_as_longlong((double)kmin));
+    atomicMax((long long*)&inst(d, I_KMAX, c), __double_as_longlong((double)kmax));
+  }
+}
+
 // The level means of accelerate_crm.F90:196-250 after micro_proc, minus those of the last
 // diagnose; flags a mean t change above 5 K (ceaseflag) in gmax[3].
 template <int NX, typename R, typename S_>
@@ -2846,7 +2959,8 @@ __global__ void CRM_LB k_micro(DevT<R> d, int accel) {
   const R powg1 = (3 + B_GRAU) / R(4.), powg2 = (5 + B_GRAU) / R(8.);
   int kmin = nzm, kmax = -1;
   // t, qt, qp (and the winds for the level means) of the next level, read one level ahead
-  const size_t o0 = ((size_t)c * nzm) * NX + i;
+  const LevelChunk ch = level_chunk(nzm);
+  const size_t o0 = ((size_t)c * nzm + ch.k0) * NX + i;
   R t_pre = d.t[o0], qt_pre = d.qt[o0], qp_pre = d.qp[o0], u_pre = d.u[o0];
   R v_pre = y3 ? d.v[o0] : R(0.0);
   // KUR: w of levels k and k+1 (the second read one level ahead) and tkh of level k
@@ -2858,11 +2972,11 @@ __global__ void CRM_LB k_micro(DevT<R> d, int accel) {
   const cprof<double> kur_grdf = profcd(d, P_GRDFX, c);
   const double kur_dxf = sqrt((1. / d.dx) * (1. / d.dx) + (y3 ? (1. / d.dx) * (1. / d.dx) : 0.0));
   if constexpr (KUR) {
-    w_a = Wk(0);
-    w_b = Wk(1);
+    w_a = Wk(ch.k0);
+    w_b = Wk(ch.k0 + 1);
     tkh_pre = d.tkh[o0];
   }
-  for (int k = 0; k < nzm; k++) {
+  for (int k = ch.k0; k < ch.k1; k++) {
     size_t o = ((size_t)c * nzm + k) * NX + i;
     // the precip_init coefficients are constant during this kernel: scalar loads, which do
     // not wait for the vector prefetch of the next level (a vector load here would)
@@ -3121,10 +3235,7 @@ __global__ void CRM_LB k_micro(DevT<R> d, int accel) {
   if (accel) return;
   kmin = s.imin(kmin);
   kmax = s.imax(kmax);
-  if (live && i == 0) {
-    inst(d, I_KMIN, c) = kmin;
-    inst(d, I_KMAX, c) = kmax;
-  }
+  if (live && i == 0) ice_range(d, c, kmin, kmax);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -3145,7 +3256,8 @@ __global__ void CRM_LB k_accel(DevT<R> d, double factor, int uv) {
   const bool apply = *(volatile unsigned long long*)&d.gmax[3] == 0;
   const double tmin = 50.;
   int kmin = nzm, kmax = -1;
-  for (int k = 0; k < nzm; k++) {
+  const LevelChunk ch = level_chunk(nzm);
+  for (int k = ch.k0; k < ch.k1; k++) {
     size_t o = ((size_t)c * nzm + k) * NX + i;
     R t = d.t[o], q = d.qt[o], qp = d.qp[o], qn = d.qn[o];
     R qv = d.qv[o], qcl = d.qcl[o], qci = d.qci[o], qpl = d.qpl[o], qpi = d.qpi[o];
@@ -3187,17 +3299,58 @@ __global__ void CRM_LB k_accel(DevT<R> d, double factor, int uv) {
   }
   kmin = s.imin(kmin);
   kmax = s.imax(kmax);
-  if (live && i == 0) {
-    inst(d, I_KMIN, c) = kmin;
-    inst(d, I_KMAX, c) = kmax;
-  }
+  if (live && i == 0) ice_range(d, c, kmin, kmax);
 }
 
 // ------------------------------------------------------------------------------------------
 // Per-GCM-substep statistics: crm_module.F90:896-1073.  Accumulated on the device in
 // profiles indexed by CRM level (w level for the mass fluxes) and per-instance sums.
 // ------------------------------------------------------------------------------------------
-template <int NX, typename R>
+// Column water paths from the top (the reference's level nz-k, crm_module.F90:903-945): the cloud
+// top and the cloud covers, which depend on the sum over all levels above.
+struct WaterPaths {
+  static constexpr double thr = R4(0.001);
+  double cwp = 0, cwph = 0, cwpm = 0, cwpl = 0, clt = 0, cmt = 0, cht = 0, ctt = 0;
+  bool flag_top = true;
+  // one level further down, of condensate qcl + qci; 1 where it is the column's cloud top
+  __device__ __forceinline__ double level(double rho, double adz, double dz, double pres, double qcl, double qci) {
+    const double tmp1 = rho * adz * dz * (qcl + qci);
+    cwp += tmp1;
+    ctt = fmax(1.0, ctt);
+    double top_hit = 0.0;
+    if (cwp > thr && flag_top) {
+      top_hit = 1.0;
+      flag_top = false;
+    }
+    if (pres >= 700.) {
+      cwpl += tmp1;
+      clt = fmax(1.0, clt);
+    } else if (pres < 400.) {
+      cwph += tmp1;
+      cht = fmax(1.0, cht);
+    } else {
+      cwpm += tmp1;
+      cmt = fmax(1.0, cmt);
+    }
+    return top_hit;
+  }
+  template <typename R, typename S_>
+  __device__ __forceinline__ void covers(const DevT<R>& d, const S_& s, int c, bool live) const {
+    double cv[4] = {cwp > thr ? ctt : 0.0, cwph > thr ? cht : 0.0, cwpm > thr ? cmt : 0.0, cwpl > thr ? clt : 0.0};
+    s.multi_sum(cv);
+    if (live) {
+      if (s.owns(0)) accum(&inst(d, I_CLTOT, c), cv[0]);
+      if (s.owns(1)) accum(&inst(d, I_CLHGH, c), cv[1]);
+      if (s.owns(2)) accum(&inst(d, I_CLMED, c), cv[2]);
+      if (s.owns(3)) accum(&inst(d, I_CLLOW, c), cv[3]);
+    }
+  }
+};
+
+// COLS: one sweep over all levels does the water paths and the level statistics.  Otherwise the
+// levels are dealt to gridDim.y - 1 chunks, and the last workgroup of an instance takes the
+// water paths alone, from the two fields they need.
+template <int NX, typename R, bool COLS>
 __global__ void CRM_LB k_stats(DevT<R> d) {
   CRM_STOP_CHECK(d);
   SegFor<NX> s;
@@ -3209,7 +3362,7 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
   const double* rhow = prof(d, P_RHOW, c);
   const double* adz = prof(d, P_ADZ, c);
   const double* pres = prof(d, P_PRES, c);
-  const double thr = R4(0.001), wmin = 2.;
+  const double thr = WaterPaths::thr, wmin = 2.;
   const int nxr = d.nx_rad, g = NX / nxr, ir = rad_col(d, i);
   auto Q = [&](const R* p, int k) -> double { return p[((size_t)c * nzm + k) * NX + i]; };
   auto Wv = [&](int k) -> double { return d.w[((size_t)c * nz + k) * NX + i]; };
@@ -3228,7 +3381,7 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
     double qcl, qci, qpl, qpi, tabs, qv, w, rho, rhow, adz, pres;
     R ra[5];
   };
-  auto load = [&](int k, Lvl& L) {
+  auto load = [&](int k, Lvl& L, bool sums = true) {
     L.qcl = Q(d.qcl, k);
     L.qci = Q(d.qci, k);
     L.qpl = Q(d.qpl, k);
@@ -3241,14 +3394,47 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
     L.adz = adz[k];
     L.pres = pres[k];
     for (int q = 0; q < 5; q++) L.ra[q] = R(0.0);
-    if (rad_owner)
+    if (rad_owner && sums)
       for (int q = 0; q < 5; q++) L.ra[q] = d.rad[q * rad_blk + rad_at(k)];
   };
-  double cwp = 0, cwph = 0, cwpm = 0, cwpl = 0, clt = 0, cmt = 0, cht = 0, ctt = 0;
-  bool flag_top = true;
-  double w_up = Wv(nzm);  // lid
+  WaterPaths wp;
+  LevelChunk ch{0, nzm};
+  if constexpr (!COLS) {
+    const int nch = (int)gridDim.y - 1, y = (int)blockIdx.y;
+    if (y == nch) {
+      // NB levels are read together (a read after an addition would wait behind it)
+      constexpr int NB = 8;
+      for (int kt = nzm - 1; kt >= 0; kt -= NB) {
+        double v[NB][5];
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+          const int k = ::max(kt - j, 0);
+          v[j][0] = rho[k];
+          v[j][1] = adz[k];
+          v[j][2] = pres[k];
+          v[j][3] = Q(d.qcl, k);
+          v[j][4] = Q(d.qci, k);
+        }
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+          if (kt - j < 0) break;
+          const double hit = wp.level(v[j][0], v[j][1], dz, v[j][2], v[j][3], v[j][4]);
+          if (s.any(hit != 0.0)) {  // adding zero changes nothing
+            const double n = s.sum(hit);
+            if (live && i == 0) accum(&prof(d, P_CLDTOP, c)[nzm - 1 - (kt - j)], n);
+          }
+        }
+      }
+      wp.covers(d, s, c, live);
+      return;
+    }
+    ch = LevelChunk{(int)((unsigned)nzm * y / nch), (int)((unsigned)nzm * (y + 1) / nch)};
+  }
+  double w_up = Wv(ch.k1);  // the lid for the top chunk
   Lvl up2{}, up{}, cur, nxt{};
-  load(nzm - 1, cur);
+  if (ch.k1 + 1 < nzm) load(ch.k1 + 1, up2, false);
+  if (ch.k1 < nzm) load(ch.k1, up, false);
+  load(ch.k1 - 1, cur);
   // mass flux through a w level with vertical velocity wj (crm_module.F90:1017-1049): the level
   // whose condensate decides is Xu (the level below, or the surface level) for an updraft and
   // the level above (Xa, or Xb, the top level, when a is false) for a downdraft; one saturation
@@ -3272,7 +3458,7 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
       mdi = (!upd && (cloudy || dq > R4(1.0e-4))) ? f : 0.0;
     }
   };
-  for (int k = nzm - 1; k >= 0; k--) {
+  for (int k = ch.k1 - 1; k >= ch.k0; k--) {
     // at k = 0 level 0 again, unused (unconditional, as above); its radiation sums are read
     // before this level's are written, and never written from that read
     load(::max(k - 1, 0), nxt);
@@ -3280,25 +3466,8 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
     const R* ra = cur.ra;
     const double qcl = cur.qcl, qci = cur.qci, qpl = cur.qpl, qpi = cur.qpi, tabs = cur.tabs;
     const double wk = cur.w;
-    // column water paths from the top (the reference's level nz-k)
-    double tmp1 = cur.rho * cur.adz * dz * (qcl + qci);
-    cwp += tmp1;
-    ctt = fmax(1.0, ctt);
     double top_hit = 0.0;
-    if (cwp > thr && flag_top) {
-      top_hit = 1.0;
-      flag_top = false;
-    }
-    if (cur.pres >= 700.) {
-      cwpl += tmp1;
-      clt = fmax(1.0, clt);
-    } else if (cur.pres < 400.) {
-      cwph += tmp1;
-      cht = fmax(1.0, cht);
-    } else {
-      cwpm += tmp1;
-      cmt = fmax(1.0, cmt);
-    }
+    if constexpr (COLS) top_hit = wp.level(cur.rho, cur.adz, dz, cur.pres, qcl, qci);
     // level statistics (the reference's level k)
     double mass = cur.rho * cur.adz * dz;
     double ws = w_up + wk;
@@ -3331,7 +3500,7 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
     const double r_t = rs[0], r_qv = rs[1], r_qc = rs[2], r_qi = rs[3], r_cld = rs[4];
     if (live) {
       // the reference's index mix for the cloud top (crm_module.F90:918-925)
-      if (s.owns(0)) accum(&prof(d, P_CLDTOP, c)[nzm - 1 - k], sv[0]);
+      if (COLS && s.owns(0)) accum(&prof(d, P_CLDTOP, c)[nzm - 1 - k], sv[0]);
       if (s.owns(1)) accum(&prof(d, P_CLD, c)[k], sv[1]);
       if (s.owns(2)) accum(&prof(d, P_MCUP, c)[k], sv[2]);
       if (s.owns(3)) accum(&prof(d, P_MCDN, c)[k], sv[3]);
@@ -3354,6 +3523,7 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
     up = cur;
     cur = nxt;
   }
+  if (ch.k0 > 0) return;
   {  // w level 0, with level 0 (now up) below and level 1 (up2) above
     double mui = 0, mdi = 0;
     mass_flux(w_up, up.rhow, up, up2, up, nzm > 1, mui, mdi);
@@ -3364,14 +3534,7 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
       if (s.owns(9)) accum(&prof(d, P_MDI, c)[0], sv[9]);
     }
   }
-  double cv[4] = {cwp > thr ? ctt : 0.0, cwph > thr ? cht : 0.0, cwpm > thr ? cmt : 0.0, cwpl > thr ? clt : 0.0};
-  s.multi_sum(cv);
-  if (live) {
-    if (s.owns(0)) accum(&inst(d, I_CLTOT, c), cv[0]);
-    if (s.owns(1)) accum(&inst(d, I_CLHGH, c), cv[1]);
-    if (s.owns(2)) accum(&inst(d, I_CLMED, c), cv[2]);
-    if (s.owns(3)) accum(&inst(d, I_CLLOW, c), cv[3]);
-  }
+  if constexpr (COLS) wp.covers(d, s, c, live);
 }
 
 // ------------------------------------------------------------------------------------------

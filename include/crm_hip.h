@@ -227,15 +227,17 @@ int crm_hip_set_schedule(crm_hip_ctx *ctx, const int block[CRM_HIP_NKERNEL]);
 int crm_hip_get_schedule(const crm_hip_ctx *ctx, int block[CRM_HIP_NKERNEL]);
 
 /* Launch variant ("tile shape") of each kernel class of a context, 0 the default; results are
- * bitwise the same in every variant. CRM_K_PRESS of 2D 64-column CRMs: 0 one instance per
- * 4-wave workgroup (two workgroups per CU), 1 one instance on 8 waves with the gradient pass's
- * inputs kept in registers from the right-hand side pass (one workgroup per CU), 2 and 3 as 0
- * with two or four levels of each pass unrolled together, 4 as 0 with the Thomas factors in
- * registers (the workgroup's LDS is the slab alone: three workgroups per CU). CRM_K_MPDATA: 0 the default number
- * of levels per trip of the sweep's steady state (two for 2D 64-column CRMs, else one), 1 the
- * other, 2 and 3 as 0 and 1 with the registers bounded for three waves per SIMD, 4 and 5 as 0
- * and 2 with each of the three scalars advected on its own waves. Other classes have variant 0
- * only. */
+ * bitwise the same in every variant. CRM_K_PRESS of 2D 64-column CRMs: 0 chosen by the batch's
+ * size (4 beyond 512 instances at 28 and 58 levels, else one instance per 4-wave workgroup with the
+ * Thomas factors in LDS, two workgroups per CU), 1 one instance on 8 waves with the gradient pass's
+ * inputs kept in registers from the right-hand side pass (one workgroup per CU), 2 and 3 the 4-wave
+ * workgroup with two or four levels of each pass unrolled together, 4 the 4-wave workgroup with
+ * the Thomas factors in registers (the workgroup's LDS is the slab alone: three workgroups per
+ * CU). CRM_K_MPDATA (each scalar on its own waves): 0 chosen by the batch's size (small batches deal
+ * the levels to several workgroups; large ones take 2 at 64 columns in 2D, else 4), 1 the other
+ * number of levels per trip of the sweep's steady state than the default (two for 2D 64-column
+ * CRMs, else one), 2 and 3 the default and 1 with the registers bounded for three waves per SIMD,
+ * 4 the default with unbounded registers, 5 as 2. Other classes have variant 0 only. */
 int crm_hip_set_variants(crm_hip_ctx *ctx, const int variant[CRM_HIP_NKERNEL]);
 int crm_hip_get_variants(const crm_hip_ctx *ctx, int variant[CRM_HIP_NKERNEL]);
 
