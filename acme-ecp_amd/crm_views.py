@@ -7,6 +7,7 @@ column-major with pcols leading.  `CrmCase` holds numpy arrays with exactly thos
 Fortran order and builds the pointer views that the C ABI takes.
 """
 import ctypes as C
+import struct
 
 import numpy as np
 
@@ -60,8 +61,6 @@ CrmOutputView = _struct("CrmOutputView", OUT_ORDER)
 def _ptr(a):
     if a is None:
         return c_dp()
-    if isinstance(a, int):        # a raw device address
-        return C.cast(C.c_void_p(a), c_dp)
     assert a.dtype == np.float64 and a.flags["F_CONTIGUOUS"]
     return a.ctypes.data_as(c_dp)
 
@@ -118,9 +117,14 @@ class CrmCase:
                 CrmOutputView(*[_ptr(self.out[f]) for f in OUT_ORDER]))
 
 
+def _struct_at(cls, order, addr):
+    """A view struct over raw addresses (integers, None for a null pointer).  The struct is made
+    of its bytes: converting some 90 addresses of a call to pointer objects one by one took 90 us,
+    more than most of the kernels it is made for."""
+    return cls.from_buffer_copy(struct.pack("%dP" % len(order), *[addr[f] or 0 for f in order]))
+
+
 def views_from_addresses(inp, state, rad, out):
     """Views over device arrays given as dicts name -> integer address."""
-    return (CrmInputView(*[_ptr(inp[f]) for f in INPUT_ORDER]),
-            CrmStateView(*[_ptr(state[f]) for f in STATE_ORDER]),
-            CrmRadView(*[_ptr(rad[f]) for f in RAD_ORDER]),
-            CrmOutputView(*[_ptr(out[f]) for f in OUT_ORDER]))
+    return (_struct_at(CrmInputView, INPUT_ORDER, inp), _struct_at(CrmStateView, STATE_ORDER, state),
+            _struct_at(CrmRadView, RAD_ORDER, rad), _struct_at(CrmOutputView, OUT_ORDER, out))
