@@ -1,15 +1,16 @@
 // crm_mlp.hip -- the pointwise network that stands in for the bulk microphysics, trained and
-// evaluated on the matrix cores: BF16 operands, FP32 accumulation (v_mfma_f32_16x16x16_bf16),
-// FP32 master weights and Adam moments.
+// evaluated on the matrix cores: BF16 operands, FP32 accumulation (v_mfma_f32_16x16x16_bf16 and
+// 16x16x32), FP32 master weights and Adam moments.
 //
-// Every layer, forward and backward, is one GEMM C = A (M x K) * B (K x N) with arbitrary
-// strides for A and B, so the transposes of the backward pass cost nothing; the epilogue adds
-// the bias and applies ReLU (forward), or applies the ReLU mask of the forward activations
-// (backward), or accumulates weight gradients split over the batch (FP32 atomics).
+// A training step is two launches: k_train takes a tile of rows per workgroup through the forward
+// and backward passes and leaves its share of the loss and of every gradient in memory; k_reduce
+// adds the shares in a fixed order, applies Adam and writes the new weights in the orders in
+// which the kernels read them.  As one GEMM launch per layer and direction, with column sums,
+// clears, Adam and two repacking kernels (21 launches, gradients by atomics), a step of 16,384
+// rows took 292 us.
 //
-// Layouts (row-major, y = x W + b): the 9 inputs are padded to 16 columns and the 6 outputs
-// to 16, with zero weights in the padding; batches are padded to a multiple of 16 rows with
-// zero inputs and zero output gradients, so padded rows contribute nothing to any gradient.
+// The 9 inputs are padded to 16 and the 6 outputs to 16, with zero weights in the padding; rows
+// past the batch have zero inputs and zero output gradients, so they contribute nothing.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,171 +23,312 @@
 
 namespace crm_mlp_ns {
 
-enum { EPI_F32 = 0, EPI_BIAS_RELU_BF16 = 1, EPI_BIAS_F32 = 2, EPI_MASK_BF16 = 3, EPI_ATOMIC_F32 = 4 };
+// Offsets (bf16 elements) of the weights in the fragment order of the fused inference (F).
+constexpr int F_L1 = 0;                    // layer 1: 8 output blocks x 64 lanes x 4 (K = 16)
+constexpr int F_L2 = F_L1 + 8 * 64 * 4;    // layer 2: (8 output x 4 K blocks) x 64 lanes x 8
+constexpr int F_L3 = F_L2 + 32 * 64 * 8;   // layer 3: as layer 2
+constexpr int F_L4 = F_L3 + 32 * 64 * 8;   // layer 4: 4 K blocks x 64 lanes x 8 (16 outputs)
+constexpr int F_SIZE = F_L4 + 4 * 64 * 8;
+constexpr int B_SIZE = 3 * NH + NP;        // biases b1 b2 b3 b4
 
-// One wave per 16 x 16 tile of C; blockIdx.y selects a chunk of K (EPI_ATOMIC_F32 only).
-// A[m][k] = A[m*sam + k*sak], B[k][n] = B[k*sbk + n*sbn]; M, N, K, kchunk multiples of 16.
-// MFMA 16x16x16 BF16 operand layout (lane l, r = l % 16, q = l / 16):
-//   A: row r, k = 4q..4q+3     B: k = 4q..4q+3, column r     D: rows 4q..4q+3, column r
-template <int EPI>
-__global__ void __launch_bounds__(256) k_gemm(const bf16* A, long sam, long sak, const bf16* B, long sbk, long sbn,
-                                              int M, int N, int K, int kchunk, const float* bias,
-                                              const bf16* mask, long smm, float* Cf, bf16* Cb, long ldc) {
-  const int lane = threadIdx.x & 63;
-  const long wave = ((long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int tiles_n = N / 16;
-  const long tm = wave / tiles_n, tn = wave % tiles_n;
-  if (tm * 16 >= M) return;  // the whole wave leaves together
-  const int r = lane & 15, q = lane >> 4;
-  const int k0 = blockIdx.y * kchunk, k1 = min(K, k0 + kchunk);
-  f4 acc = {0.f, 0.f, 0.f, 0.f};
-  const bf16* a = A + (tm * 16 + r) * sam;
-  const bf16* b = B + (tn * 16 + r) * sbn;
-  for (int k = k0; k < k1; k += 16) {
-    s4 av, bv;
-    // K contiguous (forward activations, transposed weights): one 8-byte load per operand
-    if (sak == 1) {
-      av = *(const s4*)&a[k + 4 * q];
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; j++) av[j] = (short)a[(long)(k + 4 * q + j) * sak];
+// The training orders: blocks of 64 lanes x 4, an A operand of v_mfma_f32_16x16x16_bf16 each.
+// Forward (rows = outputs of the layer), block ob * (K blocks) + kb; backward (rows = inputs),
+// block ib * (output blocks) + nb, for layers 4, 3 and 2.
+constexpr int FRAG = 64 * 4;
+constexpr int T_L1 = 0, T_L2 = T_L1 + 8 * FRAG, T_L3 = T_L2 + 64 * FRAG, T_L4 = T_L3 + 64 * FRAG;
+constexpr int T_B4 = T_L4 + 8 * FRAG, T_B3 = T_B4 + 8 * FRAG, T_B2 = T_B3 + 64 * FRAG;
+constexpr int T_SIZE = T_B2 + 64 * FRAG;
+
+typedef unsigned u4 __attribute__((ext_vector_type(4)));  // 8 bf16, element 0 in the low half
+typedef unsigned u2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bh2 __attribute__((ext_vector_type(2)));
+typedef short sh2 __attribute__((ext_vector_type(2)));
+
+// The copies of the parameters that the kernels read (device memory).
+struct Weights {
+  bf16 *F, *T;                // weights in inference and training order
+  float *b1, *b2, *b3, *b4;   // biases (b4 padded to 16)
+};
+
+// Packed parameter idx of value w into every copy.  Element (k, n) of a layer is lane
+// n % 16 + 16 (k % 16 / 4), slot k % 4 of its forward block; in a 32-wide K block of the inference
+// order the slots of a lane are k % 4 and 4 + k % 4 (its two 16-wide halves).
+__device__ __forceinline__ void place(const Weights& o, int idx, float w) {
+  auto layer = [&](int off, int nout, int f, int t, int tb, bool wide) {
+    const int e = idx - off, k = e / nout, n = e % nout;
+    const bf16 h = to_bf16(w);
+    const int ob = n / 16, kb = k / 16, lane = n % 16 + 16 * (k % 16 / 4), i = k % 4;
+    const int kbs = wide ? 8 : 1;
+    o.T[t + (ob * kbs + kb) * FRAG + lane * 4 + i] = h;
+    o.F[f + (wide ? ((ob * 4 + k / 32) * 64 + lane) * 8 + 4 * (kb & 1) + i : (ob * 64 + lane) * 4 + i)] = h;
+    if (tb >= 0) {
+      const int nbs = nout == NH ? 8 : 1;
+      o.T[tb + (kb * nbs + ob) * FRAG + (k % 16 + 16 * (n % 16 / 4)) * 4 + n % 4] = h;
     }
-    if (sbk == 1) {
-      bv = *(const s4*)&b[k + 4 * q];
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; j++) bv[j] = (short)b[(long)(k + 4 * q + j) * sbk];
-    }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+  };
+  if (idx < OFF_B1) {
+    layer(OFF_W1, NH, F_L1, T_L1, -1, false);
+  } else if (idx < OFF_W2) {
+    o.b1[idx - OFF_B1] = w;
+  } else if (idx < OFF_B2) {
+    layer(OFF_W2, NH, F_L2, T_L2, T_B2, true);
+  } else if (idx < OFF_W3) {
+    o.b2[idx - OFF_B2] = w;
+  } else if (idx < OFF_B3) {
+    layer(OFF_W3, NH, F_L3, T_L3, T_B3, true);
+  } else if (idx < OFF_W4) {
+    o.b3[idx - OFF_B3] = w;
+  } else if (idx < OFF_B4) {
+    layer(OFF_W4, CRM_MLP_NOUT, F_L4, T_L4, T_B4, true);
+  } else {
+    o.b4[idx - OFF_B4] = w;
   }
+}
+// (one thread per parameter; the padding of every copy stays zero from its allocation)
+__global__ void k_place(const float* p, Weights o) {
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx < CRM_MLP_NPARAM) place(o, idx, p[idx]);
+}
+
+// ---- training --------------------------------------------------------------------------------
+constexpr int TROWS = 64;     // rows of a tile, 16 per wave
+constexpr int TLD = TROWS + 4;  // row stride of a [feature][row] tile in LDS: 8-byte reads of 16 features spread over the banks
+constexpr int PSTRIDE = (CRM_MLP_NPARAM + 1 + 63) / 64 * 64;  // a workgroup's shares: gradients, squared error
+
+__device__ __forceinline__ f4 mfma16(s4 a, s4 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ s4 pack4(const float (&v)[4]) {
+  s4 r;
+#pragma unroll
+  for (int j = 0; j < 4; j++) r[j] = (short)to_bf16(v[j]);
+  return r;
+}
+
+// acc[ob] = sum over kb of W block (ob, kb) times in[kb]; the K blocks in order, so that each sum
+// has one order, and the output blocks inside, so that eight products are in flight.  The weights
+// of the whole layer are read before its first product (128 registers of the 512 a wave has
+// here): left to itself the compiler reads eight blocks at a time and waits out the L2's latency
+// eight times a layer (91 us a launch at 16,384 rows).
+template <int OB, int KB>
+__device__ __forceinline__ void blocks(const bf16* W, const s4 (&in)[KB], f4 (&acc)[OB], int lane) {
+  s4 w[KB][OB];
+#pragma unroll
+  for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++) w[kb][ob] = *(const s4*)&W[(ob * KB + kb) * FRAG + lane * 4];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int ob = 0; ob < OB; ob++) acc[ob] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++) acc[ob] = mfma16(w[kb][ob], in[kb], acc[ob]);
+}
+
+// Loss and gradients of the rows of this workgroup's tiles (64 at a time) into part[blockIdx.x].
+// The layers run transposed, as in the fused inference below: the weights are the A operand and
+// the rows the B operand, so one layer's D fragment -- lane (r, q) holds features 4q..4q+3 of row
+// r -- is the next one's B fragment, forward and backward, and a wave takes its 16 rows through
+// both passes in registers.  The weight gradients contract over the rows, which lie across the
+// lanes: every wave leaves its activations and pre-activation gradients in LDS as [feature][row]
+// tiles, and the four waves share the 144 16 x 16 gradient blocks, whose accumulators stay in
+// registers over the workgroup's tiles.  109 KB of LDS: one workgroup per CU, and a grid of at
+// most one per CU.  Bound by latency: 424 MFMAs per wave and tile are 3 us at the matrix rate; the
+// shares (142 KB per workgroup, written here and read by k_reduce) are 73 MB at 256 workgroups.
+__global__ void __launch_bounds__(256) k_train(const float* X, const float* T, int n, Weights w, const float* norm,
+                                               float* part) {
+  __shared__ __attribute__((aligned(16))) bf16 sX[KP][TLD], sH[3][NH][TLD], sY[NP][TLD], sD[3][NH][TLD];
+  __shared__ float red[4];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, r = lane & 15, q = lane >> 4;
+  float mean[4], rs[4], osc[4], b4[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    const long m = tm * 16 + 4 * q + j, n = tn * 16 + r;
-    const float v = acc[j];
-    if constexpr (EPI == EPI_F32) Cf[m * ldc + n] = v;
-    if constexpr (EPI == EPI_ATOMIC_F32) unsafeAtomicAdd(&Cf[m * ldc + n], v);
-    if constexpr (EPI == EPI_BIAS_F32) Cf[m * ldc + n] = v + bias[n];
-    if constexpr (EPI == EPI_BIAS_RELU_BF16) Cb[m * ldc + n] = to_bf16(fmaxf(v + bias[n], 0.f));
-    if constexpr (EPI == EPI_MASK_BF16) Cb[m * ldc + n] = to_bf16(from_bf16(mask[m * smm + n]) > 0.f ? v : 0.f);
+    mean[j] = norm[NORM_MEAN + 4 * q + j];
+    rs[j] = norm[NORM_RSCALE + 4 * q + j];
+    osc[j] = norm[NORM_OSCALE + 4 * q + j];
+    b4[j] = w.b4[4 * q + j];
   }
-}
-
-// Raw inputs X[n][9] -> normalised BF16 rows [mp][16] (zero padding).
-__global__ void k_inputs(const float* X, int n, int mp, const float* norm, bf16* Xn) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)mp * KP) return;
-  const long m = idx / KP;
-  const int c = (int)(idx % KP);
-  float v = 0.f;
-  if (m < n && c < CRM_MLP_NIN) v = (X[m * CRM_MLP_NIN + c] - norm[NORM_MEAN + c]) * norm[NORM_RSCALE + c];
-  Xn[idx] = to_bf16(v);
-}
-
-// Loss of the normalised outputs and its gradient: dY = 2 (Y - T / oscale) / (6 n) in BF16.
-// Grid-stride over the elements; one atomic per workgroup (a few hundred in all, so they do not
-// queue on the one address).
-__global__ void k_loss(const float* Y, const float* T, int n, int mp, const float* norm, bf16* dY, float* loss) {
-  __shared__ float red[4];
-  float e2 = 0.f;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < (long)mp * NP;
-       idx += (long)gridDim.x * blockDim.x) {
-    const long m = idx / NP;
-    const int c = (int)(idx % NP);
-    float g = 0.f;
-    if (m < n && c < CRM_MLP_NOUT) {
-      const float d = Y[idx] - T[m * CRM_MLP_NOUT + c] / norm[NORM_OSCALE + c];
-      e2 += d * d;
-      g = 2.f * d / (6.f * (float)n);
+  f4 g1[2], g2[2][8], g3[2][8], g4[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    g1[i] = g4[i] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int o = 0; o < 8; o++) g2[i][o] = g3[i][o] = f4{0.f, 0.f, 0.f, 0.f};
+  }
+  float gb[3] = {0.f, 0.f, 0.f}, gb4 = 0.f, e2 = 0.f;
+  const int row = 16 * wave + r;
+  for (int tile = blockIdx.x; tile * TROWS < n; tile += gridDim.x) {
+    const long m = (long)tile * TROWS + row;
+    const bool have = m < n;
+    // an offset the compiler cannot see through, so that the weight reads stay inside the loop
+    // (hoisted out of it, the network would be held in registers and spill)
+    int fo = 0;
+    asm volatile("" : "+v"(fo));
+    const bf16* W = w.T + fo;
+    s4 x[1], h[3][8], d[8], y[1];
+    f4 acc[8];
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int c = 4 * q + j;
+      v[j] = have && c < CRM_MLP_NIN ? (X[m * CRM_MLP_NIN + c] - mean[j]) * rs[j] : 0.f;
     }
-    dY[idx] = to_bf16(g);
+    x[0] = pack4(v);
+#pragma unroll
+    for (int j = 0; j < 4; j++) sX[4 * q + j][row] = (bf16)x[0][j];
+    // bias and ReLU of a layer's sums, to registers and LDS
+    auto activate = [&](const float* bias, int l) {
+#pragma unroll
+      for (int ob = 0; ob < 8; ob++) {
+        const f4 b = *(const f4*)&bias[16 * ob + 4 * q];
+        float a[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) a[j] = fmaxf(acc[ob][j] + b[j], 0.f);
+        h[l][ob] = pack4(a);
+#pragma unroll
+        for (int j = 0; j < 4; j++) sH[l][16 * ob + 4 * q + j][row] = (bf16)h[l][ob][j];
+      }
+    };
+    blocks<8, 1>(W + T_L1, x, acc, lane);
+    activate(w.b1, 0);
+    blocks<8, 8>(W + T_L2, h[0], acc, lane);
+    activate(w.b2, 1);
+    blocks<8, 8>(W + T_L3, h[1], acc, lane);
+    activate(w.b3, 2);
+    f4 out[1];
+    blocks<1, 8>(W + T_L4, h[2], out, lane);
+    // loss of the normalised outputs and its gradient 2 (y - t') / (6 n)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int c = 4 * q + j;
+      v[j] = 0.f;
+      if (have && c < CRM_MLP_NOUT) {
+        const float e = (out[0][j] + b4[j]) - T[m * CRM_MLP_NOUT + c] / osc[j];
+        e2 += e * e;
+        v[j] = 2.f * e / (6.f * (float)n);
+      }
+    }
+    y[0] = pack4(v);
+#pragma unroll
+    for (int j = 0; j < 4; j++) sY[4 * q + j][row] = (bf16)y[0][j];
+    // the ReLU mask of a layer's back-propagated sums, to registers and LDS
+    auto mask = [&](int l) {
+#pragma unroll
+      for (int ib = 0; ib < 8; ib++) {
+        float a[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) a[j] = from_bf16((bf16)h[l][ib][j]) > 0.f ? acc[ib][j] : 0.f;
+        d[ib] = pack4(a);
+#pragma unroll
+        for (int j = 0; j < 4; j++) sD[l][16 * ib + 4 * q + j][row] = (bf16)d[ib][j];
+      }
+    };
+    blocks<8, 1>(W + T_B4, y, acc, lane);
+    mask(2);
+    blocks<8, 8>(W + T_B3, d, acc, lane);
+    mask(1);
+    blocks<8, 8>(W + T_B2, d, acc, lane);
+    mask(0);
+    __syncthreads();
+    // weight gradients: this wave's input blocks 2 wave and 2 wave + 1 (layer 1: output blocks)
+#pragma unroll
+    for (int ks = 0; ks < TROWS / 16; ks++) {
+      const int c = 16 * ks + 4 * q;
+      auto at = [&](const bf16* p) { return *(const s4*)p; };
+      const s4 xa = at(&sX[r][c]), ya = at(&sY[r][c]);
+      s4 a1[2], a2[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int f = 16 * (2 * wave + i) + r;
+        a1[i] = at(&sH[0][f][c]);
+        a2[i] = at(&sH[1][f][c]);
+        g1[i] = mfma16(xa, at(&sD[0][f][c]), g1[i]);
+        g4[i] = mfma16(at(&sH[2][f][c]), ya, g4[i]);
+      }
+#pragma unroll
+      for (int o = 0; o < 8; o++) {
+        const s4 d2 = at(&sD[1][16 * o + r][c]), d3 = at(&sD[2][16 * o + r][c]);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          g2[i][o] = mfma16(a1[i], d2, g2[i][o]);
+          g3[i][o] = mfma16(a2[i], d3, g3[i][o]);
+        }
+      }
+    }
+    // bias gradients: sums over the rows
+    if (t < NH) {
+#pragma unroll
+      for (int l = 0; l < 3; l++)
+        for (int c = 0; c < TROWS; c += 4) {
+          const s4 a = *(const s4*)&sD[l][t][c];
+#pragma unroll
+          for (int j = 0; j < 4; j++) gb[l] += from_bf16((bf16)a[j]);
+        }
+      if (t < NP)
+        for (int c = 0; c < TROWS; c++) gb4 += from_bf16(sY[t][c]);
+    }
+    __syncthreads();
   }
-  for (int o = 32; o >= 1; o >>= 1) e2 += __shfl_xor(e2, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e2;
+  float* o = part + (size_t)blockIdx.x * PSTRIDE;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int b = 2 * wave + i;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int k = 4 * q + j, f = 16 * b + k;
+      if (k < CRM_MLP_NIN) o[OFF_W1 + k * NH + 16 * b + r] = g1[i][j];
+      if (r < CRM_MLP_NOUT) o[OFF_W4 + f * CRM_MLP_NOUT + r] = g4[i][j];
+#pragma unroll
+      for (int ob = 0; ob < 8; ob++) {
+        o[OFF_W2 + f * NH + 16 * ob + r] = g2[i][ob][j];
+        o[OFF_W3 + f * NH + 16 * ob + r] = g3[i][ob][j];
+      }
+    }
+  }
+  if (t < NH) {
+    o[OFF_B1 + t] = gb[0];
+    o[OFF_B2 + t] = gb[1];
+    o[OFF_B3 + t] = gb[2];
+    if (t < CRM_MLP_NOUT) o[OFF_B4 + t] = gb4;
+  }
+  for (int k = 32; k >= 1; k >>= 1) e2 += __shfl_xor(e2, k, 64);
+  if (lane == 0) red[wave] = e2;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const float b = red[0] + red[1] + red[2] + red[3];
-    if (b != 0.f) unsafeAtomicAdd(loss, b / (6.f * (float)n));
-  }
+  if (t == 0) o[CRM_MLP_NPARAM] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// Column sums of a BF16 [mp][ld] matrix over its rows, accumulated into out[ncol] (FP32).  A
-// workgroup (256 threads) covers 64 columns with 4 row groups that meet in LDS; blockIdx.y
-// splits the rows.
-__global__ void k_colsum(const bf16* G, int mp, int ld, int ncol, float* out) {
+// Sums of the np workgroups' shares, 64 parameters per workgroup and a quarter of the shares per
+// wave.  ADAM: the update of the parameters and of every copy of the weights; otherwise the
+// gradient to g.  The loss goes to `loss` (host memory the device can write).
+template <bool ADAM>
+__global__ void __launch_bounds__(256) k_reduce(const float* part, int np, int n, float* g, float* p, float* m, float* v,
+                                                float lr, float c1, float c2, Weights w, float* loss) {
   __shared__ float red[4][64];
-  const int cl = threadIdx.x & 63, grp = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + cl;
-  const long step = (long)gridDim.y * 4;
-  float sacc = 0.f;
-  if (c < ncol)
-    for (long m = (long)blockIdx.y * 4 + grp; m < mp; m += step) sacc += from_bf16(G[m * ld + c]);
-  red[grp][cl] = sacc;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, idx = blockIdx.x * 64 + lane;
+  float s = 0.f;
+#pragma unroll 8
+  for (int k = wave; k < np; k += 4) s += part[(size_t)k * PSTRIDE + idx];
+  red[wave][lane] = s;
   __syncthreads();
-  if (grp == 0 && c < ncol) unsafeAtomicAdd(&out[c], (red[0][cl] + red[1][cl]) + (red[2][cl] + red[3][cl]));
-}
-
-// Packed FP32 parameters -> padded BF16 weights and FP32 biases used by the GEMMs.
-__global__ void k_unpack(const float* p, bf16* W1, bf16* W2, bf16* W3, bf16* W4, float* b1, float* b2, float* b3,
-                         float* b4) {
-  int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  // W1p [16][128]
-  if (idx < KP * NH) {
-    int k = idx / NH, n = idx % NH;
-    W1[idx] = to_bf16(k < CRM_MLP_NIN ? p[OFF_W1 + k * NH + n] : 0.f);
+  if (wave > 0 || idx > CRM_MLP_NPARAM) return;
+  const float gi = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+  if (idx == CRM_MLP_NPARAM) {
+    *loss = gi / (6.f * (float)n);
+    return;
   }
-  if (idx < NH * NH) {
-    W2[idx] = to_bf16(p[OFF_W2 + idx]);
-    W3[idx] = to_bf16(p[OFF_W3 + idx]);
-  }
-  // W4p [128][16]
-  if (idx < NH * NP) {
-    int k = idx / NP, n = idx % NP;
-    W4[idx] = to_bf16(n < CRM_MLP_NOUT ? p[OFF_W4 + k * CRM_MLP_NOUT + n] : 0.f);
-  }
-  if (idx < NH) {
-    b1[idx] = p[OFF_B1 + idx];
-    b2[idx] = p[OFF_B2 + idx];
-    b3[idx] = p[OFF_B3 + idx];
-  }
-  if (idx < NP) b4[idx] = idx < CRM_MLP_NOUT ? p[OFF_B4 + idx] : 0.f;
-}
-
-// Padded gradients -> packed gradient vector.
-__global__ void k_pack_grad(const float* gW1, const float* gW2, const float* gW3, const float* gW4, const float* gb1,
-                            const float* gb2, const float* gb3, const float* gb4, float* g) {
-  int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= CRM_MLP_NPARAM) return;
-  float v;
-  if (idx < OFF_B1) {
-    v = gW1[idx];  // rows 0..8 of [16][128]
-  } else if (idx < OFF_W2) {
-    v = gb1[idx - OFF_B1];
-  } else if (idx < OFF_B2) {
-    v = gW2[idx - OFF_W2];
-  } else if (idx < OFF_W3) {
-    v = gb2[idx - OFF_B2];
-  } else if (idx < OFF_B3) {
-    v = gW3[idx - OFF_W3];
-  } else if (idx < OFF_W4) {
-    v = gb3[idx - OFF_B3];
-  } else if (idx < OFF_B4) {
-    int e = idx - OFF_W4, k = e / CRM_MLP_NOUT, n = e % CRM_MLP_NOUT;
-    v = gW4[k * NP + n];
+  if constexpr (ADAM) {
+    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+    float mi = b1 * m[idx] + (1.f - b1) * gi;
+    float vi = b2 * v[idx] + (1.f - b2) * gi * gi;
+    m[idx] = mi;
+    v[idx] = vi;
+    const float pn = p[idx] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    p[idx] = pn;
+    place(w, idx, pn);
   } else {
-    v = gb4[idx - OFF_B4];
+    g[idx] = gi;
   }
-  g[idx] = v;
-}
-
-__global__ void k_adam(float* p, const float* g, float* m, float* v, float lr, float c1, float c2) {
-  int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= CRM_MLP_NPARAM) return;
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  float mi = b1 * m[idx] + (1.f - b1) * g[idx];
-  float vi = b2 * v[idx] + (1.f - b2) * g[idx] * g[idx];
-  m[idx] = mi;
-  v[idx] = vi;
-  p[idx] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
 // Fused inference, the whole network in registers.  The layers run transposed, H^T = W^T A^T:
@@ -196,50 +338,10 @@ __global__ void k_adam(float* p, const float* g, float* m, float* v, float lr, f
 // 128-wide layers use v_mfma_f32_16x16x32_bf16, whose 32 K slots a lane fills with eight
 // values; the K order inside a 32-feature block is a free choice as long as A and B agree,
 // and we take slot (q, i) = feature 4q + i (i < 4) or 16 + 4q + (i - 4) (i >= 4), which is
-// exactly the two D fragments of output blocks 2kb and 2kb + 1.  The weights are stored once
-// per network in that fragment order (k_frags: each lane's operand is 8 or 16 contiguous
-// bytes) and copied into LDS by every workgroup; a wave owns 64 points (4 blocks of 16) per
+// exactly the two D fragments of output blocks 2kb and 2kb + 1.  The weights are stored in that
+// fragment order (place: each lane's operand is 8 or 16 contiguous bytes) and copied into LDS by every workgroup; a wave owns 64 points (4 blocks of 16) per
 // tile and reads each weight fragment once for the 4 blocks.  The grid is persistent: two
 // workgroups per CU (the weights take 74 KiB of LDS) loop over the tiles.
-constexpr int F_L1 = 0;                     // layer 1: 8 output blocks x 64 lanes x 4 (K = 16)
-constexpr int F_L2 = F_L1 + 8 * 64 * 4;     // layer 2: (8 output x 4 K blocks) x 64 lanes x 8
-constexpr int F_L3 = F_L2 + 32 * 64 * 8;    // layer 3: as layer 2
-constexpr int F_L4 = F_L3 + 32 * 64 * 8;    // layer 4: 4 K blocks x 64 lanes x 8 (16 outputs)
-constexpr int F_SIZE = F_L4 + 4 * 64 * 8;   // bf16 elements
-constexpr int B_SIZE = 3 * NH + NP;         // biases b1 b2 b3 b4
-
-typedef unsigned u4 __attribute__((ext_vector_type(4)));  // 8 bf16, element 0 in the low half
-typedef unsigned u2 __attribute__((ext_vector_type(2)));
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef float f2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bh2 __attribute__((ext_vector_type(2)));
-typedef short sh2 __attribute__((ext_vector_type(2)));
-
-// Input feature (or K index inside a 32-block) of slot i of lane quarter q.
-__device__ __forceinline__ int slot32(int q, int i) { return i < 4 ? 4 * q + i : 16 + 4 * q + (i - 4); }
-
-// Weights in fragment order, from the packed FP32 parameters (one thread per element).
-__global__ void k_frags(const float* p, bf16* F) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= F_SIZE) return;
-  float w = 0.f;
-  if (idx < F_L2) {
-    const int ob = idx / 256, l = (idx / 4) % 64, i = idx % 4;
-    const int n = 16 * ob + l % 16, k = 4 * (l / 16) + i;
-    if (k < CRM_MLP_NIN) w = p[OFF_W1 + k * NH + n];
-  } else if (idx < F_L4) {
-    const int j = idx < F_L3 ? idx - F_L2 : idx - F_L3, off = idx < F_L3 ? OFF_W2 : OFF_W3;
-    const int fr = j / 512, ob = fr / 4, kb = fr % 4, l = (j / 8) % 64, i = j % 8;
-    const int n = 16 * ob + l % 16, k = 32 * kb + slot32(l / 16, i);
-    w = p[off + k * NH + n];
-  } else {
-    const int j = idx - F_L4, kb = j / 512, l = (j / 8) % 64, i = j % 8;
-    const int n = l % 16, k = 32 * kb + slot32(l / 16, i);
-    if (n < CRM_MLP_NOUT) w = p[OFF_W4 + k * CRM_MLP_NOUT + n];
-  }
-  F[idx] = to_bf16(w);
-}
-
 __device__ __forceinline__ f4 mfma32(u4 a, u4 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
 }
@@ -411,17 +513,13 @@ struct crm_mlp {
   int device = 0;
   hipStream_t s = nullptr;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // packed FP32
-  bf16 *W1 = nullptr, *W2 = nullptr, *W3 = nullptr, *W4 = nullptr;
-  bf16* F = nullptr;  // weights in the fragment order of the fused inference
-  int ncu = 0;        // compute units of the device (persistent inference grid)
-  float *b1 = nullptr, *b2 = nullptr, *b3 = nullptr, *b4 = nullptr;
-  float* gpad = nullptr;  // gW1 gW2 gW3 gW4 gb1 gb2 gb3 gb4, contiguous
+  Weights w{};
+  int ncu = 0;            // compute units of the device (persistent grids)
   float* norm = nullptr;  // [NORM_SIZE]
   float host_norm[NORM_SIZE] = {};
-  float* loss = nullptr;
-  long cap = 0;  // rows of the work buffers
-  bf16 *Xn = nullptr, *H1 = nullptr, *H2 = nullptr, *H3 = nullptr, *dY = nullptr, *dA = nullptr, *dB = nullptr;
-  float* Y = nullptr;
+  float* loss = nullptr;  // pinned host memory, written by k_reduce
+  int cap = 0;            // workgroups' shares in part
+  float* part = nullptr;
   long step = 0;
 };
 
@@ -434,98 +532,31 @@ void launch_infer(hipStream_t s, const crm_mlp* m, const float* X, long n, float
   if (n > 0) k_infer<MODE><<<dim3((unsigned)grid), dim3(256), 0, s>>>(X, n, mlp_view(m), Y);
 }
 
-constexpr size_t GPAD = (size_t)KP * NH + 2 * NH * NH + NH * NP + 3 * NH + NP;
-
 #define MLPCHECK(x)                                   \
   do {                                                \
     if ((x) != hipSuccess) return CRM_ERR_DEVICE;     \
   } while (0)
 
-int ensure_rows(crm_mlp* m, long rows) {
-  if (rows <= m->cap) return CRM_OK;
-  bf16* bufs[] = {m->Xn, m->H1, m->H2, m->H3, m->dY, m->dA, m->dB};
-  for (bf16* b : bufs)
-    if (b) (void)hipFree(b);
-  if (m->Y) (void)hipFree(m->Y);
-  m->cap = 0;
-  MLPCHECK(hipMalloc(&m->Xn, rows * KP * sizeof(bf16)));
-  MLPCHECK(hipMalloc(&m->H1, rows * NH * sizeof(bf16)));
-  MLPCHECK(hipMalloc(&m->H2, rows * NH * sizeof(bf16)));
-  MLPCHECK(hipMalloc(&m->H3, rows * NH * sizeof(bf16)));
-  MLPCHECK(hipMalloc(&m->dY, rows * NP * sizeof(bf16)));
-  MLPCHECK(hipMalloc(&m->dA, rows * NH * sizeof(bf16)));
-  MLPCHECK(hipMalloc(&m->dB, rows * NH * sizeof(bf16)));
-  MLPCHECK(hipMalloc(&m->Y, rows * NP * sizeof(float)));
-  m->cap = rows;
-  return CRM_OK;
-}
-
-template <int EPI>
-void gemm(hipStream_t s, const bf16* A, long sam, long sak, const bf16* B, long sbk, long sbn, int M, int N, int K,
-          const float* bias, const bf16* mask, long smm, float* Cf, bf16* Cb, long ldc, int ksplit = 1) {
-  const long waves = (long)(M / 16) * (N / 16);
-  int kchunk = K;
-  if (ksplit > 1) kchunk = ((K / ksplit + 15) / 16) * 16;
-  const int ny = (K + kchunk - 1) / kchunk;
-  dim3 grid((unsigned)((waves + 3) / 4), (unsigned)ny);
-  k_gemm<EPI><<<grid, dim3(256), 0, s>>>(A, sam, sak, B, sbk, sbn, M, N, K, kchunk, bias, mask, smm, Cf, Cb, ldc);
-}
-
-// forward pass of mp (padded) rows already in Xn; leaves H1..H3 and the normalised Y
-void forward_rows(crm_mlp* m, int mp) {
-  hipStream_t s = m->s;
-  gemm<EPI_BIAS_RELU_BF16>(s, m->Xn, KP, 1, m->W1, NH, 1, mp, NH, KP, m->b1, nullptr, 0, nullptr, m->H1, NH);
-  gemm<EPI_BIAS_RELU_BF16>(s, m->H1, NH, 1, m->W2, NH, 1, mp, NH, NH, m->b2, nullptr, 0, nullptr, m->H2, NH);
-  gemm<EPI_BIAS_RELU_BF16>(s, m->H2, NH, 1, m->W3, NH, 1, mp, NH, NH, m->b3, nullptr, 0, nullptr, m->H3, NH);
-  gemm<EPI_BIAS_F32>(s, m->H3, NH, 1, m->W4, NP, 1, mp, NP, NH, m->b4, nullptr, 0, m->Y, nullptr, NP);
-}
-
-// loss and gradients into gpad for n rows of X/T (device)
-int backward(crm_mlp* m, const float* X, const float* T, int n) {
-  hipStream_t s = m->s;
-  const int mp = (n + 15) / 16 * 16;
-  int rc = ensure_rows(m, mp);
-  if (rc) return rc;
-  k_inputs<<<dim3((unsigned)(((long)mp * KP + 255) / 256)), dim3(256), 0, s>>>(X, n, mp, m->norm, m->Xn);
-  forward_rows(m, mp);
-  MLPCHECK(hipMemsetAsync(m->loss, 0, sizeof(float), s));
-  MLPCHECK(hipMemsetAsync(m->gpad, 0, GPAD * sizeof(float), s));
-  k_loss<<<dim3((unsigned)std::min<long>(((long)mp * NP + 255) / 256, 256)), dim3(256), 0, s>>>(m->Y, T, n, mp, m->norm,
-                                                                                               m->dY, m->loss);
-  float* gW1 = m->gpad;
-  float* gW2 = gW1 + KP * NH;
-  float* gW3 = gW2 + NH * NH;
-  float* gW4 = gW3 + NH * NH;
-  float* gb1 = gW4 + NH * NP;
-  float* gb2 = gb1 + NH;
-  float* gb3 = gb2 + NH;
-  float* gb4 = gb3 + NH;
-  const int ks = std::max(1, mp / 256);  // split the batch reduction of the weight gradients
-  const dim3 cs(2, 64);
-  // layer 4
-  gemm<EPI_ATOMIC_F32>(s, m->H3, 1, NH, m->dY, NP, 1, NH, NP, mp, nullptr, nullptr, 0, gW4, nullptr, NP, ks);
-  k_colsum<<<dim3(1, 64), dim3(256), 0, s>>>(m->dY, mp, NP, NP, gb4);
-  gemm<EPI_MASK_BF16>(s, m->dY, NP, 1, m->W4, 1, NP, mp, NH, NP, nullptr, m->H3, NH, nullptr, m->dA, NH);
-  // layer 3
-  gemm<EPI_ATOMIC_F32>(s, m->H2, 1, NH, m->dA, NH, 1, NH, NH, mp, nullptr, nullptr, 0, gW3, nullptr, NH, ks);
-  k_colsum<<<cs, dim3(256), 0, s>>>(m->dA, mp, NH, NH, gb3);
-  gemm<EPI_MASK_BF16>(s, m->dA, NH, 1, m->W3, 1, NH, mp, NH, NH, nullptr, m->H2, NH, nullptr, m->dB, NH);
-  // layer 2
-  gemm<EPI_ATOMIC_F32>(s, m->H1, 1, NH, m->dB, NH, 1, NH, NH, mp, nullptr, nullptr, 0, gW2, nullptr, NH, ks);
-  k_colsum<<<cs, dim3(256), 0, s>>>(m->dB, mp, NH, NH, gb2);
-  gemm<EPI_MASK_BF16>(s, m->dB, NH, 1, m->W2, 1, NH, mp, NH, NH, nullptr, m->H1, NH, nullptr, m->dA, NH);
-  // layer 1
-  gemm<EPI_ATOMIC_F32>(s, m->Xn, 1, KP, m->dA, NH, 1, KP, NH, mp, nullptr, nullptr, 0, gW1, nullptr, NH, ks);
-  k_colsum<<<cs, dim3(256), 0, s>>>(m->dA, mp, NH, NH, gb1);
-  k_pack_grad<<<dim3((CRM_MLP_NPARAM + 255) / 256), dim3(256), 0, s>>>(gW1, gW2, gW3, gW4, gb1, gb2, gb3, gb4, m->g);
+// the forward and backward pass of n rows of X and T (device), and the sums of its shares
+template <bool ADAM>
+int step(crm_mlp* m, const float* X, const float* T, int n, float lr, float c1, float c2) {
+  const int np = (int)std::min<long>(((long)n + TROWS - 1) / TROWS, m->ncu);
+  if (np > m->cap) {
+    if (m->part) (void)hipFree(m->part);
+    m->part = nullptr;
+    m->cap = 0;
+    MLPCHECK(hipMalloc(&m->part, (size_t)np * PSTRIDE * sizeof(float)));
+    m->cap = np;
+  }
+  k_train<<<dim3((unsigned)np), dim3(256), 0, m->s>>>(X, T, n, m->w, m->norm, m->part);
+  k_reduce<ADAM><<<dim3(PSTRIDE / 64), dim3(256), 0, m->s>>>(m->part, np, n, m->g, m->p, m->m, m->v, lr, c1, c2, m->w,
+                                                            m->loss);
   MLPCHECK(hipGetLastError());
   return CRM_OK;
 }
 
-void unpack(crm_mlp* m) {
-  k_unpack<<<dim3((NH * NH + 255) / 256), dim3(256), 0, m->s>>>(m->p, m->W1, m->W2, m->W3, m->W4, m->b1, m->b2, m->b3,
-                                                                 m->b4);
-  k_frags<<<dim3((F_SIZE + 255) / 256), dim3(256), 0, m->s>>>(m->p, m->F);
+void place_params(crm_mlp* m) {
+  k_place<<<dim3((CRM_MLP_NPARAM + 255) / 256), dim3(256), 0, m->s>>>(m->p, m->w);
 }
 }  // namespace
 
@@ -544,16 +575,12 @@ int crm_mlp_create(crm_mlp** out, int device) {
             hipMalloc(&m->g, CRM_MLP_NPARAM * sizeof(float)) == hipSuccess &&
             hipMalloc(&m->m, CRM_MLP_NPARAM * sizeof(float)) == hipSuccess &&
             hipMalloc(&m->v, CRM_MLP_NPARAM * sizeof(float)) == hipSuccess &&
-            hipMalloc(&m->W1, KP * NH * sizeof(bf16)) == hipSuccess &&
-            hipMalloc(&m->W2, NH * NH * sizeof(bf16)) == hipSuccess &&
-            hipMalloc(&m->W3, NH * NH * sizeof(bf16)) == hipSuccess &&
-            hipMalloc(&m->W4, NH * NP * sizeof(bf16)) == hipSuccess &&
-            hipMalloc(&m->F, F_SIZE * sizeof(bf16)) == hipSuccess &&
-            hipMalloc(&m->b1, NH * sizeof(float)) == hipSuccess && hipMalloc(&m->b2, NH * sizeof(float)) == hipSuccess &&
-            hipMalloc(&m->b3, NH * sizeof(float)) == hipSuccess && hipMalloc(&m->b4, NP * sizeof(float)) == hipSuccess &&
-            hipMalloc(&m->gpad, GPAD * sizeof(float)) == hipSuccess &&
+            hipMalloc(&m->w.F, F_SIZE * sizeof(bf16)) == hipSuccess &&
+            hipMalloc(&m->w.T, T_SIZE * sizeof(bf16)) == hipSuccess &&
+            hipMalloc(&m->w.b1, NH * sizeof(float)) == hipSuccess && hipMalloc(&m->w.b2, NH * sizeof(float)) == hipSuccess &&
+            hipMalloc(&m->w.b3, NH * sizeof(float)) == hipSuccess && hipMalloc(&m->w.b4, NP * sizeof(float)) == hipSuccess &&
             hipMalloc(&m->norm, NORM_SIZE * sizeof(float)) == hipSuccess &&
-            hipMalloc(&m->loss, sizeof(float)) == hipSuccess;
+            hipHostMalloc(&m->loss, sizeof(float), hipHostMallocDefault) == hipSuccess;
   if (!ok) {
     crm_mlp_destroy(m);
     return CRM_ERR_NOMEM;
@@ -563,6 +590,9 @@ int crm_mlp_create(crm_mlp** out, int device) {
     return CRM_ERR_DEVICE;
   }
   (void)hipMemset(m->p, 0, CRM_MLP_NPARAM * sizeof(float));
+  (void)hipMemset(m->w.F, 0, F_SIZE * sizeof(bf16));
+  (void)hipMemset(m->w.T, 0, T_SIZE * sizeof(bf16));
+  (void)hipMemset(m->w.b4, 0, NP * sizeof(float));
   (void)hipMemset(m->m, 0, CRM_MLP_NPARAM * sizeof(float));
   (void)hipMemset(m->v, 0, CRM_MLP_NPARAM * sizeof(float));
   for (int c = 0; c < 16; c++) {
@@ -573,7 +603,7 @@ int crm_mlp_create(crm_mlp** out, int device) {
     m->host_norm[NORM_HI + c] = INFINITY;
   }
   (void)hipMemcpy(m->norm, m->host_norm, sizeof(m->host_norm), hipMemcpyHostToDevice);
-  unpack(m);
+  place_params(m);
   (void)hipStreamSynchronize(m->s);
   *out = m;
   return CRM_OK;
@@ -582,10 +612,10 @@ int crm_mlp_create(crm_mlp** out, int device) {
 int crm_mlp_destroy(crm_mlp* m) {
   if (!m) return CRM_ERR_ARG;
   (void)hipSetDevice(m->device);
-  void* bufs[] = {m->p, m->g, m->m, m->v, m->W1, m->W2, m->W3, m->W4, m->F, m->b1, m->b2, m->b3, m->b4, m->gpad,
-                  m->norm, m->loss, m->Xn, m->H1, m->H2, m->H3, m->dY, m->dA, m->dB, m->Y};
+  void* bufs[] = {m->p, m->g, m->m, m->v, m->w.F, m->w.T, m->w.b1, m->w.b2, m->w.b3, m->w.b4, m->norm, m->part};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
+  if (m->loss) (void)hipHostFree(m->loss);
   if (m->s) (void)hipStreamDestroy(m->s);
   delete m;
   return CRM_OK;
@@ -597,7 +627,7 @@ int crm_mlp_set_params(crm_mlp* m, const float* params) {
   MLPCHECK(hipMemsetAsync(m->m, 0, CRM_MLP_NPARAM * sizeof(float), m->s));
   MLPCHECK(hipMemsetAsync(m->v, 0, CRM_MLP_NPARAM * sizeof(float), m->s));
   m->step = 0;
-  unpack(m);
+  place_params(m);
   MLPCHECK(hipStreamSynchronize(m->s));
   return CRM_OK;
 }
@@ -642,25 +672,22 @@ int crm_mlp_forward(crm_mlp* m, const float* X, int n, float* Y) {
 
 int crm_mlp_grad(crm_mlp* m, const float* X, const float* T, int n, float* grad, float* loss) {
   if (!m || !X || !T || n < 1) return CRM_ERR_ARG;
-  int rc = backward(m, X, T, n);
+  int rc = step<false>(m, X, T, n, 0.f, 1.f, 1.f);
   if (rc) return rc;
   if (grad) MLPCHECK(hipMemcpyAsync(grad, m->g, CRM_MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, m->s));
-  if (loss) MLPCHECK(hipMemcpyAsync(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost, m->s));
   MLPCHECK(hipStreamSynchronize(m->s));
+  if (loss) *loss = *m->loss;
   return CRM_OK;
 }
 
 int crm_mlp_train_step(crm_mlp* m, const float* X, const float* T, int n, float lr, float* loss) {
   if (!m || !X || !T || n < 1 || !(lr > 0.f)) return CRM_ERR_ARG;
-  int rc = backward(m, X, T, n);
+  const float k = (float)(m->step + 1), c1 = 1.f - std::pow(0.9f, k), c2 = 1.f - std::pow(0.999f, k);
+  int rc = step<true>(m, X, T, n, lr, c1, c2);
   if (rc) return rc;
   m->step++;
-  const float c1 = 1.f - std::pow(0.9f, (float)m->step), c2 = 1.f - std::pow(0.999f, (float)m->step);
-  k_adam<<<dim3((CRM_MLP_NPARAM + 255) / 256), dim3(256), 0, m->s>>>(m->p, m->g, m->m, m->v, lr, c1, c2);
-  unpack(m);
-  if (loss) MLPCHECK(hipMemcpyAsync(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost, m->s));
-  MLPCHECK(hipGetLastError());
   MLPCHECK(hipStreamSynchronize(m->s));
+  if (loss) *loss = *m->loss;
   return CRM_OK;
 }
 
@@ -670,15 +697,11 @@ int crm_mlp_train_step(crm_mlp* m, const float* X, const float* T, int n, float 
 namespace crm_mlp_ns {
 MlpView mlp_view(const crm_mlp* m) {
   MlpView v;
-  v.W1 = m->W1;
-  v.W2 = m->W2;
-  v.W3 = m->W3;
-  v.W4 = m->W4;
-  v.F = m->F;
-  v.b1 = m->b1;
-  v.b2 = m->b2;
-  v.b3 = m->b3;
-  v.b4 = m->b4;
+  v.F = m->w.F;
+  v.b1 = m->w.b1;
+  v.b2 = m->w.b2;
+  v.b3 = m->w.b3;
+  v.b4 = m->w.b4;
   v.norm = m->norm;
   return v;
 }

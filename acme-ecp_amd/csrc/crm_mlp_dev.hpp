@@ -36,11 +36,9 @@ __device__ __forceinline__ bf16 to_bf16(float x) {  // round to nearest, ties to
 }
 __device__ __forceinline__ float from_bf16(bf16 h) { return __uint_as_float((unsigned)h << 16); }
 
-// Device-side view of a network: padded BF16 weights W1[16][128], W2, W3 [128][128],
-// W4[128][16], the same weights in the fragment order of the fused inference (F), FP32 biases
-// (b4 padded to 16), the normalisation block.
+// Device-side view of a network: BF16 weights in the fragment order of the fused inference (F),
+// FP32 biases (b4 padded to 16), the normalisation block.
 struct MlpView {
-  const bf16 *W1 = nullptr, *W2 = nullptr, *W3 = nullptr, *W4 = nullptr;
   const bf16* F = nullptr;
   const float *b1 = nullptr, *b2 = nullptr, *b3 = nullptr, *b4 = nullptr;
   const float* norm = nullptr;
