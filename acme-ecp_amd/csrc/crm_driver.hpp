@@ -475,82 +475,36 @@ static int upload_transform(Engine<R>* ctx, int nx, int ny, double dx, Transform
 
 // ---- kernel dispatch over the compile-time column count ------------------------------------
 // Launch variants ("tile shapes") the autotuner chooses among, per kernel class: the pressure
-// solve of 2D 64-column CRMs has five (0: chosen by the batch's size; 1: one instance on 8 waves
-// with every level's inputs of the gradient pass kept in registers, one workgroup per CU; 2 and
-// 3: one instance per 4-wave workgroup, two workgroups per CU, two or four levels of each pass
-// unrolled together; 4: the same, one level at a time, with the Thomas factors in registers, so
-// that the workgroup needs only the slab of LDS), MPDATA six (0: chosen by the batch's size; 1:
-// the other number of levels per trip; 2, 3: as the default and 1 with registers bounded for
-// three waves per SIMD; 4: the default number of levels, registers unbounded; 5: as 2).  Results
-// are bitwise the same in every variant of a class.
+// solve of 2D 64-column CRMs has five (waves of an instance's workgroup x levels whose loads a
+// wave issues together: 0 8 x 4, 1 8 x 2, 2 4 x 4, 3 4 x 2, 4 16 x 2), MPDATA six (0: chosen by the
+// batch's size; 1: the other number of levels per trip; 2, 3: as the default and 1 with registers
+// bounded for three waves per SIMD; 4: the default number of levels, registers unbounded; 5: as
+// 2).  Results are bitwise the same in every variant of a class.
+//
+// 8 x 4 was the fastest or within 2% of it at every size of the pressure solve that was timed (us
+// of a launch, 8 x 4 against the best of 1 to 4: 4096 x 64 x 28 508 and 508, mixed 295 and 298;
+// 500 x 64 x 58 65 and 66), so the other column counts have no variants.
 static int variants_of(int kid, int nx, bool y3) {
   if (kid == CRM_K_PRESS) return (nx == 64 && !y3) ? 5 : 1;
   if (kid == CRM_K_MPDATA) return 6;
   return 1;
 }
 
+template <int NX, typename R, typename G, int NW, int PB>
+static void start_press(int nzm, hipStream_t s, const DevT<R>& d, int na, int nb, int nc) {
+  constexpr int NI = PressShape<NX>::NI;
+  k_press<NX, R, G, NW, PB><<<dim3((unsigned)((d.ncrms + NI - 1) / NI)), dim3(64 * NW), PressShape<NX>::lds_bytes(nzm), s>>>(
+      d, na, nb, nc);
+}
 template <int NX, typename R, typename G>
-static void launch_press(int nzm, dim3 g, dim3 b, size_t sh, hipStream_t s, const DevT<R>& d, int na, int nb, int nc,
-                         int variant) {
-  // 28 and 58 levels (the reference's SP configurations) have compile-time level loops; any
-  // other level count up to 64 runs the same kernels with the count read at run time (NZM 0)
-  const bool z28 = nzm == 28, z58 = nzm == 58;
-  const dim3 gi((unsigned)d.ncrms);
-  if constexpr (NX == 64 && !G::Y3) {  // matrix-core transforms
-    // variant 0: the factors in registers once more instances wait than two workgroups per CU
-    // hold (4096 x 64 x 58: 590 -> 535 us FP64, 390 -> 345 mixed), else the 0 below (500 x 64 x
-    // 58: 75 against 78 us)
-    if (variant == 0 && d.ncrms > 512) variant = 4;
-    if (!z28 && !z58) {
-      k_press64<0, R, G><<<gi, b, press64_lds_bytes<0>(), s>>>(d, na, nb, nc);
-    } else if (variant == 0) {  // one instance per 4-wave block
-      if (z28)
-        k_press64<28, R, G><<<gi, b, press64_lds_bytes<28>(), s>>>(d, na, nb, nc);
-      else
-        k_press64<58, R, G><<<gi, b, press64_lds_bytes<58>(), s>>>(d, na, nb, nc);
-    } else if (variant == 2) {  // the same, two levels per trip
-      if (z28)
-        k_press64<28, R, G, 2><<<gi, b, press64_lds_bytes<28>(), s>>>(d, na, nb, nc);
-      else
-        k_press64<58, R, G, 2><<<gi, b, press64_lds_bytes<58>(), s>>>(d, na, nb, nc);
-    } else if (variant == 3) {  // the same, four levels per trip
-      if (z28)
-        k_press64<28, R, G, 4><<<gi, b, press64_lds_bytes<28>(), s>>>(d, na, nb, nc);
-      else
-        k_press64<58, R, G, 4><<<gi, b, press64_lds_bytes<58>(), s>>>(d, na, nb, nc);
-    } else if (variant == 4) {  // variant 0 with the Thomas factors in registers
-      if (z28)
-        k_press64<28, R, G, 1, true><<<gi, b, press64_slab_bytes(), s>>>(d, na, nb, nc);
-      else
-        k_press64<58, R, G, 1, true><<<gi, b, press64_slab_bytes(), s>>>(d, na, nb, nc);
-    } else {  // one instance per 8-wave block, inputs of the gradient pass in registers
-      if (z28)
-        k_press64r<28, R><<<gi, dim3(512), press64_lds_bytes<28>(), s>>>(d, na, nb, nc);
-      else
-        k_press64r<58, R><<<gi, dim3(512), press64_lds_bytes<58>(), s>>>(d, na, nb, nc);
-    }
-  } else if constexpr (NX == 64) {  // 3D 8 x 8: one instance per 4-wave block
-    if (z28)
-      k_press64<28, R, G><<<gi, b, press64_lds_bytes<28>(), s>>>(d, na, nb, nc);
-    else if (z58)
-      k_press64<58, R, G><<<gi, b, press64_lds_bytes<58>(), s>>>(d, na, nb, nc);
-    else
-      k_press64<0, R, G><<<gi, b, press64_lds_bytes<0>(), s>>>(d, na, nb, nc);
-  } else if constexpr (NX == 128) {  // one instance per block of 4 waves
-    if (z28)
-      k_press128<28, R><<<gi, b, (size_t)28 * 128 * sizeof(double), s>>>(d, na, nb, nc);
-    else if (z58)
-      k_press128<58, R><<<gi, b, (size_t)58 * 128 * sizeof(double), s>>>(d, na, nb, nc);
-    else  // the Thomas factors in LDS after the slab
-      k_press128<0, R><<<gi, b, (size_t)2 * nzm * 128 * sizeof(double), s>>>(d, na, nb, nc);
-  } else {
-    if (z28)
-      k_press<NX, 28, R, G><<<g, b, sh, s>>>(d, na, nb, nc);
-    else if (z58)
-      k_press<NX, 58, R, G><<<g, b, sh, s>>>(d, na, nb, nc);
-    else  // the Thomas factors in LDS after the slab
-      k_press<NX, 0, R, G><<<g, b, 2 * sh, s>>>(d, na, nb, nc);
+static void launch_press(int nzm, hipStream_t s, const DevT<R>& d, int na, int nb, int nc, int variant) {
+  if constexpr (NX == 64 && !G::Y3) {
+    if (variant == 1) return start_press<NX, R, G, 8, 2>(nzm, s, d, na, nb, nc);
+    if (variant == 2) return start_press<NX, R, G, 4, 4>(nzm, s, d, na, nb, nc);
+    if (variant == 3) return start_press<NX, R, G, 4, 2>(nzm, s, d, na, nb, nc);
+    if (variant == 4) return start_press<NX, R, G, 16, 2>(nzm, s, d, na, nb, nc);
   }
+  start_press<NX, R, G, 8, 4>(nzm, s, d, na, nb, nc);
 }
 
 // o: where the advected fields go (their own buffers, or the hand-over buffers of split sweeps)
@@ -932,10 +886,6 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
   d.samp_stride = ctx->samp_stride;
   double dt3[3] = {0.0, 0.0, 0.0};
   int na = 0, nb = 1, nc = 2;
-  // k_press: the 64/nx instances of one wave per block (k_press64, k_press128: one per block)
-  const int press_per_block = nx < 64 ? 64 / nx : 1;
-  const dim3 gpress((unsigned)((ncrms + press_per_block - 1) / press_per_block));
-  const size_t press_lds = (size_t)nzm * 64 * sizeof(double);
   unsigned long long err_flag = 0;
   unsigned long long tail[2] = {0, 0};  // read back after the call: the largest nprec, the error flag
   HIPCHECK(hipEventRecord(ctx->ev0, s));
@@ -1001,7 +951,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
           NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad)));
           NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
           NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
-          NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, gpress, b256, press_lds, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
+          NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
           k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
           NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA])));
           NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp)));
@@ -1112,7 +1062,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
         NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad)));
         NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
         NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
-        NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, gpress, b256, press_lds, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
+        NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
         k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
         NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA])));
         NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp)));
@@ -1179,7 +1129,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       if (last && phase_stop == 9) goto stopped;
       TIMED(CRM_K_MOM, NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na))));
       if (last && phase_stop == 11) goto stopped;
-      TIMED(CRM_K_PRESS, NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, gpress, b256, press_lds, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS]))));
+      TIMED(CRM_K_PRESS, NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS]))));
       if (last && phase_stop == 13) goto stopped;
       k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
       TIMED(CRM_K_MPDATA, NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA]))));

@@ -1228,361 +1228,69 @@ __global__ void CRM_LB k_mom(DevT<R> d, int na) {
 // Pressure: press_rhs.F90:8-106, the fft991 x-transform as dense operators (see
 // fft991_operator.hpp; in 3D the x-y Kronecker operator, dy == dx), the vertical Thomas sweep
 // of pressure.F90:160-237, the inverse transform, press_grad.F90:8-76, then adams.F90:7-40.
-// 4 waves share the 64/NX instances of one wave; levels are dealt round-robin to the waves;
-// the slab lives in LDS; the Thomas sweep runs on wave 0 with its factor in registers (NZM
-// compile-time) or, for NZM == 0 (any level count, read from d.nzm), in LDS after the slab.
-// ------------------------------------------------------------------------------------------
-template <int NX, int NZM, typename R, typename G = SegFor<NX>>
-__global__ void CRM_LB k_press(DevT<R> d, int na, int nb, int nc) {
-  CRM_STOP_CHECK(d);
-  extern __shared__ double slab[];  // [64/NX instances][nzm][NX] == [nzm][64] per lane column
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = lane & (NX - 1);
-  const int cg = blockIdx.x * (64 / NX) + lane / NX;
-  const bool live = cg < d.ncrms;
-  const int c = live ? cg : d.ncrms - 1;
-  G s;
-  const int nzm = NZM > 0 ? NZM : d.nzm, nz = nzm + 1;
-  const double dz = inst(d, I_DZ, c);
-  const double* adz = prof(d, P_ADZ, c);
-  const double* adzw = prof(d, P_ADZW, c);
-  const double* rho = prof(d, P_RHO, c);
-  const double* rhow = prof(d, P_RHOW, c);
-  auto P = [&](int k, int col) -> double& { return slab[(size_t)k * 64 + (lane - i) + col]; };
-  const double rdx = 1. / d.dx, btat = d.bt / d.at, ctat = d.ct / d.at;
-  const double dta = 1. / d.dt3na / d.at;
-  const R *ua = d.dudt[na], *ub = d.dudt[nb], *uc = d.dudt[nc];
-  const R *wa = d.dwdt[na], *wb = d.dwdt[nb], *wc = d.dwdt[nc];
-  // 1. right-hand side
-  for (int k = wave; k < nzm; k += 4) {
-    size_t o = ((size_t)c * nzm + k) * NX + i;
-    size_t ow = ((size_t)c * nz + k) * NX + i;
-    size_t own = ow + NX;
-    double rdz = 1. / (adz[k] * dz);
-    double rup = rhow[k + 1] / rho[k] * rdz;
-    double rdn = rhow[k] / rho[k] * rdz;
-    double uu = d.u[o], uap = ua[o], ubp = ub[o], ucp = uc[o];
-    double pv;
-    if constexpr (G::Y3) {  // press_rhs.F90:45-69
-      double vv = d.v[o], vap = d.dvdt[na][o], vbp = d.dvdt[nb][o], vcp = d.dvdt[nc][o];
-      pv = (rdx * (s.rot(uu, 1) - uu) + rdx * (s.roty(vv, 1) - vv) + (d.w[own] * rup - d.w[ow] * rdn)) * dta +
-           (rdx * (s.rot(uap, 1) - uap) + rdx * (s.roty(vap, 1) - vap) + (wa[own] * rup - wa[ow] * rdn)) +
-           btat * (rdx * (s.rot(ubp, 1) - ubp) + rdx * (s.roty(vbp, 1) - vbp) + (wb[own] * rup - wb[ow] * rdn)) +
-           ctat * (rdx * (s.rot(ucp, 1) - ucp) + rdx * (s.roty(vcp, 1) - vcp) + (wc[own] * rup - wc[ow] * rdn));
-    } else {
-      pv = (rdx * (s.rot(uu, 1) - uu) + (d.w[own] * rup - d.w[ow] * rdn)) * dta +
-           (rdx * (s.rot(uap, 1) - uap) + (wa[own] * rup - wa[ow] * rdn)) +
-           btat * (rdx * (s.rot(ubp, 1) - ubp) + (wb[own] * rup - wb[ow] * rdn)) +
-           ctat * (rdx * (s.rot(ucp, 1) - ucp) + (wc[own] * rup - wc[ow] * rdn));
-    }
-    P(k, i) = pv * rho[k];
-  }
-  __syncthreads();
-  // 2. forward transform: slot m of level k (every lane reads the whole row before any
-  // lane overwrites its entry, hence the barrier between the sum and the store)
-  for (int k0 = 0; k0 < nzm; k0 += 4) {
-    const int k = k0 + wave;
-    double acc = 0.0;
-    if (k < nzm) {
-#pragma unroll 8
-      for (int q = 0; q < NX; q++) acc += d.Ft[q * NX + i] * P(k, q);
-    }
-    __syncthreads();
-    if (k < nzm) P(k, i) = acc;
-  }
-  __syncthreads();
-  // 3. Thomas sweep per slot (wave 0)
-  if (wave == 0) {
-    const double eig = d.eign[i];
-    constexpr int NA = NZM > 0 ? NZM : 1;
-    double alfa_r[NA];
-    double* alfa_l = slab + (size_t)nzm * 64;
-    auto alfa = [&](int k) -> double& {
-      if constexpr (NZM > 0)
-        return alfa_r[k];
-      else
-        return alfa_l[(size_t)k * 64 + lane];
-    };
-    auto acoef = [&](int k) { return rhow[k] / (adz[k] * adzw[k] * dz * dz); };
-    auto ccoef = [&](int k) { return rhow[k + 1] / (adz[k] * adzw[k + 1] * dz * dz); };
-    double b;
-    if (i == 0)
-      b = 1.0 / (eig * rho[0] - acoef(0) - ccoef(0));
-    else
-      b = 1.0 / (eig * rho[0] - ccoef(0));
-    alfa(0) = -ccoef(0) * b;
-    double beta = P(0, i) * b;
-    P(0, i) = beta;
-    auto down = [&](int k) {
-      double ak = acoef(k), ck = ccoef(k);
-      double e = 1.0 / (eig * rho[k] - ak - ck + ak * alfa(k - 1));
-      alfa(k) = -ck * e;
-      beta = (P(k, i) - ak * beta) * e;
-      P(k, i) = beta;
-    };
-    // unrolled with a compile-time level count, so the factors stay in registers
-    if constexpr (NZM > 0) {
-#pragma unroll
-      for (int k = 1; k < NZM - 1; k++) down(k);
-    } else {
-      for (int k = 1; k < nzm - 1; k++) down(k);
-    }
-    {
-      int k = nzm - 1;
-      double ak = acoef(k);
-      double top = (P(k, i) - ak * beta) / (eig * rho[k] - ak + ak * alfa(k - 1));
-      P(k, i) = top;
-      auto up = [&](int kk) {
-        top = alfa(kk) * top + P(kk, i);
-        P(kk, i) = top;
-      };
-      if constexpr (NZM > 0) {
-#pragma unroll
-        for (int kk = NZM - 2; kk >= 0; kk--) up(kk);
-      } else {
-        for (int kk = nzm - 2; kk >= 0; kk--) up(kk);
-      }
-    }
-  }
-  __syncthreads();
-  // 4. inverse transform (same read-all-then-store pattern)
-  for (int k0 = 0; k0 < nzm; k0 += 4) {
-    const int k = k0 + wave;
-    double acc = 0.0;
-    if (k < nzm) {
-#pragma unroll 8
-      for (int q = 0; q < NX; q++) acc += d.Gt[q * NX + i] * P(k, q);
-    }
-    __syncthreads();
-    if (k < nzm) P(k, i) = acc;
-  }
-  __syncthreads();
-  // 5. pressure gradient, then Adams-Bashforth and the half-step Courant velocities
-  const double dtdx = d.dtn / d.dx, dtdz = d.dtn / dz, dt3 = d.dt3na;
-  R* uan = d.dudt[na];
-  R* wan = d.dwdt[na];
-  R* unc = d.dudt[nc];
-  R* wnc = d.dwdt[nc];
-  for (int k = wave; k < nzm; k += 4) {
-    size_t o = ((size_t)c * nzm + k) * NX + i;
-    size_t ow = ((size_t)c * nz + k) * NX + i;
-    double pk = P(k, i);
-    double pim = s.rot(pk, -1);
-    double pkb = P(k > 0 ? k - 1 : 0, i);
-    double rdz = 1. / (dz * adzw[k]);
-    double du_a = ua[o] - (pk - pim) * rdx;
-    double dw_a = wa[ow] - (pk - pkb) * rdz;
-    double uu = d.u[o], ww = d.w[ow];
-    double un = uu + dt3 * (d.at * du_a + d.bt * ub[o] + d.ct * uc[o]);
-    double wn = ww + dt3 * (d.at * dw_a + d.bt * wb[ow] + d.ct * wc[ow]);
-    double dv_a = 0.0, vn = 0.0, vv = 0.0;
-    if constexpr (G::Y3) {  // press_grad.F90:29, adams.F90:29,32
-      double pjm = s.roty(pk, -1);
-      dv_a = d.dvdt[na][o] - (pk - pjm) * rdx;
-      vv = d.v[o];
-      vn = vv + dt3 * (d.at * dv_a + d.bt * d.dvdt[nb][o] + d.ct * d.dvdt[nc][o]);
-    }
-    if (live) {
-      uan[o] = du_a;
-      wan[ow] = dw_a;
-      unc[o] = un;
-      wnc[ow] = wn;
-      d.u[o] = 0.5 * (uu + un) * (rho[k] * dtdx);
-      d.w[ow] = 0.5 * (ww + wn) * (rhow[k] * dtdz);
-      if constexpr (G::Y3) {
-        d.dvdt[na][o] = dv_a;
-        d.dvdt[nc][o] = vn;
-        d.v[o] = 0.5 * (vv + vn) * (rho[k] * dtdx);
-      }
-    }
-  }
-  if (wave == 0 && live) wnc[((size_t)c * nz + nzm) * NX + i] = 0.0;
-}
-
-// ------------------------------------------------------------------------------------------
-// Pressure for 128-column CRMs: k_press's algorithm and operation order with one instance per
-// block of 4 waves, as two groups of 128 columns to which the levels are dealt alternately.
-// The slab [NZM][128] lives in LDS.  Column neighbours are read from memory (right-hand side)
-// or from the slab (gradient), so no cross-wave exchange is needed; the Thomas sweep runs on
-// group 0.
-// ------------------------------------------------------------------------------------------
-template <int NZM, typename R>
-__global__ void CRM_LB k_press128(DevT<R> d, int na, int nb, int nc) {
-  CRM_STOP_CHECK(d);
-  constexpr int NX = 128;
-  extern __shared__ double slab[];  // [nzm][128]
-  const int i = threadIdx.x & (NX - 1), grp = threadIdx.x >> 7;
-  const int c = blockIdx.x;  // one block per instance
-  const int ip = (i + 1) & (NX - 1), im = (i - 1) & (NX - 1);
-  const int nzm = NZM > 0 ? NZM : d.nzm, nz = nzm + 1;
-  const double dz = inst(d, I_DZ, c);
-  const double* adz = prof(d, P_ADZ, c);
-  const double* adzw = prof(d, P_ADZW, c);
-  const double* rho = prof(d, P_RHO, c);
-  const double* rhow = prof(d, P_RHOW, c);
-  auto P = [&](int k, int col) -> double& { return slab[(size_t)k * NX + col]; };
-  const double rdx = 1. / d.dx, btat = d.bt / d.at, ctat = d.ct / d.at;
-  const double dta = 1. / d.dt3na / d.at;
-  const R *ua = d.dudt[na], *ub = d.dudt[nb], *uc = d.dudt[nc];
-  const R *wa = d.dwdt[na], *wb = d.dwdt[nb], *wc = d.dwdt[nc];
-  // 1. right-hand side
-  for (int k = grp; k < nzm; k += 2) {
-    const size_t row = ((size_t)c * nzm + k) * NX, o = row + i, op = row + ip;
-    const size_t ow = ((size_t)c * nz + k) * NX + i, own = ow + NX;
-    double rdz = 1. / (adz[k] * dz);
-    double rup = rhow[k + 1] / rho[k] * rdz;
-    double rdn = rhow[k] / rho[k] * rdz;
-    double uu = d.u[o], uap = ua[o], ubp = ub[o], ucp = uc[o];
-    double pv = (rdx * ((double)d.u[op] - uu) + (d.w[own] * rup - d.w[ow] * rdn)) * dta +
-                (rdx * ((double)ua[op] - uap) + (wa[own] * rup - wa[ow] * rdn)) +
-                btat * (rdx * ((double)ub[op] - ubp) + (wb[own] * rup - wb[ow] * rdn)) +
-                ctat * (rdx * ((double)uc[op] - ucp) + (wc[own] * rup - wc[ow] * rdn));
-    P(k, i) = pv * rho[k];
-  }
-  // one 128-point transform of every level of the slab in place, P(k, i) <- sum_q M[q][i]
-  // P(k, q): each operator entry is read once and applied to all of the group's levels (an
-  // accumulator per level in registers, each summed in q order as a per-level loop would);
-  // every level is read before any is overwritten
-  constexpr int NJ = (NZM > 0 ? NZM : 64) / 2 + 1;  // levels per group, an upper bound
-  auto transform = [&](const double* __restrict__ M) {
-    double acc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) acc[j] = 0.0;
-    __syncthreads();
-    for (int q = 0; q < NX; q++) {
-      const double m = M[q * NX + i];
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        const int k = grp + 2 * j;
-        if (k < nzm) acc[j] += m * P(k, q);
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-      const int k = grp + 2 * j;
-      if (k < nzm) P(k, i) = acc[j];
-    }
-    __syncthreads();
-  };
-  // 2. forward transform
-  transform(d.Ft);
-  // 3. Thomas sweep per slot (group 0)
-  if (grp == 0) {
-    const double eig = d.eign[i];
-    constexpr int NA = NZM > 0 ? NZM : 1;
-    double alfa_r[NA];
-    double* alfa_l = slab + (size_t)nzm * NX;  // NZM == 0: the factors in LDS after the slab
-    auto alfa = [&](int k) -> double& {
-      if constexpr (NZM > 0)
-        return alfa_r[k];
-      else
-        return alfa_l[(size_t)k * NX + i];
-    };
-    auto acoef = [&](int k) { return rhow[k] / (adz[k] * adzw[k] * dz * dz); };
-    auto ccoef = [&](int k) { return rhow[k + 1] / (adz[k] * adzw[k + 1] * dz * dz); };
-    double b;
-    if (i == 0)
-      b = 1.0 / (eig * rho[0] - acoef(0) - ccoef(0));
-    else
-      b = 1.0 / (eig * rho[0] - ccoef(0));
-    alfa(0) = -ccoef(0) * b;
-    double beta = P(0, i) * b;
-    P(0, i) = beta;
-    auto down = [&](int k) {
-      double ak = acoef(k), ck = ccoef(k);
-      double e = 1.0 / (eig * rho[k] - ak - ck + ak * alfa(k - 1));
-      alfa(k) = -ck * e;
-      beta = (P(k, i) - ak * beta) * e;
-      P(k, i) = beta;
-    };
-    // unrolled with a compile-time level count, so the factors stay in registers
-    if constexpr (NZM > 0) {
-#pragma unroll
-      for (int k = 1; k < NZM - 1; k++) down(k);
-    } else {
-      for (int k = 1; k < nzm - 1; k++) down(k);
-    }
-    {
-      int k = nzm - 1;
-      double ak = acoef(k);
-      double top = (P(k, i) - ak * beta) / (eig * rho[k] - ak + ak * alfa(k - 1));
-      P(k, i) = top;
-      auto up = [&](int kk) {
-        top = alfa(kk) * top + P(kk, i);
-        P(kk, i) = top;
-      };
-      if constexpr (NZM > 0) {
-#pragma unroll
-        for (int kk = NZM - 2; kk >= 0; kk--) up(kk);
-      } else {
-        for (int kk = nzm - 2; kk >= 0; kk--) up(kk);
-      }
-    }
-  }
-  // 4. inverse transform (its leading barrier also ends the Thomas sweep)
-  transform(d.Gt);
-  // 5. pressure gradient, then Adams-Bashforth and the half-step Courant velocities
-  const double dtdx = d.dtn / d.dx, dtdz = d.dtn / dz, dt3 = d.dt3na;
-  R* uan = d.dudt[na];
-  R* wan = d.dwdt[na];
-  R* unc = d.dudt[nc];
-  R* wnc = d.dwdt[nc];
-  for (int k = grp; k < nzm; k += 2) {
-    size_t o = ((size_t)c * nzm + k) * NX + i;
-    size_t ow = ((size_t)c * nz + k) * NX + i;
-    double pk = P(k, i);
-    double pim = P(k, im);
-    double pkb = P(k > 0 ? k - 1 : 0, i);
-    double rdz = 1. / (dz * adzw[k]);
-    double du_a = ua[o] - (pk - pim) * rdx;
-    double dw_a = wa[ow] - (pk - pkb) * rdz;
-    double uu = d.u[o], ww = d.w[ow];
-    double un = uu + dt3 * (d.at * du_a + d.bt * ub[o] + d.ct * uc[o]);
-    double wn = ww + dt3 * (d.at * dw_a + d.bt * wb[ow] + d.ct * wc[ow]);
-    uan[o] = du_a;
-    wan[ow] = dw_a;
-    unc[o] = un;
-    wnc[ow] = wn;
-    d.u[o] = 0.5 * (uu + un) * (rho[k] * dtdx);
-    d.w[ow] = 0.5 * (ww + wn) * (rhow[k] * dtdz);
-  }
-  if (grp == 0) wnc[((size_t)c * nz + nzm) * NX + i] = 0.0;
-}
-
-// ------------------------------------------------------------------------------------------
-// Pressure for 64-column CRMs with the x-transforms on the matrix cores.  Same algorithm and
-// operation order per level as k_press; the two transforms are the GEMMs
-//   C[k][s] = sum_i P[k][i] Ft[i][s]   and   P'[k][i] = sum_s C[k][s] Gt[s][i]
-// (levels padded to 64 rows) done with v_mfma_f64_16x16x4f64: wave w owns output columns
-// 16w..16w+15 and keeps the matching 16 k-step fragments of Ft (then Gt) in registers; the
-// A fragments stream from the LDS slab.  One instance per block of 4 waves.
+// Workgroups of NW waves.  A row of the LDS slab is a level of the 64/NX instances of one wave (128
+// columns: of one instance, on two waves); the rows are dealt round-robin to the waves, and the
+// loads of PB of a wave's rows are issued before any is used.
+//
+// The transforms C[k][s] = sum_i P[k][i] F[i][s] of an instance's NX columns run on
+// v_mfma_f64_16x16x4f64: a wave makes 16 slots of some 16-level tiles, with its columns of the
+// operator in registers, and reads only its own instance's levels from the slab (so a non-finite
+// value stays in its instance).  The matrix cores add the products of an output one by one, each
+// fused and rounded (measured: the bits of a scalar fma chain in the same order), so the results
+// are those of the loop they replaced, an fma per operator entry and level: at 256 x 128 x 58
+// that loop's LDS reads and at 16 x 32 x 28 its re-reads of the operator made the two transforms
+// most of the kernel.
+//
+// A launch, before (the loops at 8, 16, 32 and 128 columns; 64: 4 waves, the factors in LDS or in
+// registers) -> now, us: 256 x 128 x 58 217 -> 88, 16 x 32 x 28 31 -> 18, 866 x 32 x 28 54 -> 30,
+// 1024 x 4x4 x 28 36 -> 24, 500 x 64 x 58 75 -> 65, 4096 x 64 x 28 535 -> 508 and mixed 345 -> 295.
+// Bound: memory, in phases.  The registers of the batched loads allow two workgroups of a CU, so
+// the transforms and the sweep of one are covered by the loads and stores of one other; at 4096
+// instances a launch moves 22 words per cell (8 of them again, for the gradient) at 2.5 TB/s.
+//
+// The Thomas sweep runs on one wave (128 columns: two), lane = slot, its factors in LDS.  The
+// level coefficients do not depend on the recurrence: all waves compute them before it, and the
+// sweep reads each level's coefficients and right-hand side one level ahead, so that it waits on
+// one division per level.
 //
 // MFMA f64 16x16x4 operand layout (lane l of the wave):
 //   A[16x4]: row l%16, col l/16      B[4x16]: row l/16, col l%16
 //   D[16x16]: element j of the result vector is row 4*j + l/16, col l%16
 // ------------------------------------------------------------------------------------------
 typedef double v4d __attribute__((ext_vector_type(4)));
-constexpr int PLD = 66;  // slab row stride in doubles: conflict-free A-fragment reads
 
-// UNR: levels of the right-hand side and gradient passes unrolled together, so that their
-// loads are in flight at once (a launch variant the autotuner may choose).  RALF: the Thomas
-// factors in registers of the sweeping wave instead of LDS (NZM > 0 only), so that the block
-// needs only the slab and three blocks fit a CU instead of two (another launch variant).
-template <int NZM, typename R, typename G = Seg<64>, int UNR = 1, bool RALF = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RALF ? 3 : CRM_WAVES_PER_EU)))
-k_press64(DevT<R> d, int na, int nb, int nc) {
+template <int NX>
+struct PressShape {
+  static constexpr int COLS = NX < 64 ? 64 : NX;   // columns of a slab row
+  static constexpr int NI = COLS / NX;             // instances of a workgroup
+  static constexpr int LD = COLS + 2;              // slab row stride: conflict-free A-fragment reads
+  static constexpr int WPR = COLS / 64;            // waves of a row
+  static size_t lds_bytes(int nzm) {
+    const size_t rows = (size_t)(nzm + 15) / 16 * 16;
+    return (rows * LD + (size_t)nzm * COLS + (size_t)3 * NI * nzm) * sizeof(double);
+  }
+};
+
+// NW: waves of the workgroup; PB: rows of a wave whose loads are issued together
+template <int NX, typename R, typename G, int NW = 8, int PB = 4>
+__global__ void __launch_bounds__(64 * NW) k_press(DevT<R> d, int na, int nb, int nc) {
   CRM_STOP_CHECK(d);
-  static_assert(!RALF || NZM > 0, "factors in registers: compile-time level count");
-  constexpr int NX = 64, NK = 64;
+  using SH = PressShape<NX>;
+  constexpr int COLS = SH::COLS, NI = SH::NI, LD = SH::LD, WPR = SH::WPR;
+  constexpr int RW = NW / WPR;  // rows in flight across the waves
   extern __shared__ double lds[];
-  const int c = blockIdx.x;  // grid is exactly ncrms blocks
-  double* P = lds;              // [NK][PLD] slab: rhs, coefficients, pressure
-  double* ALF = lds + NK * PLD; // [nzm][64] Thomas factors (not allocated with RALF)
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int i = lane;
-  G s;  // 3D (8 x 8 columns): the transforms are the x-y Kronecker operators, dy == dx
-  const int nzm = NZM > 0 ? NZM : d.nzm, nz = nzm + 1;
+  const int nzm = d.nzm, nz = nzm + 1;
+  double* P = lds;                                           // [rows][LD]: rhs, coefficients, pressure
+  double* ALF = P + (size_t)((nzm + 15) / 16 * 16) * LD;     // [nzm][COLS] Thomas factors
+  double* CA = ALF + (size_t)nzm * COLS;                     // [NI][nzm] a, c, rho of the sweep
+  double *CC = CA + NI * nzm, *CR = CC + NI * nzm;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int col = 64 * (wave % WPR) + lane, i = col & (NX - 1), w0 = wave / WPR;
+  const int cg = (int)blockIdx.x * NI + col / NX;
+  const bool live = cg < d.ncrms;
+  int c = live ? cg : d.ncrms - 1;
+  if constexpr (NX >= 64) c = __builtin_amdgcn_readfirstlane(c);
+  G s;
   const double dz = inst(d, I_DZ, c);
   const double* adz = prof(d, P_ADZ, c);
   const double* adzw = prof(d, P_ADZW, c);
@@ -1592,183 +1300,172 @@ k_press64(DevT<R> d, int na, int nb, int nc) {
   const double dta = 1. / d.dt3na / d.at;
   const R *ua = d.dudt[na], *ub = d.dudt[nb], *uc = d.dudt[nc];
   const R *wa = d.dwdt[na], *wb = d.dwdt[nb], *wc = d.dwdt[nc];
-  const int r16 = lane & 15, q4 = lane >> 4;
-  // 1. right-hand side (rows >= nzm of the slab are zero).  The loads of UNR levels are
-  // issued before any of them is used (2D), so that they are in flight together.
-  static_assert(UNR == 1 || !G::Y3, "levels per trip: 2D only");
-  for (int k0 = wave; k0 < NK; k0 += 4 * UNR) {
-    double ld_[UNR][12];
+  // the sweep's level coefficients
+  for (int t = threadIdx.x; t < NI * nzm; t += 64 * NW) {
+    const int g = t / nzm, k = t - g * nzm, cc = ::min((int)blockIdx.x * NI + g, d.ncrms - 1);
+    const double *adz_ = prof(d, P_ADZ, cc), *adzw_ = prof(d, P_ADZW, cc), *rhow_ = prof(d, P_RHOW, cc);
+    const double dz_ = inst(d, I_DZ, cc);
+    CA[t] = rhow_[k] / (adz_[k] * adzw_[k] * dz_ * dz_);
+    CC[t] = rhow_[k + 1] / (adz_[k] * adzw_[k + 1] * dz_ * dz_);
+    CR[t] = prof(d, P_RHO, cc)[k];
+  }
+  // value of the next column of a row: a lane rotation, or (128 columns) read from memory
+  auto next = [&](const R* p, size_t row, double v) {
+    if constexpr (NX > 64)
+      return (double)p[row + ((i + 1) & (NX - 1))];
+    else
+      return (double)s.rot(v, 1);
+  };
+  // 1. right-hand side
+  for (int k0 = w0; k0 < nzm; k0 += RW * PB) {
+    double v[PB][16];
 #pragma unroll
-    for (int q = 0; q < UNR; q++) {
-      const int k = k0 + 4 * q;
-      if (!G::Y3 && k < nzm) {
-        const size_t o = ((size_t)c * nzm + k) * NX + i, ow = ((size_t)c * nz + k) * NX + i, own = ow + NX;
-        ld_[q][0] = d.u[o];
-        ld_[q][1] = ua[o];
-        ld_[q][2] = ub[o];
-        ld_[q][3] = uc[o];
-        ld_[q][4] = d.w[ow];
-        ld_[q][5] = wa[ow];
-        ld_[q][6] = wb[ow];
-        ld_[q][7] = wc[ow];
-        ld_[q][8] = d.w[own];
-        ld_[q][9] = wa[own];
-        ld_[q][10] = wb[own];
-        ld_[q][11] = wc[own];
+    for (int q = 0; q < PB; q++) {
+      const int k = ::min(k0 + RW * q, nzm - 1);
+      const size_t row = ((size_t)c * nzm + k) * NX, o = row + i, ow = ((size_t)c * nz + k) * NX + i, own = ow + NX;
+      v[q][0] = d.u[o];
+      v[q][1] = ua[o];
+      v[q][2] = ub[o];
+      v[q][3] = uc[o];
+      v[q][4] = d.w[ow];
+      v[q][5] = wa[ow];
+      v[q][6] = wb[ow];
+      v[q][7] = wc[ow];
+      v[q][8] = d.w[own];
+      v[q][9] = wa[own];
+      v[q][10] = wb[own];
+      v[q][11] = wc[own];
+      if constexpr (G::Y3) {
+        v[q][12] = d.v[o];
+        v[q][13] = d.dvdt[na][o];
+        v[q][14] = d.dvdt[nb][o];
+        v[q][15] = d.dvdt[nc][o];
+      } else if constexpr (NX > 64) {
+        v[q][12] = next(d.u, row, 0.0);
+        v[q][13] = next(ua, row, 0.0);
+        v[q][14] = next(ub, row, 0.0);
+        v[q][15] = next(uc, row, 0.0);
       }
     }
 #pragma unroll
-    for (int q = 0; q < UNR; q++) {
-    const int k = k0 + 4 * q;
-    double pv = 0.0;
-    if (k < nzm) {
-      size_t o = ((size_t)c * nzm + k) * NX + i;
-      size_t ow = ((size_t)c * nz + k) * NX + i;
-      size_t own = ow + NX;
+    for (int q = 0; q < PB; q++) {
+      const int k = k0 + RW * q;
+      if (k >= nzm) break;
       double rdz = 1. / (adz[k] * dz);
       double rup = rhow[k + 1] / rho[k] * rdz;
       double rdn = rhow[k] / rho[k] * rdz;
+      const double uu = v[q][0], uap = v[q][1], ubp = v[q][2], ucp = v[q][3];
+      double pv;
       if constexpr (G::Y3) {  // press_rhs.F90:45-69
-        double uu = d.u[o], uap = ua[o], ubp = ub[o], ucp = uc[o];
-        double vv = d.v[o], vap = d.dvdt[na][o], vbp = d.dvdt[nb][o], vcp = d.dvdt[nc][o];
-        pv = (rdx * (s.rot(uu, 1) - uu) + rdx * (s.roty(vv, 1) - vv) + (d.w[own] * rup - d.w[ow] * rdn)) * dta +
-             (rdx * (s.rot(uap, 1) - uap) + rdx * (s.roty(vap, 1) - vap) + (wa[own] * rup - wa[ow] * rdn)) +
-             btat * (rdx * (s.rot(ubp, 1) - ubp) + rdx * (s.roty(vbp, 1) - vbp) + (wb[own] * rup - wb[ow] * rdn)) +
-             ctat * (rdx * (s.rot(ucp, 1) - ucp) + rdx * (s.roty(vcp, 1) - vcp) + (wc[own] * rup - wc[ow] * rdn));
+        const double vv = v[q][12], vap = v[q][13], vbp = v[q][14], vcp = v[q][15];
+        pv = (rdx * (s.rot(uu, 1) - uu) + rdx * (s.roty(vv, 1) - vv) + (v[q][8] * rup - v[q][4] * rdn)) * dta +
+             (rdx * (s.rot(uap, 1) - uap) + rdx * (s.roty(vap, 1) - vap) + (v[q][9] * rup - v[q][5] * rdn)) +
+             btat * (rdx * (s.rot(ubp, 1) - ubp) + rdx * (s.roty(vbp, 1) - vbp) + (v[q][10] * rup - v[q][6] * rdn)) +
+             ctat * (rdx * (s.rot(ucp, 1) - ucp) + rdx * (s.roty(vcp, 1) - vcp) + (v[q][11] * rup - v[q][7] * rdn));
       } else {
-        const double uu = ld_[q][0], uap = ld_[q][1], ubp = ld_[q][2], ucp = ld_[q][3];
-        pv = (rdx * (s.rot(uu, 1) - uu) + (ld_[q][8] * rup - ld_[q][4] * rdn)) * dta +
-             (rdx * (s.rot(uap, 1) - uap) + (ld_[q][9] * rup - ld_[q][5] * rdn)) +
-             btat * (rdx * (s.rot(ubp, 1) - ubp) + (ld_[q][10] * rup - ld_[q][6] * rdn)) +
-             ctat * (rdx * (s.rot(ucp, 1) - ucp) + (ld_[q][11] * rup - ld_[q][7] * rdn));
+        double un, uan_, ubn, ucn;  // the next column's
+        if constexpr (NX > 64) {
+          un = v[q][12], uan_ = v[q][13], ubn = v[q][14], ucn = v[q][15];
+        } else {
+          un = s.rot(uu, 1), uan_ = s.rot(uap, 1), ubn = s.rot(ubp, 1), ucn = s.rot(ucp, 1);
+        }
+        pv = (rdx * (un - uu) + (v[q][8] * rup - v[q][4] * rdn)) * dta +
+             (rdx * (uan_ - uap) + (v[q][9] * rup - v[q][5] * rdn)) +
+             btat * (rdx * (ubn - ubp) + (v[q][10] * rup - v[q][6] * rdn)) +
+             ctat * (rdx * (ucn - ucp) + (v[q][11] * rup - v[q][7] * rdn));
       }
-      pv = pv * rho[k];
-    }
-    if (k < NK) P[k * PLD + i] = pv;
+      P[k * LD + col] = pv * rho[k];
     }
   }
-  // one 64x64x64 transform of the slab in place: P <- P * M (M row-major 64x64)
-  auto transform = [&](const double* M) {
-    double bf[16];
+  const int r16 = lane & 15, q4 = lane >> 4;
+  // the transform of every row by M [NX][NX] in place; wave w makes the 16 slots of column block
+  // w % (COLS / 16) for every (NW / blocks)-th tile of 16 rows.  8 columns: a block holds two
+  // instances, each the lower half of a 16-wide tile of its own.
+  auto transform = [&](const double* __restrict__ M) {
+    constexpr int NCB = COLS / 16, RG = NW / NCB, RT = 4 / RG;  // column blocks, row groups, row tiles of a wave
+    constexpr int SUB = NX == 8 ? 2 : 1, KS = NX / 4;
+    const int cb = wave % NCB, rg = wave / NCB;
+    const int kbase = NX >= 16 ? 16 * cb / NX * NX : 16 * cb;  // first slab column of the instance
+    double bf[KS];
 #pragma unroll
-    for (int j = 0; j < 16; j++) bf[j] = M[(4 * j + q4) * NX + 16 * wave + r16];
-    v4d acc[4];
+    for (int j = 0; j < KS; j++) {
+      if constexpr (NX == 8)
+        bf[j] = r16 < 8 ? M[(4 * j + q4) * NX + r16] : 0.0;
+      else
+        bf[j] = M[(4 * j + q4) * NX + ((16 * cb + r16) & (NX - 1))];
+    }
+    v4d acc[RT][SUB];
 #pragma unroll
-    for (int r = 0; r < 4; r++) acc[r] = v4d{0.0, 0.0, 0.0, 0.0};
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+      for (int u = 0; u < SUB; u++) acc[r][u] = v4d{0.0, 0.0, 0.0, 0.0};
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
+    for (int r = 0; r < RT; r++) {
+      const int t = rg + RG * r;
+      if (16 * t < nzm) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        double a = P[(16 * r + r16) * PLD + 4 * j + q4];
-        acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bf[j], acc[r], 0, 0, 0);
+        for (int u = 0; u < SUB; u++)
+#pragma unroll
+          for (int j = 0; j < KS; j++)
+            acc[r][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(P[(16 * t + r16) * LD + kbase + 8 * u + 4 * j + q4], bf[j],
+                                                             acc[r][u], 0, 0, 0);
       }
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 4; r++)
+    for (int r = 0; r < RT; r++) {
+      const int t = rg + RG * r;
+      if (16 * t < nzm) {
 #pragma unroll
-      for (int jj = 0; jj < 4; jj++) P[(16 * r + 4 * jj + q4) * PLD + 16 * wave + r16] = acc[r][jj];
+        for (int u = 0; u < SUB; u++)
+          if (NX >= 16 || r16 < 8) {
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) P[(16 * t + 4 * jj + q4) * LD + 16 * cb + 8 * u + r16] = acc[r][u][jj];
+          }
+      }
+    }
     __syncthreads();
   };
   // 2. forward transform
   transform(d.Ft);
-  // 3. Thomas sweep per slot (wave 0, lane = slot), factors in LDS
-  if (wave == 0) {
-    static_assert(NZM <= 64, "one level per lane");  // NZM == 0: the host admits nzm <= 64
+  // 3. Thomas sweep per slot
+  if (wave < WPR) {
     const double eig = d.eign[i];
-    // the level coefficients do not depend on the recurrence: lane k computes level k's,
-    // and the sweep broadcasts them (the sweep then waits on one division per level, not
-    // three plus the profile loads)
-    const int kl = i < nzm ? i : nzm - 1;
-    const double ac_l = rhow[kl] / (adz[kl] * adzw[kl] * dz * dz);
-    const double cc_l = rhow[kl + 1] / (adz[kl] * adzw[kl + 1] * dz * dz);
-    const double rho_l = rho[kl];
-    auto lane_of = [](double v, int k) {
-      const long long b = __double_as_longlong(v);
-      const int lo = __builtin_amdgcn_readlane((int)b, k), hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-      return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-    };
-    auto acoef = [&](int k) { return lane_of(ac_l, k); };
-    auto ccoef = [&](int k) { return lane_of(cc_l, k); };
+    const double *ca = CA + col / NX * nzm, *cc = CC + col / NX * nzm, *cr = CR + col / NX * nzm;
     double b;
     if (i == 0)
-      b = 1.0 / (eig * rho[0] - acoef(0) - ccoef(0));
+      b = 1.0 / (eig * cr[0] - ca[0] - cc[0]);
     else
-      b = 1.0 / (eig * rho[0] - ccoef(0));
-    // the factors: LDS, or (RALF) an array the unrolled sweeps index with constants, which
-    // the compiler keeps in registers
-    double alf_r[RALF ? (NZM > 0 ? NZM : 1) : 1];
-    auto put_alf = [&](int k, double v) {
-      if constexpr (RALF)
-        alf_r[k] = v;
-      else
-        ALF[k * 64 + i] = v;
-    };
-    auto get_alf = [&](int k) {
-      if constexpr (RALF)
-        return alf_r[k];
-      else
-        return ALF[k * 64 + i];
-    };
-    double alfa = -ccoef(0) * b;
-    put_alf(0, alfa);
-    double beta = P[i] * b;
-    P[i] = beta;
-    auto fwd = [&](int k) {
-      double ak = acoef(k), ck = ccoef(k);
-      double e = 1.0 / (eig * lane_of(rho_l, k) - ak - ck + ak * alfa);
+      b = 1.0 / (eig * cr[0] - cc[0]);
+    double alfa = -cc[0] * b;
+    ALF[col] = alfa;
+    double beta = P[col] * b;
+    P[col] = beta;
+    double ak_n = ca[1], ck_n = cc[1], rk_n = cr[1], pk_n = P[LD + col];
+    for (int k = 1; k < nzm - 1; k++) {
+      const double ak = ak_n, ck = ck_n, rk = rk_n, pk = pk_n;
+      ak_n = ca[k + 1];
+      ck_n = cc[k + 1];
+      rk_n = cr[k + 1];
+      pk_n = P[(k + 1) * LD + col];
+      double e = 1.0 / (eig * rk - ak - ck + ak * alfa);
       alfa = -ck * e;
-      put_alf(k, alfa);
-      beta = (P[k * PLD + i] - ak * beta) * e;
-      P[k * PLD + i] = beta;
-    };
-    if constexpr (RALF) {
-      // the same operations as fwd, with the terms that do not depend on the recurrence (the
-      // coefficient broadcasts and the slab read) fetched one level ahead, so that they
-      // overlap the previous level's division instead of waiting behind it
-      double ak_n = acoef(1), ck_n = ccoef(1), rk_n = lane_of(rho_l, 1), pk_n = P[PLD + i];
-#pragma unroll
-      for (int k = 1; k < NZM - 1; k++) {
-        const double ak = ak_n, ck = ck_n, rk = rk_n, pk = pk_n;
-        if (k + 1 < NZM - 1) {
-          ak_n = acoef(k + 1);
-          ck_n = ccoef(k + 1);
-          rk_n = lane_of(rho_l, k + 1);
-          pk_n = P[(k + 1) * PLD + i];
-        }
-        double e = 1.0 / (eig * rk - ak - ck + ak * alfa);
-        alfa = -ck * e;
-        put_alf(k, alfa);
-        beta = (pk - ak * beta) * e;
-        P[k * PLD + i] = beta;
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-      for (int k = 1; k < nzm - 1; k++) fwd(k);
+      ALF[k * COLS + col] = alfa;
+      beta = (pk - ak * beta) * e;
+      P[k * LD + col] = beta;
     }
     {
-      int k = nzm - 1;
-      double ak = acoef(k);
-      double top = (P[k * PLD + i] - ak * beta) / (eig * rho[k] - ak + ak * alfa);
-      P[k * PLD + i] = top;
-      auto bwd = [&](int kk) {
-        top = get_alf(kk) * top + P[kk * PLD + i];
-        P[kk * PLD + i] = top;
-      };
-      if constexpr (RALF) {
-        // bwd with the slab read one level ahead
-        double pn = P[(NZM - 2) * PLD + i];
-#pragma unroll
-        for (int kk = NZM - 2; kk >= 0; kk--) {
-          const double pk = pn;
-          if (kk > 0) pn = P[(kk - 1) * PLD + i];
-          top = get_alf(kk) * top + pk;
-          P[kk * PLD + i] = top;
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      } else {
-        for (int kk = nzm - 2; kk >= 0; kk--) bwd(kk);
+      double top = (pk_n - ak_n * beta) / (eig * rk_n - ak_n + ak_n * alfa);
+      P[(nzm - 1) * LD + col] = top;
+      double an = ALF[(nzm - 2) * COLS + col], pn = P[(nzm - 2) * LD + col];
+      for (int kk = nzm - 2; kk >= 0; kk--) {
+        const double af = an, pk = pn;
+        const int kb = ::max(kk - 1, 0);
+        an = ALF[kb * COLS + col];
+        pn = P[kb * LD + col];
+        top = af * top + pk;
+        P[kk * LD + col] = top;
       }
     }
   }
@@ -1780,233 +1477,90 @@ k_press64(DevT<R> d, int na, int nb, int nc) {
   R* wan = d.dwdt[na];
   R* unc = d.dudt[nc];
   R* wnc = d.dwdt[nc];
-  for (int k0 = wave; k0 < nzm; k0 += 4 * UNR) {
-    double lg_[UNR][8];
-#pragma unroll
-    for (int q = 0; q < UNR; q++) {
-      const int k = k0 + 4 * q;
-      if (k < nzm) {
-        const size_t o = ((size_t)c * nzm + k) * NX + i, ow = ((size_t)c * nz + k) * NX + i;
-        lg_[q][0] = ua[o];
-        lg_[q][1] = wa[ow];
-        lg_[q][2] = d.u[o];
-        lg_[q][3] = d.w[ow];
-        lg_[q][4] = ub[o];
-        lg_[q][5] = uc[o];
-        lg_[q][6] = wb[ow];
-        lg_[q][7] = wc[ow];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < UNR; q++) {
-    const int k = k0 + 4 * q;
-    if (k >= nzm) break;
-    size_t o = ((size_t)c * nzm + k) * NX + i;
-    size_t ow = ((size_t)c * nz + k) * NX + i;
-    double pk = P[k * PLD + i];
-    double pim = s.rot(pk, -1);
-    double pkb = P[(k > 0 ? k - 1 : 0) * PLD + i];
-    double rdz = 1. / (dz * adzw[k]);
-    double du_a = lg_[q][0] - (pk - pim) * rdx;
-    double dw_a = lg_[q][1] - (pk - pkb) * rdz;
-    double uu = lg_[q][2], ww = lg_[q][3];
-    // the b and c terms of the Adams-Bashforth step are summed first, as k_press64r keeps
-    // that sum in registers: both kernels give the same bits
-    double un = uu + dt3 * (d.at * du_a + (d.bt * lg_[q][4] + d.ct * lg_[q][5]));
-    double wn = ww + dt3 * (d.at * dw_a + (d.bt * lg_[q][6] + d.ct * lg_[q][7]));
-    if constexpr (G::Y3) {  // press_grad.F90:29, adams.F90:29,32
-      double pjm = s.roty(pk, -1);
-      double dv_a = d.dvdt[na][o] - (pk - pjm) * rdx;
-      double vv = d.v[o];
-      double vn = vv + dt3 * (d.at * dv_a + d.bt * d.dvdt[nb][o] + d.ct * d.dvdt[nc][o]);
-      d.dvdt[na][o] = dv_a;
-      d.dvdt[nc][o] = vn;
-      d.v[o] = 0.5 * (vv + vn) * (rho[k] * dtdx);
-    }
-    uan[o] = du_a;
-    wan[ow] = dw_a;
-    unc[o] = un;
-    wnc[ow] = wn;
-    d.u[o] = 0.5 * (uu + un) * (rho[k] * dtdx);
-    d.w[ow] = 0.5 * (ww + wn) * (rhow[k] * dtdz);
-    }
-  }
-  if (wave == 0) wnc[((size_t)c * nz + nzm) * NX + i] = 0.0;
-}
-
-// k_press64 for 2D CRMs of 64 columns on 8 waves (one instance per 512-thread workgroup):
-// wave w owns the slab rows k = w + 8 j.  The right-hand side pass keeps, per row, what the
-// gradient pass needs (u, w, their tendencies dudt(na), dwdt(na), and the b/c terms of the
-// Adams-Bashforth step) in registers, so the velocities and the Adams-Bashforth history are
-// read from memory once per launch instead of twice.  Eight waves of one workgroup fill a CU
-// as two four-wave workgroups of k_press64 do.
-template <int NZM, typename R>
-__global__ void __launch_bounds__(512) k_press64r(DevT<R> d, int na, int nb, int nc) {
-  CRM_STOP_CHECK(d);
-  constexpr int NX = 64, NK = 64, NW = 8;
-  constexpr int NJ = (NZM + NW - 1) / NW;  // rows of the level range per wave
-  extern __shared__ double lds[];
-  double* P = lds;              // [NK][PLD] slab: rhs, coefficients, pressure
-  double* ALF = lds + NK * PLD; // [NZM][64] Thomas factors
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = blockIdx.x;  // grid is exactly ncrms blocks
-  const int i = lane;
-  Seg<64> s;
-  const int nz = NZM + 1;
-  const double dz = inst(d, I_DZ, c);
-  const double* adz = prof(d, P_ADZ, c);
-  const double* adzw = prof(d, P_ADZW, c);
-  const double* rho = prof(d, P_RHO, c);
-  const double* rhow = prof(d, P_RHOW, c);
-  const double rdx = 1. / d.dx, btat = d.bt / d.at, ctat = d.ct / d.at;
-  const double dta = 1. / d.dt3na / d.at;
-  const R *ua = d.dudt[na], *ub = d.dudt[nb], *uc = d.dudt[nc];
-  const R *wa = d.dwdt[na], *wb = d.dwdt[nb], *wc = d.dwdt[nc];
-  const int r16 = lane & 15, q4 = lane >> 4;
-  // the gradient pass's inputs of each owned level
-  double cu[NJ], cua[NJ], cub[NJ], cw[NJ], cwa[NJ], cwb[NJ];
-  // 1. right-hand side (rows >= NZM of the slab are zero)
-#pragma unroll
-  for (int j = 0; j < NK / NW; j++) {
-    const int k = wave + NW * j;
-    double pv = 0.0;
-    if (k < NZM) {
-      size_t o = ((size_t)c * NZM + k) * NX + i;
-      size_t ow = ((size_t)c * nz + k) * NX + i;
-      size_t own = ow + NX;
-      double rdz = 1. / (adz[k] * dz);
-      double rup = rhow[k + 1] / rho[k] * rdz;
-      double rdn = rhow[k] / rho[k] * rdz;
-      double uu = d.u[o], uap = ua[o], ubp = ub[o], ucp = uc[o];
-      double ww = d.w[ow], wap = wa[ow], wbp = wb[ow], wcp = wc[ow];
-      pv = (rdx * (s.rot(uu, 1) - uu) + (d.w[own] * rup - ww * rdn)) * dta +
-           (rdx * (s.rot(uap, 1) - uap) + (wa[own] * rup - wap * rdn)) +
-           btat * (rdx * (s.rot(ubp, 1) - ubp) + (wb[own] * rup - wbp * rdn)) +
-           ctat * (rdx * (s.rot(ucp, 1) - ucp) + (wc[own] * rup - wcp * rdn));
-      pv = pv * rho[k];
-      if (j < NJ) {
-        cu[j] = uu;
-        cua[j] = uap;
-        cub[j] = d.bt * ubp + d.ct * ucp;
-        cw[j] = ww;
-        cwa[j] = wap;
-        cwb[j] = d.bt * wbp + d.ct * wcp;
-      }
-    }
-    P[k * PLD + i] = pv;
-  }
-  // one 64x64x64 transform of the slab in place: P <- P * M (M row-major 64x64); wave w makes
-  // output columns 16 (w & 3) .. +15 of row tiles 2 (w >> 2) and 2 (w >> 2) + 1
-  auto transform = [&](const double* M) {
-    const int cb = wave & 3, rb = (wave >> 2) * 2;
-    double bf[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) bf[j] = M[(4 * j + q4) * NX + 16 * cb + r16];
-    v4d acc[2];
-#pragma unroll
-    for (int r = 0; r < 2; r++) acc[r] = v4d{0.0, 0.0, 0.0, 0.0};
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-#pragma unroll
-      for (int r = 0; r < 2; r++) {
-        double a = P[(16 * (rb + r) + r16) * PLD + 4 * j + q4];
-        acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bf[j], acc[r], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-      for (int jj = 0; jj < 4; jj++) P[(16 * (rb + r) + 4 * jj + q4) * PLD + 16 * cb + r16] = acc[r][jj];
-    __syncthreads();
-  };
-  // 2. forward transform
-  transform(d.Ft);
-  // 3. Thomas sweep per slot (wave 0, lane = slot), factors in LDS; as in k_press64
-  if (wave == 0) {
-    static_assert(NZM <= 64, "one level per lane");
-    const double eig = d.eign[i];
-    const int kl = i < NZM ? i : NZM - 1;
-    const double ac_l = rhow[kl] / (adz[kl] * adzw[kl] * dz * dz);
-    const double cc_l = rhow[kl + 1] / (adz[kl] * adzw[kl + 1] * dz * dz);
-    const double rho_l = rho[kl];
-    auto lane_of = [](double v, int k) {
-      const long long b = __double_as_longlong(v);
-      const int lo = __builtin_amdgcn_readlane((int)b, k), hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-      return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-    };
-    auto acoef = [&](int k) { return lane_of(ac_l, k); };
-    auto ccoef = [&](int k) { return lane_of(cc_l, k); };
-    double b;
-    if (i == 0)
-      b = 1.0 / (eig * rho[0] - acoef(0) - ccoef(0));
+  // the weighted tendencies of the three time levels; which of the first two products is rounded
+  // by itself is spelled out where the compiler's choice hangs on the arrangement of the loop
+  auto ab3 = [&](double a, double b, double c_) {
+    if constexpr (std::is_same<R, double>::value && (NX == 128 || (NX == 16 && G::Y3)))
+      return fma(d.ct, c_, fma(d.at, a, d.bt * b));
+    else if constexpr (std::is_same<R, double>::value && NX == 64)
+      return fma(d.ct, c_, fma(d.bt, b, d.at * a));
     else
-      b = 1.0 / (eig * rho[0] - ccoef(0));
-    double alfa = -ccoef(0) * b;
-    ALF[i] = alfa;
-    double beta = P[i] * b;
-    P[i] = beta;
-    for (int k = 1; k < NZM - 1; k++) {
-      double ak = acoef(k), ck = ccoef(k);
-      double e = 1.0 / (eig * lane_of(rho_l, k) - ak - ck + ak * alfa);
-      alfa = -ck * e;
-      ALF[k * 64 + i] = alfa;
-      beta = (P[k * PLD + i] - ak * beta) * e;
-      P[k * PLD + i] = beta;
+      return d.at * a + d.bt * b + d.ct * c_;
+  };
+  auto bc = [&](double b, double c_) {
+    if constexpr (std::is_same<R, double>::value && G::Y3)
+      return fma(d.bt, b, d.ct * c_);
+    else
+      return d.bt * b + d.ct * c_;
+  };
+  for (int k0 = w0; k0 < nzm; k0 += RW * PB) {
+    double v[PB][12];
+#pragma unroll
+    for (int q = 0; q < PB; q++) {
+      const int k = ::min(k0 + RW * q, nzm - 1);
+      const size_t o = ((size_t)c * nzm + k) * NX + i, ow = ((size_t)c * nz + k) * NX + i;
+      v[q][0] = ua[o];
+      v[q][1] = wa[ow];
+      v[q][2] = d.u[o];
+      v[q][3] = d.w[ow];
+      v[q][4] = ub[o];
+      v[q][5] = uc[o];
+      v[q][6] = wb[ow];
+      v[q][7] = wc[ow];
+      if constexpr (G::Y3) {
+        v[q][8] = d.dvdt[na][o];
+        v[q][9] = d.v[o];
+        v[q][10] = d.dvdt[nb][o];
+        v[q][11] = d.dvdt[nc][o];
+      }
     }
-    {
-      int k = NZM - 1;
-      double ak = acoef(k);
-      double top = (P[k * PLD + i] - ak * beta) / (eig * rho[k] - ak + ak * alfa);
-      P[k * PLD + i] = top;
-      for (int kk = NZM - 2; kk >= 0; kk--) {
-        top = ALF[kk * 64 + i] * top + P[kk * PLD + i];
-        P[kk * PLD + i] = top;
+#pragma unroll
+    for (int q = 0; q < PB; q++) {
+      const int k = k0 + RW * q;
+      if (k >= nzm) break;
+      const size_t o = ((size_t)c * nzm + k) * NX + i, ow = ((size_t)c * nz + k) * NX + i;
+      double pk = P[k * LD + col];
+      double pim;
+      if constexpr (NX > 64)
+        pim = P[k * LD + ((i - 1) & (NX - 1))];
+      else
+        pim = s.rot(pk, -1);
+      double pkb = P[(k > 0 ? k - 1 : 0) * LD + col];
+      double rdz = 1. / (dz * adzw[k]);
+      double du_a = v[q][0] - (pk - pim) * rdx;
+      double dw_a = v[q][1] - (pk - pkb) * rdz;
+      double uu = v[q][2], ww = v[q][3];
+      double un, wn;
+      if constexpr (NX == 64) {  // the b and c terms first
+        un = uu + dt3 * (d.at * du_a + bc(v[q][4], v[q][5]));
+        wn = ww + dt3 * (d.at * dw_a + bc(v[q][6], v[q][7]));
+      } else {
+        un = uu + dt3 * ab3(du_a, v[q][4], v[q][5]);
+        wn = ww + dt3 * ab3(dw_a, v[q][6], v[q][7]);
+      }
+      double dv_a = 0.0, vn = 0.0, vv = 0.0;
+      if constexpr (G::Y3) {  // press_grad.F90:29, adams.F90:29,32
+        double pjm = s.roty(pk, -1);
+        dv_a = v[q][8] - (pk - pjm) * rdx;
+        vv = v[q][9];
+        vn = vv + dt3 * ab3(dv_a, v[q][10], v[q][11]);
+      }
+      if (live) {
+        uan[o] = du_a;
+        wan[ow] = dw_a;
+        unc[o] = un;
+        wnc[ow] = wn;
+        d.u[o] = 0.5 * (uu + un) * (rho[k] * dtdx);
+        d.w[ow] = 0.5 * (ww + wn) * (rhow[k] * dtdz);
+        if constexpr (G::Y3) {
+          d.dvdt[na][o] = dv_a;
+          d.dvdt[nc][o] = vn;
+          d.v[o] = 0.5 * (vv + vn) * (rho[k] * dtdx);
+        }
       }
     }
   }
-  // 4. inverse transform (its leading barrier also ends the Thomas sweep)
-  transform(d.Gt);
-  // 5. pressure gradient, then Adams-Bashforth and the half-step Courant velocities, from the
-  // registers of pass 1
-  const double dtdx = d.dtn / d.dx, dtdz = d.dtn / dz, dt3 = d.dt3na;
-  R* uan = d.dudt[na];
-  R* wan = d.dwdt[na];
-  R* unc = d.dudt[nc];
-  R* wnc = d.dwdt[nc];
-#pragma unroll
-  for (int j = 0; j < NJ; j++) {
-    const int k = wave + NW * j;
-    if (k < NZM) {
-      size_t o = ((size_t)c * NZM + k) * NX + i;
-      size_t ow = ((size_t)c * nz + k) * NX + i;
-      double pk = P[k * PLD + i];
-      double pim = s.rot(pk, -1);
-      double pkb = P[(k > 0 ? k - 1 : 0) * PLD + i];
-      double rdz = 1. / (dz * adzw[k]);
-      double du_a = cua[j] - (pk - pim) * rdx;
-      double dw_a = cwa[j] - (pk - pkb) * rdz;
-      double uu = cu[j], ww = cw[j];
-      double un = uu + dt3 * (d.at * du_a + cub[j]);
-      double wn = ww + dt3 * (d.at * dw_a + cwb[j]);
-      uan[o] = du_a;
-      wan[ow] = dw_a;
-      unc[o] = un;
-      wnc[ow] = wn;
-      d.u[o] = 0.5 * (uu + un) * (rho[k] * dtdx);
-      d.w[ow] = 0.5 * (ww + wn) * (rhow[k] * dtdz);
-    }
-  }
-  if (wave == 0) wnc[((size_t)c * nz + NZM) * NX + i] = 0.0;
-}
-
-template <int NZM>
-constexpr size_t press64_lds_bytes() {  // NZM == 0: room for the most levels, 64
-  return (size_t)(64 * PLD + (NZM > 0 ? NZM : 64) * 64) * sizeof(double);
-}
-constexpr size_t press64_slab_bytes() {  // the slab alone (Thomas factors in registers)
-  return (size_t)64 * PLD * sizeof(double);
+  if (w0 == 0 && live) wnc[((size_t)c * nz + nzm) * NX + i] = 0.0;
 }
 
 // ------------------------------------------------------------------------------------------

@@ -227,13 +227,9 @@ int crm_hip_set_schedule(crm_hip_ctx *ctx, const int block[CRM_HIP_NKERNEL]);
 int crm_hip_get_schedule(const crm_hip_ctx *ctx, int block[CRM_HIP_NKERNEL]);
 
 /* Launch variant ("tile shape") of each kernel class of a context, 0 the default; results are
- * bitwise the same in every variant. CRM_K_PRESS of 2D 64-column CRMs: 0 chosen by the batch's
- * size (4 beyond 512 instances at 28 and 58 levels, else one instance per 4-wave workgroup with the
- * Thomas factors in LDS, two workgroups per CU), 1 one instance on 8 waves with the gradient pass's
- * inputs kept in registers from the right-hand side pass (one workgroup per CU), 2 and 3 the 4-wave
- * workgroup with two or four levels of each pass unrolled together, 4 the 4-wave workgroup with
- * the Thomas factors in registers (the workgroup's LDS is the slab alone: three workgroups per
- * CU). CRM_K_MPDATA (each scalar on its own waves): 0 chosen by the batch's size (small batches deal
+ * bitwise the same in every variant. CRM_K_PRESS of 2D 64-column CRMs: an
+ * instance on a workgroup of 8 waves (0, 1), 4 (2, 3) or 16 (4), with four (0, 2) or two (1, 3, 4)
+ * levels of each wave loaded together. CRM_K_MPDATA (each scalar on its own waves): 0 chosen by the batch's size (small batches deal
  * the levels to several workgroups; large ones take 2 at 64 columns in 2D, else 4), 1 the other
  * number of levels per trip of the sweep's steady state than the default (two for 2D 64-column
  * CRMs, else one), 2 and 3 the default and 1 with the registers bounded for three waves per SIMD,

@@ -7,8 +7,10 @@ count that leaves a wave partly empty."""
 import numpy as np
 import pytest
 
+import oracle_lib
 from crm_hip import CrmHip, DeviceCase
 from crm_inputs import add_convection, make_case
+from parity import convective_case, relerr
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +71,30 @@ def test_sedimentation_substeps_of_a_chunked_column():
     for group in ("state", "rad", "out"):
         for k, v in getattr(res[0], group).items():
             assert np.array_equal(v, getattr(res[1], group)[k][:2]), (group, k)
+
+
+# The pressure solve's tiles of 16 levels (one level over and under a tile, the fewest, the most), its
+# lane and column geometries, and instance counts that leave a workgroup partly empty.
+@pytest.mark.parametrize("nx,nz,n", [(8, 8, 9), (8, 17, 7), (16, 16, 5), (16, 31, 3), (32, 33, 3), (32, 49, 1),
+                                     (64, 8, 2), (64, 15, 1), (64, 48, 3), (64, 64, 2), (128, 9, 1), (128, 64, 2)])
+def test_pressure_solve_at_tile_edges(nx, nz, n):
+    """The first substep up to and with the pressure solve against the C restatement, within the
+    parity bar of one substep (1e-10 of each field's largest value): the transform's sums of up to
+    128 products and the sweep of up to 64 levels round at 1e-16 each.  Every variant gives the
+    same bits."""
+    dt = 20.0 * 28 / max(nz, 28)
+    case = convective_case(n, nx=nx, nz=nz, dx=2000.0, dt=dt, seed=nx + nz)
+    o = oracle_lib.oracle()
+    assert o.run(case.copy(), dt, 13) == 0
+    size = n * (nz + 1) * nx
+    fields = ("u", "w", "dudt_na", "dwdt_na", "dudt_nc", "dwdt_nc")
+    got = {}
+    for variant in range(5 if nx == 64 else 1):
+        with CrmHip(0) as hip:
+            hip.set_variants({"press": variant})
+            assert hip.debug_run(case.copy(), dt, 13) == 0
+            got[variant] = {f: hip.debug_get(f, size).copy() for f in fields}
+        for f in fields:
+            assert np.array_equal(got[variant][f], got[0][f]), (variant, f)
+    for f in fields:
+        assert relerr(got[0][f], o.field(f, size)) <= 1e-10, f
