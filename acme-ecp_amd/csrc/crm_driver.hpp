@@ -902,10 +902,12 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
   int nstep = 0;
   d.stop = nullptr;
   // Whole-call graph: the call's substeps captured once with one subcycle each and replayed;
-  // k_decide stops the replay at the first substep that needs more subcycles (every later
+  // decide() stops the replay at the first substep that needs more subcycles (every later
   // kernel returns at entry), and the loop below resumes that substep from the host's record
-  // of its bookkeeping before it (slot rotation, buffer swaps, Adams-Bashforth history).
-  if (ctx->use_graphs >= CRM_GRAPHS_CALL && !sc && !acc && !net_inputs && ctx->prof_mask == 0 && phase_stop == 0 &&
+  // of its bookkeeping before it (slot rotation, buffer swaps, Adams-Bashforth history).  A call
+  // with mean-state acceleration queues the same sequence launch by launch: the host's read of
+  // the maximum and the flag every substep left the device idle for 45 us of 600 (500 x 64 x 58).
+  if (ctx->use_graphs >= CRM_GRAPHS_CALL && !sc && !net_inputs && ctx->prof_mask == 0 && phase_stop == 0 &&
       nstop <= 2048) {
     struct Snap {
       int na, nb, nc;
@@ -938,21 +940,16 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
         d.dt3na = dt3[na];
         if (launch) {
           // the kurant maximum of substep n: from k_kurant at the first substep, after it from
-          // the previous substep's k_micro (the same state, the same maximum); the slots are
-          // cleared once k_decide has read them, for this substep's k_micro (the last
-          // substep's maximum is not read)
-          if (n == 1) {
-            k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_FLAGS, d.stop);
-            NX_DISPATCH(nx, (k_kurant<NXV, R><<<L.g(CRM_K_KURANT), L.b(CRM_K_KURANT), 0, s>>>(d)));
-          }
-          k_decide<<<1, 64, 0, s>>>(gmax, n, ctx->debug_stop);
-          k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_FLAGS, d.stop);
-          k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d);
+          // the previous substep's k_micro (the same state, the same maximum; with acceleration,
+          // which then still changes the winds, from k_kurant again); the decision clears the
+          // slots for the next (the last substep's maximum is not read)
+          if (n == 1) k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_FLAGS, d.stop);
+          if (n == 1 || acc) NX_DISPATCH(nx, (k_kurant<NXV, R><<<L.g(CRM_K_KURANT), L.b(CRM_K_KURANT), 0, s>>>(d)));
+          k_precip_init<R, true><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128) + 1), dim3(128), 0, s>>>(d, ctx->debug_stop);
           NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad)));
           NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
           NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
           NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
-          k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
           NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA])));
           NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp)));
         }
@@ -961,7 +958,12 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
         if (y3) std::swap(d.v, d.dvdt[nc]);
         if (launch) {
           NX_DISPATCH(nx, (launch_diffuse<NXV, R, GEO>(L, d, after_precip())));
-          NX_DISPATCH(nx, (k_micro<NXV, R, true><<<L.g(CRM_K_MICRO), L.b(CRM_K_MICRO), 0, s>>>(d, 0)));
+          if (acc) {
+            NX_DISPATCH(nx, (k_micro<NXV, R><<<L.g(CRM_K_MICRO), L.b(CRM_K_MICRO), 0, s>>>(d, 1)));
+            NX_DISPATCH(nx, (k_accel<NXV, R><<<L.g(CRM_K_MICRO), L.b(CRM_K_MICRO), 0, s>>>(d, acc_f, ctx->acc_uv)));
+          } else {
+            NX_DISPATCH(nx, (k_micro<NXV, R, true><<<L.g(CRM_K_MICRO), L.b(CRM_K_MICRO), 0, s>>>(d, 0)));
+          }
         }
         int nn = na;
         na = nc;
@@ -973,7 +975,12 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       }
     };
     HIPCHECK(hipMemsetAsync(gmax + GMAX_STOP, 0, sizeof(unsigned long long), s));
-    if (jc) {  // one graph with the other classes of crm_hip_run_many
+    if (acc) {
+      rc = arrival.alone();
+      if (rc) return rc;
+      sequence(true);
+      HIPCHECK(hipGetLastError());
+    } else if (jc) {  // one graph with the other classes of crm_hip_run_many
       HIPCHECK(hipEventRecord(ctx->ev_ready, s));
       arrival.done = true;
       rc = jc->arrive(slot, true, s, ctx->ev_ready, key, [&](bool launch) { sequence(launch); });
@@ -994,7 +1001,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       }
       HIPCHECK(hipGraphLaunch(exec, s));
     }
-    ctx->graph_launches += nstop;
+    if (!acc) ctx->graph_launches += nstop;
     unsigned long long stopped_at = 0;
     HIPCHECK(hipMemcpyAsync(&stopped_at, gmax + GMAX_STOP, sizeof(stopped_at), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
@@ -1008,7 +1015,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       d = sn.d;
       for (int j = 0; j < 3; j++) dt3[j] = sn.dt3[j];
       nstep = (int)stopped_at - 1;
-      ctx->graph_launches -= nstop - nstep;
+      if (!acc) ctx->graph_launches -= nstop - nstep;
     }
     if (nstep >= 1) ctx->stats.ncycle_max = std::max(ctx->stats.ncycle_max, 1);
     d.stop = nullptr;
@@ -1058,12 +1065,11 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       d.dt3na = dt3[na];
       const double* qrad = qrad_buf;
       auto body = [&]() {
-        k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d);
+        k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d, 0);
         NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad)));
         NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
         NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
         NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
-        k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
         NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA])));
         NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp)));
         std::swap(d.u, d.dudt[nc]);
@@ -1121,7 +1127,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       d.dt3na = dt3[na];
       if (icyc == 1)
         TIMED(CRM_K_PRECIP_INIT,
-              (k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d)));
+              (k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d, 0)));
       const double* qrad = qrad_buf;
       TIMED(CRM_K_PRE, NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad))));
       if (last && phase_stop == 7) goto stopped;
@@ -1131,7 +1137,6 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       if (last && phase_stop == 11) goto stopped;
       TIMED(CRM_K_PRESS, NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS]))));
       if (last && phase_stop == 13) goto stopped;
-      k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_PCFL, d.stop);
       TIMED(CRM_K_MPDATA, NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA]))));
       TIMED(CRM_K_PRECIP, NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp))));
       if (last && phase_stop == 15) goto stopped;

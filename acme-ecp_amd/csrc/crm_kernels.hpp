@@ -20,7 +20,7 @@ namespace CRM_NS {
 #endif
 #define CRM_LB __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CRM_WAVES_PER_EU)))
 
-// A captured call runs every substep with one subcycle; k_decide sets gmax[GMAX_STOP] to the
+// A call queued whole runs every substep with one subcycle; decide() sets gmax[GMAX_STOP] to the
 // first substep that needs more, and every kernel of the call then returns at entry (the flag
 // is the same for every thread, so no workgroup barrier is split); the host resumes that
 // substep eagerly.  d.stop is null outside such a call.
@@ -53,16 +53,25 @@ __global__ void k_zero_u64(unsigned long long* __restrict__ p, size_t n) {
     p[j] = 0ull;
 }
 
-// The subcycle decision of kurant.F90:53-75 on the device, for a captured call: one subcycle
-// when cfl / 0.7 <= 1; anything else (more subcycles, the reference's abort, a non-finite
-// value) stops the captured call at this substep for the host to take over; so does
-// nstep == stop_at (a test hook, 0 when off).
-__global__ void k_decide(unsigned long long* gmax, int nstep, int stop_at) {
-  if (threadIdx.x != 0 || gmax[GMAX_STOP]) return;
-  unsigned long long cbits = 0;
-  for (int j = 0; j < KURANT_SLOTS; j++) cbits = ::max(cbits, gmax[GMAX_FLAGS + j * KURANT_STRIDE]);
+// The subcycle decision of kurant.F90:53-75 on the device, for a call queued whole, by one wave
+// of substep nstep's first kernel: one subcycle when cfl / 0.7 <= 1; anything else (more
+// subcycles, the reference's abort, a non-finite value) stops the queued call at this substep for
+// the host to take over; so does the acceleration's 5 K flag (gmax[3]), and nstep == stop_at (a
+// test hook, 0 when off).  The maximum's slots are cleared for the next one gathered.
+__device__ __forceinline__ void decide(unsigned long long* gmax, int nstep, int stop_at) {
+  const int l = threadIdx.x & 63;
+  unsigned long long* slot = gmax + GMAX_FLAGS + (l & (KURANT_SLOTS - 1)) * KURANT_STRIDE;
+  unsigned long long cbits = *slot;
+  for (int m = KURANT_SLOTS / 2; m; m >>= 1) {
+    const unsigned long long o = __shfl_xor(cbits, m);
+    cbits = o > cbits ? o : cbits;
+  }
   const double q = __longlong_as_double((long long)cbits) / (double)0.7f;
-  if (!(q <= 1.0) || nstep == stop_at) gmax[GMAX_STOP] = (unsigned long long)nstep;
+  if (!(q <= 1.0) || nstep == stop_at || gmax[3]) {
+    if (l == 0) gmax[GMAX_STOP] = (unsigned long long)nstep;
+  } else if (l < KURANT_SLOTS) {
+    *slot = 0ull;
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -472,6 +481,10 @@ __global__ void CRM_LB k_kurant(DevT<R> d) {
 template <int NX, typename R, bool CHUNKS>
 __global__ void CRM_LB k_pre(DevT<R> d, int na, const double* qrad) {
   CRM_STOP_CHECK(d);
+  // the precipitation Courant maximum's slots, read by the last k_precip, for this subcycle's
+  // k_mpdata (a launch of their own cost 5 us per subcycle)
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < KURANT_SLOTS)
+    d.gmax[GMAX_PCFL + threadIdx.x * KURANT_STRIDE] = 0ull;
   SegFor<NX> s;
   int c;
   bool live = seg_instance<NX>(d.ncrms, c);
@@ -2300,10 +2313,20 @@ __global__ void CRM_LB k_diffuse(DevT<R> d, Scalars<R> src) {
 
 // ------------------------------------------------------------------------------------------
 // Bulk microphysics coefficients per level: precip_init.F90:47-91 (one thread per level).
+// DECIDE: the first kernel of a substep of a call queued whole, whose subcycle decision one more
+// wave makes (its own launch and the clearing of the slots cost 9 us per substep at 16 x 32 x 28).
+// The other workgroups need not wait for it: a stopped substep is run again from its start, and
+// these coefficients with it.
 // ------------------------------------------------------------------------------------------
-template <typename R>
-__global__ void k_precip_init(DevT<R> d) {
+template <typename R, bool DECIDE = false>
+__global__ void k_precip_init(DevT<R> d, int stop_at) {
   CRM_STOP_CHECK(d);
+  if constexpr (DECIDE) {
+    if (blockIdx.x == gridDim.x - 1) {
+      if (threadIdx.x < 64) decide(d.gmax, d.nstep, stop_at);
+      return;
+    }
+  }
   int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= d.ncrms * d.nzm) return;
   int c = idx / d.nzm, k = idx - c * d.nzm;
@@ -2802,6 +2825,7 @@ __global__ void CRM_LB k_micro(DevT<R> d, int accel) {
 // ------------------------------------------------------------------------------------------
 template <int NX, typename R>
 __global__ void CRM_LB k_accel(DevT<R> d, double factor, int uv) {
+  CRM_STOP_CHECK(d);
   SegFor<NX> s;
   int c;
   bool live = seg_instance<NX>(d.ncrms, c);
