@@ -2900,16 +2900,15 @@ struct WaterPaths {
       top_hit = 1.0;
       flag_top = false;
     }
-    if (pres >= 700.) {
-      cwpl += tmp1;
-      clt = fmax(1.0, clt);
-    } else if (pres < 400.) {
-      cwph += tmp1;
-      cht = fmax(1.0, cht);
-    } else {
-      cwpm += tmp1;
-      cmt = fmax(1.0, cmt);
-    }
+    // selects rather than stores under branches (a store to one of several members chosen at run
+    // time would put them all in memory)
+    const bool low = pres >= 700., high = !low && pres < 400., mid = !low && !high;
+    cwpl = low ? cwpl + tmp1 : cwpl;
+    clt = low ? fmax(1.0, clt) : clt;
+    cwph = high ? cwph + tmp1 : cwph;
+    cht = high ? fmax(1.0, cht) : cht;
+    cwpm = mid ? cwpm + tmp1 : cwpm;
+    cmt = mid ? fmax(1.0, cmt) : cmt;
     return top_hit;
   }
   template <typename R, typename S_>
@@ -2925,6 +2924,14 @@ struct WaterPaths {
   }
 };
 
+// What bounds k_stats: the arithmetic of levels with condensate or drafts, and memory in the others
+// (6 fields, w and the radiation sums).  Before -> now, us a launch: 4096 x 64 x 58 372 -> 302 and
+// mixed 278 -> 235, 500 x 64 x 58 69 -> 48, 256 x 128 x 58 83 -> 57, 333 x 8x8 x 40 mixed 37 -> 25,
+// 16 x 32 x 28 15 -> 9.5: of it half by the water paths in registers (they were in memory for a
+// store under a branch, WaterPaths::level), the rest by leaving out the reductions, the saturation
+// values and the additions of levels that have nothing to add.  168 registers (three waves per
+// SIMD) spill: 302 -> 421.
+//
 // COLS: one sweep over all levels does the water paths and the level statistics.  Otherwise the
 // levels are dealt to gridDim.y - 1 chunks, and the last workgroup of an instance takes the
 // water paths alone, from the two fields they need.
@@ -2952,28 +2959,40 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
   // the fields, profiles and radiation sums of one level; the sweep runs down from the top and
   // reads level k-1 while it works on level k.  Everything the level needs from memory is in
   // this read: vector loads complete in issue order, so a read issued after the prefetch (a
-  // profile, or the radiation sums the level adds to) would wait for it.  The sums are R: in
-  // the mixed engine FP32, which halves the bytes of this kernel's largest traffic (each
-  // addition rounds once, from the FP64 sum of the two terms)
+  // profile, or the radiation sums the level adds to) would wait for it.  The radiation sums are
+  // R: FP64 sums are added to in memory, without a read; those of the mixed engine are FP32 (half
+  // the bytes of this kernel's largest traffic; each addition rounds once, from the FP64 sum of
+  // the two terms) and are read with the level.
+  constexpr bool RAD_READ = !std::is_same<R, double>::value;
   struct Lvl {
-    double qcl, qci, qpl, qpi, tabs, qv, w, rho, rhow, adz, pres;
-    R ra[5];
+    R qcl, qci, qpl, qpi, tabs, qv, w;
+    double rho, rhow, adz, pres;
+    R ra0, ra1, ra2, ra3, ra4;
   };
   auto load = [&](int k, Lvl& L, bool sums = true) {
-    L.qcl = Q(d.qcl, k);
-    L.qci = Q(d.qci, k);
-    L.qpl = Q(d.qpl, k);
-    L.qpi = Q(d.qpi, k);
-    L.tabs = Q(d.tabs, k);
-    L.qv = Q(d.qv, k);
-    L.w = Wv(k);
+    const size_t o = ((size_t)c * nzm + k) * NX + i;
+    L.qcl = d.qcl[o];
+    L.qci = d.qci[o];
+    L.qpl = d.qpl[o];
+    L.qpi = d.qpi[o];
+    L.tabs = d.tabs[o];
+    L.qv = d.qv[o];
+    L.w = d.w[((size_t)c * nz + k) * NX + i];
     L.rho = rho[k];
     L.rhow = rhow[k];
     L.adz = adz[k];
     L.pres = pres[k];
-    for (int q = 0; q < 5; q++) L.ra[q] = R(0.0);
-    if (rad_owner && sums)
-      for (int q = 0; q < 5; q++) L.ra[q] = d.rad[q * rad_blk + rad_at(k)];
+    if constexpr (RAD_READ) {
+      L.ra0 = L.ra1 = L.ra2 = L.ra3 = L.ra4 = R(0.0);
+      if (rad_owner && sums) {
+        const R* r = d.rad + rad_at(k);
+        L.ra0 = r[0];
+        L.ra1 = r[rad_blk];
+        L.ra2 = r[2 * rad_blk];
+        L.ra3 = r[3 * rad_blk];
+        L.ra4 = r[4 * rad_blk];
+      }
+    }
   };
   WaterPaths wp;
   LevelChunk ch{0, nzm};
@@ -3016,19 +3035,25 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
   // mass flux through a w level with vertical velocity wj (crm_module.F90:1017-1049): the level
   // whose condensate decides is Xu (the level below, or the surface level) for an updraft and
   // the level above (Xa, or Xb, the top level, when a is false) for a downdraft; one saturation
-  // evaluation serves both branches
+  // evaluation serves both branches, and none is made where there is no condensate (the
+  // saturation value is not negative)
   // (the levels are passed as values, selected field by field: a reference chosen at run time
   // between two records would put them in memory)
   auto mass_flux = [&](double wj, double rhowj, const Lvl& Xu, const Lvl& Xa, const Lvl& Xb, bool a,
                        double& mui, double& mdi) {
     if (wj > 0. || wj < 0.) {
       const bool upd = wj > 0.;
+      auto both = [](R p, R q) { return (double)p + (double)q; };
       const double dt = a ? Xa.tabs : Xb.tabs, dp = a ? Xa.pres : Xb.pres;
-      const double dn = a ? Xa.qcl + Xa.qci : Xb.qcl + Xb.qci, dq = a ? Xa.qpl + Xa.qpi : Xb.qpl + Xb.qpi;
-      const double xt = upd ? Xu.tabs : dt, xp = upd ? Xu.pres : dp;
-      const double xn = upd ? Xu.qcl + Xu.qci : dn;
-      const double qs = qsatw(xt, xp);
-      const bool cloudy = xn > fmin(R4(1.e-5), 0.01 * qs);
+      const double dn = a ? both(Xa.qcl, Xa.qci) : both(Xb.qcl, Xb.qci);
+      const double dq = a ? both(Xa.qpl, Xa.qpi) : both(Xb.qpl, Xb.qpi);
+      const double xt = upd ? (double)Xu.tabs : dt, xp = upd ? Xu.pres : dp;
+      const double xn = upd ? both(Xu.qcl, Xu.qci) : dn;
+      bool cloudy = false;
+      if (xn > 0.) {
+        const double qs = qsatw(xt, xp);
+        cloudy = xn > fmin(R4(1.e-5), 0.01 * qs);
+      }
       // selects rather than stores under branches (a store to one of two locals chosen at run
       // time would put them in memory)
       const double f = rhowj * wj;
@@ -3040,8 +3065,7 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
     // at k = 0 level 0 again, unused (unconditional, as above); its radiation sums are read
     // before this level's are written, and never written from that read
     load(::max(k - 1, 0), nxt);
-    const size_t rad_base = rad_at(k);
-    const R* ra = cur.ra;
+    R* const ra = d.rad + rad_at(k);
     const double qcl = cur.qcl, qci = cur.qci, qpl = cur.qpl, qpi = cur.qpi, tabs = cur.tabs;
     const double wk = cur.w;
     double top_hit = 0.0;
@@ -3070,13 +3094,17 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
     double mui = 0, mdi = 0;
     if (k + 1 < nzm) mass_flux(w_up, up.rhow, cur, up2, up, k + 2 < nzm, mui, mdi);
     double sv[10] = {top_hit, cld, mcup, mcdn, mcuup, mcudn, qcl, qci, mui, mdi};
-    s.multi_sum(sv);
+    // most levels have no condensate and no strong draft: nothing to add (cloud tops and cloudy
+    // columns have condensate)
+    const bool some = s.any(qcl != 0. || qci != 0. || mcup != 0. || mcdn != 0. || mcuup != 0. || mcudn != 0. ||
+                            mui != 0. || mdi != 0.);
+    if (some) s.multi_sum(sv);
     // radiation-column sums (crm_module.F90:979-1015)
-    double rs[5] = {tabs, fmax(0.0, cur.qv), qcl, qci, (qcl + qci > 0) ? 1.0 : 0.0};
+    double rs[5] = {tabs, fmax(0.0, (double)cur.qv), qcl, qci, (qcl + qci > 0) ? 1.0 : 0.0};
     // the group's columns: contiguous lanes in 2D, a block of rows in 3D
     if (g > 1) s.gsums2(rs, d.rad_gx, d.rad_row, d.rad_gy);
     const double r_t = rs[0], r_qv = rs[1], r_qc = rs[2], r_qi = rs[3], r_cld = rs[4];
-    if (live) {
+    if (live && some) {
       // the reference's index mix for the cloud top (crm_module.F90:918-925)
       if (COLS && s.owns(0)) accum(&prof(d, P_CLDTOP, c)[nzm - 1 - k], sv[0]);
       if (s.owns(1)) accum(&prof(d, P_CLD, c)[k], sv[1]);
@@ -3088,13 +3116,19 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
       if (s.owns(7)) accum(&prof(d, P_GICE, c)[k], sv[7]);
       if (k + 1 < nzm && s.owns(8)) accum(&prof(d, P_MUI, c)[k + 1], sv[8]);
       if (k + 1 < nzm && s.owns(9)) accum(&prof(d, P_MDI, c)[k + 1], sv[9]);
-      if (rad_owner) {
-        d.rad[0 * rad_blk + rad_base] = (R)((double)ra[0] + r_t);
-        d.rad[1 * rad_blk + rad_base] = (R)((double)ra[1] + r_qv);
-        d.rad[2 * rad_blk + rad_base] = (R)((double)ra[2] + r_qc);
-        d.rad[3 * rad_blk + rad_base] = (R)((double)ra[3] + r_qi);
-        d.rad[4 * rad_blk + rad_base] = (R)((double)ra[4] + r_cld);
-      }
+    }
+    if (rad_owner) {
+      auto add = [&](int q, R old, double v) {
+        if constexpr (RAD_READ)
+          ra[q * rad_blk] = (R)((double)old + v);
+        else
+          accum(&ra[q * rad_blk], v);
+      };
+      add(0, cur.ra0, r_t);
+      add(1, cur.ra1, r_qv);
+      if (r_qc != 0.) add(2, cur.ra2, r_qc);
+      if (r_qi != 0.) add(3, cur.ra3, r_qi);
+      if (r_cld != 0.) add(4, cur.ra4, r_cld);
     }
     w_up = wk;
     up2 = up;
