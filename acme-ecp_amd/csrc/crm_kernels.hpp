@@ -1734,21 +1734,23 @@ __device__ __forceinline__ void mpdata_one(const DevT<R>& d, const G& s, int c, 
     }
     R tq_new = R(0.0);
     if (want_cfl && (ST || (K >= 3 && K - 3 < nzm))) tq_new = F(d.tabs, K - 3);
-    // stage 0: donor-cell fluxes at level K
-    if (ST || K < nzm) {
-      f_0 = cf;
-      U_0 = cu;
-      W_0 = cw;
+    // stage 0: donor-cell fluxes at level K, zero above the top (selects: with stores under a
+    // branch the compiler kept two of the rings in memory, at 128 columns and in 3D)
+    {
+      const bool in = ST || K < nzm;
+      f_0 = in ? cf : R(0.0);
+      U_0 = in ? cu : R(0.0);
+      W_0 = in ? cw : R(0.0);
       R fkb = (ST || K >= 1) ? f_1 : f_0;
-      uu1_0 = fmax(R(0.0), U_0) * s.rot(f_0, -1) + fmin(R(0.0), U_0) * f_0;
-      ww1_0 = fmax(R(0.0), W_0) * fkb + fmin(R(0.0), W_0) * f_0;
+      const R uu = fmax(R(0.0), U_0) * s.rot(f_0, -1) + fmin(R(0.0), U_0) * f_0;
+      const R ww = fmax(R(0.0), W_0) * fkb + fmin(R(0.0), W_0) * f_0;
+      uu1_0 = in ? uu : R(0.0);
+      ww1_0 = in ? ww : R(0.0);
       if constexpr (Y3) {
-        V_0 = cv;
-        vv1_0 = fmax(R(0.0), V_0) * s.roty(f_0, -1) + fmin(R(0.0), V_0) * f_0;
+        V_0 = in ? cv : R(0.0);
+        const R vv = fmax(R(0.0), V_0) * s.roty(f_0, -1) + fmin(R(0.0), V_0) * f_0;
+        vv1_0 = in ? vv : R(0.0);
       }
-    } else {
-      f_0 = U_0 = W_0 = uu1_0 = ww1_0 = R(0.0);
-      V_0 = vv1_0 = R(0.0);
     }
     // stage 1: donor-cell update and first bounds at level K-1
     const int L1 = K - 1;
