@@ -558,6 +558,7 @@ struct Launcher {
       case CRM_K_DIFFUSE: fill = 4096, least = 2; break;
       case CRM_K_MICRO: fill = std::max(8192, 4 * waves()), least = 1; break;
       case CRM_K_STATS: fill = 2048, least = 2; break;
+      case CRM_K_FINAL: fill = std::max(8192, 2 * waves()), least = 1; break;
       default: return 1;
     }
     if (!split && (kid == CRM_K_MPDATA || kid == CRM_K_PRECIP || kid == CRM_K_DIFFUSE)) return 1;
@@ -619,6 +620,14 @@ static void launch_stats(const Launcher& L, const DevT<R>& d) {
     g.y++;
     k_stats<NX, R, false><<<g, L.b(CRM_K_STATS), 0, L.s>>>(d);
   }
+}
+
+template <int NX, typename R>
+static void launch_final(const Launcher& L, const DevT<R>& d, const crm_input_view& in, const crm_state_view& st,
+                         const crm_rad_view& rad, const crm_output_view& out, double dt_gl, int nstop) {
+  dim3 g = L.g(CRM_K_FINAL);
+  g.y++;  // one more workgroup row for what belongs to the column
+  k_final<NX, R><<<g, L.b(CRM_K_FINAL), 0, L.s>>>(d, in, st, rad, out, dt_gl, nstop);
 }
 
 // NXV: columns per instance; GEO: the lane geometry (a 2D row of NXV columns, or the 8 x 8
@@ -811,7 +820,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
     }
     HIPCHECK(hipMemcpyAsync(lat_buf, col->lat, sizeof(double) * ncrms, hipMemcpyHostToDevice, s));
   }
-  TIMED(CRM_K_SETUP, (k_setup<R><<<L.grid_inst(64), dim3(64), 0, s>>>(d, *in, ctx->coriolis ? lat_buf : nullptr)));
+  TIMED(CRM_K_SETUP, (k_setup<R><<<dim3((unsigned)ncrms), dim3(64), 0, s>>>(d, *in, ctx->coriolis ? lat_buf : nullptr)));
   TIMED(CRM_K_INIT, NX_DISPATCH(nx, (k_init<NXV, R><<<L.g(CRM_K_INIT), L.b(CRM_K_INIT), 0, s>>>(d, *in, *st, *out, dt_gl))));
   if (col && col->igstep <= 1) {
     if (!sc) {
@@ -1167,7 +1176,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
   }
   ctx->stats.nstop = nstop;
   ctx->stats.accel_ceased = ceased ? 1 : 0;
-  TIMED(CRM_K_FINAL, NX_DISPATCH(nx, (k_final<NXV, R><<<L.g(CRM_K_FINAL), L.b(CRM_K_FINAL), 0, s>>>(d, *in, *st, *rad, *out, dt_gl, nstop))));
+  TIMED(CRM_K_FINAL, NX_DISPATCH(nx, (launch_final<NXV, R>(L, d, *in, *st, *rad, *out, dt_gl, nstop))));
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipEventRecord(ctx->ev1, s));
   HIPCHECK(hipMemcpyAsync(tail, gmax + GMAX_NPREC, sizeof(tail), hipMemcpyDeviceToHost, s));

@@ -77,7 +77,9 @@ __device__ __forceinline__ void decide(unsigned long long* gmax, int nstep, int 
 // ------------------------------------------------------------------------------------------
 // Reference profiles from crm_input: crm_module.F90:320-375; grid factors sgs.F90:219-228;
 // sponge profile damping.F90:44-61; roughness crm_module.F90:583-590 (z0_est
-// crmsurface.F90:104-131).  One thread per instance.
+// crmsurface.F90:104-131).  A workgroup of one wave per instance, a lane per level (level 64 and up
+// on the first lanes again): as one thread per instance every level waited for memory in turn
+// (16 x 28 levels 133 us, 500 x 58 453 us).
 // ------------------------------------------------------------------------------------------
 __device__ double z0_est(double z, double bflx, double wnd, double ustar, double c1) {
   const double vonk = R4(0.4), am = R4(4.8), bm = R4(19.3), eps = R4(1.e-10);
@@ -94,10 +96,9 @@ __device__ double z0_est(double z, double bflx, double wnd, double ustar, double
 }
 
 template <typename R>
-__global__ void k_setup(DevT<R> d, crm_input_view in, const double* lat) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= d.ncrms) return;
-  if (lat) {
+__global__ void __launch_bounds__(64) k_setup(DevT<R> d, crm_input_view in, const double* lat) {
+  const int c = blockIdx.x, lane = threadIdx.x;  // one instance, 64 threads
+  if (lat && lane == 0) {
     // crm_module.F90:287,321-322: latitude in degrees from radians (57.296_r8), then the
     // Coriolis parameters with the REAL(4) pi and literals of the reference build
     const double pi = (double)3.141592653589793f;
@@ -121,8 +122,9 @@ __global__ void k_setup(DevT<R> d, crm_input_view in, const double* lat) {
   double* gamaz = prof(d, P_GAMAZ, c);
   double* grdf = prof(d, P_GRDFX, c);
   double* tau = prof(d, P_TAU, c);
+  // the stages hand the profiles on through memory (the barriers order them within the wave)
   double zs = IN(in.zint, plev);
-  for (int k = 0; k < nzm; k++) {
+  for (int k = lane; k < nzm; k += 64) {
     z[k] = IN(in.zmid, plev - 1 - k) - zs;
     zi[k] = IN(in.zint, plev - k) - zs;
     pres[k] = IN(in.pmid, plev - 1 - k) / 100.;
@@ -130,30 +132,39 @@ __global__ void k_setup(DevT<R> d, crm_input_view in, const double* lat) {
     bet[k] = GGR_D / IN(in.tl, plev - 1 - k);
     gamaz[k] = GGR_D / CP_D * z[k];
   }
-  zi[nzm] = IN(in.zint, plev - nzm) - zs;
-  presi[nzm] = IN(in.pint, plev - nzm) / 100.;
+  if (lane == 0) {
+    zi[nzm] = IN(in.zint, plev - nzm) - zs;
+    presi[nzm] = IN(in.pint, plev - nzm) / 100.;
+  }
+  __syncthreads();
   double dz = 0.5 * (z[0] + z[1]);
-  inst(d, I_DZ, c) = dz;
-  for (int k = 1; k < nzm; k++) adzw[k] = (z[k] - z[k - 1]) / dz;
-  adzw[0] = 1.;
-  adzw[nzm] = adzw[nzm - 1];
-  for (int k = 0; k < nzm; k++) adz[k] = (zi[k + 1] - zi[k]) / dz;
-  for (int k = 0; k < nzm; k++) rho[k] = IN(in.pdel, plev - 1 - k) / GGR_D / (adz[k] * dz);
-  for (int k = 1; k < nzm; k++) rhow[k] = (IN(in.pmid, plev - k) - IN(in.pmid, plev - 1 - k)) / GGR_D / (adzw[k] * dz);
-  rhow[0] = 2. * rhow[1] - rhow[2];
-  rhow[nzm] = 2. * rhow[nzm - 1] - rhow[nzm - 2];
-  for (int k = 0; k < nzm; k++) {
+  if (lane == 0) inst(d, I_DZ, c) = dz;
+  for (int k = lane; k <= nzm; k += 64) {
+    const int kw = ::min(k, nzm - 1);  // level nzm as the one below
+    adzw[k] = k == 0 ? 1. : (z[kw] - z[kw - 1]) / dz;
+  }
+  for (int k = lane; k < nzm; k += 64) adz[k] = (zi[k + 1] - zi[k]) / dz;
+  __syncthreads();
+  for (int k = lane; k < nzm; k += 64) rho[k] = IN(in.pdel, plev - 1 - k) / GGR_D / (adz[k] * dz);
+  for (int k = lane; k < nzm; k += 64)
+    if (k > 0) rhow[k] = (IN(in.pmid, plev - k) - IN(in.pmid, plev - 1 - k)) / GGR_D / (adzw[k] * dz);
+  __syncthreads();
+  if (lane == 0) rhow[0] = 2. * rhow[1] - rhow[2];
+  if (lane == 0) rhow[nzm] = 2. * rhow[nzm - 1] - rhow[nzm - 2];
+  __syncthreads();
+  for (int k = lane; k < nzm; k += 64) {
     double a = adz[k] * dz;
     grdf[k] = fmin(16.0, d.dx * d.dx / (a * a));
   }
   // sponge: n_damp is the deepest level within 0.4 of the domain height from the top
   int n_damp = 0;
-  for (int k = nzm - 1; k >= 0; k--)
-    if (z[nzm - 1] - z[k] < R4(0.4) * z[nzm - 1]) n_damp = nzm - k;
-  inst(d, I_NDAMP, c) = (double)n_damp;
+  for (int k = lane; k < nzm; k += 64)
+    if (z[nzm - 1] - z[k] < R4(0.4) * z[nzm - 1]) n_damp = ::max(n_damp, nzm - k);
+  for (int m = 32; m; m >>= 1) n_damp = ::max(n_damp, __shfl_xor(n_damp, m));
+  if (lane == 0) inst(d, I_NDAMP, c) = (double)n_damp;
   int kbot = nzm - 1 - n_damp;  // 0-based level of the reference's z(nzm-n_damp)
   if (kbot < 0) kbot = 0;
-  for (int k = 0; k < nzm; k++) {
+  for (int k = lane; k < nzm; k += 64) {
     tau[k] = 0.0;
     if (k + 1 >= nzm - n_damp) {
       double tt = 60. * pow(450. / 60., (z[nzm - 1] - z[k]) / (z[nzm - 1] - z[kbot]));
@@ -168,7 +179,7 @@ __global__ void k_setup(DevT<R> d, crm_input_view in, const double* lat) {
   double* irhowadz = prof(d, P_IRHOWADZ, c);
   double* ddadz = prof(d, P_DDADZ, c);
   double* pratio = prof(d, P_PRATIO, c);
-  for (int k = 0; k < nzm; k++) {
+  for (int k = lane; k < nzm; k += 64) {
     irho[k] = 1. / rho[k];
     iadz[k] = 1. / adz[k];
     irhoadz[k] = 1. / (rho[k] * adz[k]);
@@ -187,17 +198,17 @@ __global__ void k_setup(DevT<R> d, crm_input_view in, const double* lat) {
     double* sbetdz = prof(d, P_SBETDZ, c);
     double* stkmax = prof(d, P_STKMAX, c);
     const double dx = d.dx, rdx0 = 1. / dx;
-    for (int k = 0; k < nzm; k++) {
+    for (int k = lane; k < nzm; k += 64) {
       srdz[k] = 1. / (dz * adz[k]);
       srdx[k] = rdx0 * sqrt(dx * srdz[k]);
     }
-    for (int k = 0; k <= nzm; k++) {
+    for (int k = lane; k <= nzm; k += 64) {
       srdzw[k] = 1. / (dz * adzw[k]);
       srdxw[k] = rdx0 * sqrt(dx * srdzw[k]);
     }
-    sbetdz[nzm - 1] = 0.0;
-    for (int k = 0; k + 1 < nzm; k++) sbetdz[k] = 0.5 * (bet[k + 1] + bet[k]) / dz / adzw[k + 1];
-    for (int k = 0; k < nzm; k++) {
+    if (lane == 0) sbetdz[nzm - 1] = 0.0;
+    for (int k = lane; k + 1 < nzm; k += 64) sbetdz[k] = 0.5 * (bet[k + 1] + bet[k]) / dz / adzw[k + 1];
+    for (int k = lane; k < nzm; k += 64) {
       const double cx = dx * dx / d.dt / grdf[k];
       const double dzm = dz * fmin(adzw[k], adzw[k + 1]);
       const double cz = dzm * dzm / d.dt / 1.0;
@@ -205,8 +216,9 @@ __global__ void k_setup(DevT<R> d, crm_input_view in, const double* lat) {
     }
     // vertical density weight of the scalar diffusion flux (diffuse_scalar2D.F90:93)
     double* drhoi = prof(d, P_DRHOI, c);
-    for (int k = 0; k < nzm; k++) drhoi[k] = rhow[k + 1] / adzw[k + 1];
+    for (int k = lane; k < nzm; k += 64) drhoi[k] = rhow[k + 1] / adzw[k + 1];
   }
+  if (lane != 0) return;
   double ustar = sqrt(in.tau00[c] / rho[0]);
   double z0 = z0_est(z[0], in.bflxls[c], in.wndls[c], ustar, d.z0c1);
   inst(d, I_Z0, c) = fmax(R4(0.00001), fmin(1.0, z0));
@@ -3152,7 +3164,11 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
 }
 
 // ------------------------------------------------------------------------------------------
-// End of call: crm_module.F90:1078-1659.  State write-back and every crm_output member.
+// End of call: crm_module.F90:1078-1659.  State write-back and every crm_output member.  The levels
+// are dealt to gridDim.y - 1 chunks; the last workgroup of an instance does what belongs to the
+// column, a lane per GCM level.  One lane writes a level's 45 means, which waits for memory
+// several times a level: with the levels one after the other 266 us at 16 x 32 x 28 and 800 us at
+// 500 x 64 x 58.  Large batches are bound by the write-back, whose columns lie an instance count apart.
 // ------------------------------------------------------------------------------------------
 template <int NX, typename R>
 __global__ void CRM_LB k_final(DevT<R> d, crm_input_view in, crm_state_view st, crm_rad_view rad, crm_output_view out,
@@ -3175,14 +3191,14 @@ __global__ void CRM_LB k_final(DevT<R> d, crm_input_view in, crm_state_view st, 
   auto Q = [&](const R* p, int k) -> double { return p[((size_t)c * nzm + k) * NX + i]; };
   auto Wv = [&](int k) { return d.w[((size_t)c * nz + k) * NX + i]; };
   const double a_gr = A_GR();
-  double colprec = 0, colprecs = 0;
-  for (int k = 0; k < nzm; k++) {
+  const int nch = (int)gridDim.y - 1, y = (int)blockIdx.y;
+  const LevelChunk ch = {(int)((unsigned)nzm * y / nch), (int)((unsigned)nzm * (y + 1) / nch)};
+  if (y < nch) {
+  for (int k = ch.k0; k < ch.k1; k++) {
     int l = plev - 1 - k;
     double tabs = Q(d.tabs, k), qv = Q(d.qv, k), qcl = Q(d.qcl, k), qci = Q(d.qci, k);
     double qpl = Q(d.qpl, k), qpi = Q(d.qpi, k), u = Q(d.u, k), wk = Wv(k), wk1 = Wv(k + 1);
     double pd = IN(in.pdel, l);
-    colprec += s.sum((qpl + qpi) * pd);
-    colprecs += s.sum(qpi * pd);
     double tln = s.sum(tabs) * factor_xy, qln = s.sum(qv) * factor_xy;
     double qccln = s.sum(qcl) * factor_xy, qiiln = s.sum(qci) * factor_xy;
     double omg = fmax(0.0, fmin(1.0, (tabs - TGRMIN) * a_gr));
@@ -3265,9 +3281,44 @@ __global__ void CRM_LB k_final(DevT<R> d, crm_input_view in, crm_state_view st, 
       }
     }
   }
-  // GCM levels above the CRM
-  if (live && i == 0) {
-    for (int l = 0; l < ptop0; l++) {
+  // time-averaged radiation groups
+  if (live) {
+    const int nxr = d.nx_rad;
+    const double f = ((double)nxr / (double)NX) * 1.0 / (double)nstop;
+    size_t blk = (size_t)d.ncrms * nzm * nxr;
+    double* outs[5] = {rad.temperature, rad.qv, rad.qc, rad.qi, rad.cld};
+    for (int idx = ch.k0 * nxr + i; idx < ch.k1 * nxr; idx += NX) {
+      int k = idx / nxr, ir = idx - k * nxr;
+      size_t src = (size_t)c * nzm * nxr + idx;
+      size_t dst = (size_t)c + (size_t)ld * ((size_t)ir + (size_t)nxr * k);
+      for (int q = 0; q < 5; q++) outs[q][dst] = (double)d.rad[q * blk + src] * f;
+    }
+  }
+  return;
+  }
+  // the column's precipitating water, level by level (NB levels are read together)
+  double colprec = 0, colprecs = 0;
+  constexpr int NB = 8;
+  for (int kt = 0; kt < nzm; kt += NB) {
+    double v[NB][3];
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+      const int k = ::min(kt + j, nzm - 1);
+      v[j][0] = Q(d.qpl, k);
+      v[j][1] = Q(d.qpi, k);
+      v[j][2] = IN(in.pdel, plev - 1 - k);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+      if (kt + j >= nzm) break;
+      colprec += s.sum((v[j][0] + v[j][1]) * v[j][2]);
+      colprecs += s.sum(v[j][1] * v[j][2]);
+    }
+  }
+  int jt = plev, mx = 1;
+  if (live) {
+    // GCM levels above the CRM
+    for (int l = i; l < ptop0; l += NX) {
       O2(out.sltend, l) = 0.0;
       O2(out.qltend, l) = 0.0;
       O2(out.qcltend, l) = 0.0;
@@ -3280,33 +3331,33 @@ __global__ void CRM_LB k_final(DevT<R> d, crm_input_view in, crm_state_view st, 
       for (double* p : zero2) O2(p, l) = 0.0;
     }
     // mass fluxes: interface l (0..plev) is w level plev-l
-    double jt = plev * 1.0, mx = 1.0;
     const cprof<double> mui = profcd(d, P_MUI, c);
     const cprof<double> mdi = profcd(d, P_MDI, c);
     auto MU = [&](int lw) { int kw = plev - lw; return (kw >= 0 && kw <= nzm - 1) ? mui[kw] : 0.0; };
     auto MD = [&](int lw) { int kw = plev - lw; return (kw >= 0 && kw <= nzm - 1) ? mdi[kw] : 0.0; };
-    for (int l = 0; l < plev; l++) {
+    for (int l = i; l < plev; l += NX) {
       double pd = IN(in.pdel, l);
       double mu_a = MU(l), mu_b = MU(l + 1), md_a = MD(l), md_b = MD(l + 1);
       double mu = 0.5 * (mu_a + mu_b) * GGR_D / 100.;
       double md = 0.5 * (md_a + md_b) * GGR_D / 100.;
       O2(out.mu_crm, l) = mu;
       O2(out.md_crm, l) = md;
-      O2(out.eu_crm, l) = 0.;
-      O2(out.du_crm, l) = 0.;
-      O2(out.ed_crm, l) = 0.;
-      if (mu_a - mu_b > 0)
-        O2(out.eu_crm, l) = (mu_a - mu_b) * GGR_D / pd;
-      else
-        O2(out.du_crm, l) = -1.0 * (mu_a - mu_b) * GGR_D / pd;
-      if (md_b - md_a < 0) O2(out.ed_crm, l) = (md_a - md_b) * GGR_D / pd;
+      const double deu = (mu_a - mu_b) * GGR_D / pd, ddu = -1.0 * (mu_a - mu_b) * GGR_D / pd;
+      const bool ent = mu_a - mu_b > 0;
+      O2(out.eu_crm, l) = ent ? deu : 0.;
+      O2(out.du_crm, l) = ent ? 0. : ddu;
+      O2(out.ed_crm, l) = md_b - md_a < 0 ? (md_a - md_b) * GGR_D / pd : 0.;
       if (fabs(mu) > R4(1.0e-15) || fabs(md) > R4(1.0e-15)) {
-        jt = fmin((double)(l + 1), jt);
-        mx = fmax((double)(l + 1), mx);
+        jt = ::min(l + 1, jt);
+        mx = ::max(l + 1, mx);
       }
     }
-    out.jt_crm[c] = jt;
-    out.mx_crm[c] = mx;
+  }
+  jt = s.imin(jt);
+  mx = s.imax(mx);
+  if (live && i == 0) {
+    out.jt_crm[c] = (double)jt;
+    out.mx_crm[c] = (double)mx;
     out.prectend[c] = (colprec - inst(d, I_COLPREC, c)) / GGR_D * factor_xy * icrm_run_time;
     out.precstend[c] = (colprecs - inst(d, I_COLPRECS, c)) / GGR_D * factor_xy * icrm_run_time;
     out.cltot[c] = inst(d, I_CLTOT, c) * factor_xyt;
@@ -3331,19 +3382,6 @@ __global__ void CRM_LB k_final(DevT<R> d, crm_input_view in, crm_state_view st, 
       out.precl[c] = precl * factor_xy / 1000.;
       out.precsc[c] = precsc * factor_xy / 1000.;
       out.precsl[c] = precsl * factor_xy / 1000.;
-    }
-  }
-  // time-averaged radiation groups
-  if (live) {
-    const int nxr = d.nx_rad;
-    const double f = ((double)nxr / (double)NX) * 1.0 / (double)nstop;
-    size_t blk = (size_t)d.ncrms * nzm * nxr;
-    double* outs[5] = {rad.temperature, rad.qv, rad.qc, rad.qi, rad.cld};
-    for (int idx = i; idx < nzm * nxr; idx += NX) {
-      int k = idx / nxr, ir = idx - k * nxr;
-      size_t src = (size_t)c * nzm * nxr + idx;
-      size_t dst = (size_t)c + (size_t)ld * ((size_t)ir + (size_t)nxr * k);
-      for (int q = 0; q < 5; q++) outs[q][dst] = (double)d.rad[q * blk + src] * f;
     }
   }
 }
