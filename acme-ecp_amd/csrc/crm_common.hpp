@@ -666,9 +666,18 @@ using SegFor = typename SegSel<NX>::type;
 // so its instance is wave-uniform; UNIFORM tells the compiler so, which turns the per-instance
 // profile loads into scalar loads.  A kernel whose scalar registers would then spill (k_stats
 // measured slower with it) passes false.
-template <int NX, bool UNIFORM = true>
+// NEAR: for kernels that read or write the caller's arrays, where the instances lie next to each
+// other: 16 instances (a cache line of FP64) go to workgroups of one XCD, to which the hardware
+// deals every eighth, so that a line is completed in one L2 and not written in pieces by eight.
+template <int NX, bool UNIFORM = true, bool NEAR = false>
 __device__ __forceinline__ bool seg_instance(int ncrms, int& c) {
-  int g = (blockIdx.x * blockDim.x + threadIdx.x) / NX;
+  unsigned b = blockIdx.x;
+  if constexpr (NEAR) {
+    const unsigned J = ::max(1u, 16u * NX / blockDim.x), G = 8 * J;  // workgroups of 16 instances, and of eight times as many
+    const unsigned base = b / G * G, r = b - base;
+    if (base + G <= gridDim.x) b = base + (r & 7) * J + (r >> 3);
+  }
+  int g = (b * blockDim.x + threadIdx.x) / NX;
   if constexpr (NX >= 64 && UNIFORM) g = __builtin_amdgcn_readfirstlane(g);
   c = g < ncrms ? g : ncrms - 1;
   return g < ncrms;

@@ -482,7 +482,7 @@ static int upload_transform(Engine<R>* ctx, int nx, int ny, double dx, Transform
 // 2).  Results are bitwise the same in every variant of a class.
 //
 // 8 x 4 was the fastest or within 2% of it at every size of the pressure solve that was timed (us
-// of a launch, 8 x 4 against the best of 1 to 4: 4096 x 64 x 28 508 and 508, mixed 295 and 298;
+// of a launch, 8 x 4 against the best of 1 to 4: 4096 x 64 x 58 508 and 508, mixed 295 and 298;
 // 500 x 64 x 58 65 and 66), so the other column counts have no variants.
 static int variants_of(int kid, int nx, bool y3) {
   if (kid == CRM_K_PRESS) return (nx == 64 && !y3) ? 5 : 1;

@@ -79,7 +79,7 @@ __device__ __forceinline__ void decide(unsigned long long* gmax, int nstep, int 
 // sponge profile damping.F90:44-61; roughness crm_module.F90:583-590 (z0_est
 // crmsurface.F90:104-131).  A workgroup of one wave per instance, a lane per level (level 64 and up
 // on the first lanes again): as one thread per instance every level waited for memory in turn
-// (16 x 28 levels 133 us, 500 x 58 453 us).
+// (16 x 28 levels 133 us, now 14; 500 x 58 453, now 20; 4096 x 58 470, now 48).
 // ------------------------------------------------------------------------------------------
 __device__ double z0_est(double z, double bflx, double wnd, double ustar, double c1) {
   const double vonk = R4(0.4), am = R4(4.8), bm = R4(19.3), eps = R4(1.e-10);
@@ -269,7 +269,7 @@ template <int NX, typename R>
 __global__ void CRM_LB k_init(DevT<R> d, crm_input_view in, crm_state_view st, crm_output_view out, double dt_gl) {
   SegFor<NX> s;
   int c;
-  bool live = seg_instance<NX>(d.ncrms, c);
+  bool live = seg_instance<NX, true, true>(d.ncrms, c);
   const int nzm = d.nzm, nz = d.nz, ld = d.ld, plev = d.plev, i = s.i;
   const double umax = 0.5 * d.dx / d.dt, factor_xy = 1. / (double)NX, idt_gl = 1. / dt_gl;
   const bool y3 = d.ny > 1;  // 3D: NX == 64 columns = 8 x 8, lane 8 j + i is the state's (i, j)
@@ -1268,7 +1268,7 @@ __global__ void CRM_LB k_mom(DevT<R> d, int na) {
 //
 // A launch, before (the loops at 8, 16, 32 and 128 columns; 64: 4 waves, the factors in LDS or in
 // registers) -> now, us: 256 x 128 x 58 217 -> 88, 16 x 32 x 28 31 -> 18, 866 x 32 x 28 54 -> 30,
-// 1024 x 4x4 x 28 36 -> 24, 500 x 64 x 58 75 -> 65, 4096 x 64 x 28 535 -> 508 and mixed 345 -> 295.
+// 1024 x 4x4 x 28 36 -> 24, 500 x 64 x 58 75 -> 65, 4096 x 64 x 58 535 -> 508 and mixed 345 -> 295.
 // Bound: memory, in phases.  The registers of the batched loads allow two workgroups of a CU, so
 // the transforms and the sweep of one are covered by the loads and stores of one other; at 4096
 // instances a launch moves 22 words per cell (8 of them again, for the gradient) at 2.5 TB/s.
@@ -3167,15 +3167,17 @@ __global__ void CRM_LB k_stats(DevT<R> d) {
 // End of call: crm_module.F90:1078-1659.  State write-back and every crm_output member.  The levels
 // are dealt to gridDim.y - 1 chunks; the last workgroup of an instance does what belongs to the
 // column, a lane per GCM level.  One lane writes a level's 45 means, which waits for memory
-// several times a level: with the levels one after the other 266 us at 16 x 32 x 28 and 800 us at
-// 500 x 64 x 58.  Large batches are bound by the write-back, whose columns lie an instance count apart.
+// several times a level: with the levels one after the other 266 us at 16 x 32 x 28 (now 17), 800 at
+// 500 x 64 x 58 (371).  Larger batches are bound by the write-back, whose columns lie an instance
+// count apart: a line's 16 instances on one XCD (seg_instance) took 467 to 371 there, 444 to 306 at
+// 256 x 128 x 58 and 3870 to 3430 at 4096 x 64 x 58.
 // ------------------------------------------------------------------------------------------
 template <int NX, typename R>
 __global__ void CRM_LB k_final(DevT<R> d, crm_input_view in, crm_state_view st, crm_rad_view rad, crm_output_view out,
                         double dt_gl, int nstop) {
   SegFor<NX> s;
   int c;
-  bool live = seg_instance<NX>(d.ncrms, c);
+  bool live = seg_instance<NX, true, true>(d.ncrms, c);
   const int nzm = d.nzm, nz = d.nz, ld = d.ld, plev = d.plev, i = s.i;
   const double factor_xy = 1. / (double)NX, factor_xyt = factor_xy / (double)nstop;
   const double icrm_run_time = 1. / dt_gl, dz = inst(d, I_DZ, c);
