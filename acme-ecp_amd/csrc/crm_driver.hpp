@@ -89,8 +89,14 @@ struct Engine : CrmEngine {
   int acc_use = 0, acc_uv = 0;
   double acc_factor = 0.0;
   // launch schedule: threads per workgroup of each segment-kernel class (a multiple of 64 up
-  // to 256; instances per workgroup = block / columns), set by the autotuner
-  int block[CRM_K_COUNT] = {256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256};
+  // to 256; instances per workgroup = block / columns), set by the autotuner.  k_micro of the
+  // FP64 engine starts with 64: its waves end at different times, and a workgroup keeps its
+  // registers until the last (4096 x 64 x 58: 588 us with 256, 476 with 128, 454 with 64; 1024 x 64
+  // x 58: 150, 127, 126).  Mixed 246, 234, 232, but gathering the next kurant maximum it is
+  // slower (a call 431 ms with 256, 437 with 64).  The other sweeps are within 5% of 256 or slower.
+  static constexpr int MICRO_BLOCK = sizeof(R) == 8 ? 64 : 256;
+  int block[CRM_K_COUNT] = {256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256, MICRO_BLOCK, 256, 256};
+  static_assert(CRM_K_MICRO == 12, "position of k_micro's default");
   // launch variant of each kernel class (variants_of), set by the autotuner
   int variant[CRM_K_COUNT] = {};
   // HIP graphs of the steady substep (one subcycle, constant Adams-Bashforth coefficients),
@@ -1529,10 +1535,11 @@ int Engine<R>::autotune(const crm_dims* dims, const crm_column_info* col, double
     }
   }
   for (int k = 0; k < CRM_K_COUNT; k++) {
-    // 256 threads and the default variant unless another measured faster by more than 3%
-    // (timing noise of a short trial call is a few percent)
-    int bc = 2, bv = 0;
-    double bt = t[2][0][k];
+    // the default threads and variant unless another measured faster by more than 3% (timing noise
+    // of a short trial call is a few percent)
+    const int dc = k == CRM_K_MICRO && MICRO_BLOCK == 64 ? 0 : 2;
+    int bc = dc, bv = 0;
+    double bt = t[dc][0][k];
     for (int v = 0; v < variants_of(k, nxc, y3); v++)
       for (int c = 0; c < 3; c++)
         if (t[c][v][k] > 0.0 && t[c][v][k] < bt) {
@@ -1540,8 +1547,8 @@ int Engine<R>::autotune(const crm_dims* dims, const crm_column_info* col, double
           bv = v;
           bt = t[c][v][k];
         }
-    if (!(bt < 0.97 * t[2][0][k])) {
-      bc = 2;
+    if (!(bt < 0.97 * t[dc][0][k])) {
+      bc = dc;
       bv = 0;
     }
     block[k] = cand[bc];

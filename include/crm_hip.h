@@ -239,7 +239,8 @@ int crm_hip_get_variants(const crm_hip_ctx *ctx, int variant[CRM_HIP_NKERNEL]);
 
 /* Autotuner: runs the call once per candidate workgroup size (64, 128, 256) and launch variant,
  * with every kernel class timed on the context's stream, keeps the fastest (size, variant) of
- * each class (the default 256 threads and variant 0 unless another is faster by more than 3%)
+ * each class (the default threads - 256, for CRM_K_MICRO in FP64 64 - and variant 0
+ * unless another is faster by more than 3%)
  * for later calls of this context and writes the sizes to block_out (may be NULL;
  * crm_hip_get_variants gives the variants). The views are device pointers and are advanced by
  * every trial call: pass scratch copies. */
