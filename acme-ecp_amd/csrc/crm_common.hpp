@@ -13,6 +13,7 @@
 #include <stdint.h>
 
 #include "crm_pow.hpp"
+#include "crm_round.hpp"
 
 // The FP64 form is compiled in namespace crm; the mixed-precision form (FP32 bulk fields) is
 // compiled from the same sources in its own translation unit and namespace.

@@ -1299,6 +1299,9 @@ struct PressShape {
 // NW: waves of the workgroup; PB: rows of a wave whose loads are issued together
 template <int NX, typename R, typename G, int NW = 8, int PB = 4>
 __global__ void __launch_bounds__(64 * NW) k_press(DevT<R> d, int na, int nb, int nc) {
+// every fused product is spelled out, so that the bits do not hang on how the compiler arranges
+// the loops
+#pragma clang fp contract(off)
   CRM_STOP_CHECK(d);
   using SH = PressShape<NX>;
   constexpr int COLS = SH::COLS, NI = SH::NI, LD = SH::LD, WPR = SH::WPR;
@@ -1380,13 +1383,17 @@ __global__ void __launch_bounds__(64 * NW) k_press(DevT<R> d, int na, int nb, in
       double rup = rhow[k + 1] / rho[k] * rdz;
       double rdn = rhow[k] / rho[k] * rdz;
       const double uu = v[q][0], uap = v[q][1], ubp = v[q][2], ucp = v[q][3];
-      double pv;
+      // the divergence of one time level, and the sum over the levels
+      auto wz = [&](int up, int dn) { return fma(v[q][up], rup, -(v[q][dn] * rdn)); };
+      double d0, da, db, dc;
       if constexpr (G::Y3) {  // press_rhs.F90:45-69
-        const double vv = v[q][12], vap = v[q][13], vbp = v[q][14], vcp = v[q][15];
-        pv = (rdx * (s.rot(uu, 1) - uu) + rdx * (s.roty(vv, 1) - vv) + (v[q][8] * rup - v[q][4] * rdn)) * dta +
-             (rdx * (s.rot(uap, 1) - uap) + rdx * (s.roty(vap, 1) - vap) + (v[q][9] * rup - v[q][5] * rdn)) +
-             btat * (rdx * (s.rot(ubp, 1) - ubp) + rdx * (s.roty(vbp, 1) - vbp) + (v[q][10] * rup - v[q][6] * rdn)) +
-             ctat * (rdx * (s.rot(ucp, 1) - ucp) + rdx * (s.roty(vcp, 1) - vcp) + (v[q][11] * rup - v[q][7] * rdn));
+        auto div = [&](double u, double v_, double z) {
+          return fma(s.rot(u, 1) - u, rdx, (s.roty(v_, 1) - v_) * rdx) + z;
+        };
+        d0 = div(uu, v[q][12], wz(8, 4));
+        da = div(uap, v[q][13], wz(9, 5));
+        db = div(ubp, v[q][14], wz(10, 6));
+        dc = div(ucp, v[q][15], wz(11, 7));
       } else {
         double un, uan_, ubn, ucn;  // the next column's
         if constexpr (NX > 64) {
@@ -1394,11 +1401,12 @@ __global__ void __launch_bounds__(64 * NW) k_press(DevT<R> d, int na, int nb, in
         } else {
           un = s.rot(uu, 1), uan_ = s.rot(uap, 1), ubn = s.rot(ubp, 1), ucn = s.rot(ucp, 1);
         }
-        pv = (rdx * (un - uu) + (v[q][8] * rup - v[q][4] * rdn)) * dta +
-             (rdx * (uan_ - uap) + (v[q][9] * rup - v[q][5] * rdn)) +
-             btat * (rdx * (ubn - ubp) + (v[q][10] * rup - v[q][6] * rdn)) +
-             ctat * (rdx * (ucn - ucp) + (v[q][11] * rup - v[q][7] * rdn));
+        d0 = fma(un - uu, rdx, wz(8, 4));
+        da = fma(uan_ - uap, rdx, wz(9, 5));
+        db = fma(ubn - ubp, rdx, wz(10, 6));
+        dc = fma(ucn - ucp, rdx, wz(11, 7));
       }
+      const double pv = fma(dc, ctat, fma(db, btat, fma(d0, dta, da)));
       P[k * LD + col] = pv * rho[k];
     }
   }
@@ -1474,14 +1482,14 @@ __global__ void __launch_bounds__(64 * NW) k_press(DevT<R> d, int na, int nb, in
       ck_n = cc[k + 1];
       rk_n = cr[k + 1];
       pk_n = P[(k + 1) * LD + col];
-      double e = 1.0 / (eig * rk - ak - ck + ak * alfa);
+      double e = 1.0 / fma(ak, alfa, fma(eig, rk, -ak) - ck);
       alfa = -ck * e;
       ALF[k * COLS + col] = alfa;
-      beta = (pk - ak * beta) * e;
+      beta = fma(-ak, beta, pk) * e;
       P[k * LD + col] = beta;
     }
     {
-      double top = (pk_n - ak_n * beta) / (eig * rk_n - ak_n + ak_n * alfa);
+      double top = fma(-ak_n, beta, pk_n) / fma(ak_n, alfa, fma(eig, rk_n, -ak_n));
       P[(nzm - 1) * LD + col] = top;
       double an = ALF[(nzm - 2) * COLS + col], pn = P[(nzm - 2) * LD + col];
       for (int kk = nzm - 2; kk >= 0; kk--) {
@@ -1489,7 +1497,7 @@ __global__ void __launch_bounds__(64 * NW) k_press(DevT<R> d, int na, int nb, in
         const int kb = ::max(kk - 1, 0);
         an = ALF[kb * COLS + col];
         pn = P[kb * LD + col];
-        top = af * top + pk;
+        top = fma(af, top, pk);
         P[kk * LD + col] = top;
       }
     }
@@ -1502,22 +1510,14 @@ __global__ void __launch_bounds__(64 * NW) k_press(DevT<R> d, int na, int nb, in
   R* wan = d.dwdt[na];
   R* unc = d.dudt[nc];
   R* wnc = d.dwdt[nc];
-  // the weighted tendencies of the three time levels; which of the first two products is rounded
-  // by itself is spelled out where the compiler's choice hangs on the arrangement of the loop
-  auto ab3 = [&](double a, double b, double c_) {
-    if constexpr (std::is_same<R, double>::value && (NX == 128 || (NX == 16 && G::Y3)))
-      return fma(d.ct, c_, fma(d.at, a, d.bt * b));
-    else if constexpr (std::is_same<R, double>::value && NX == 64)
-      return fma(d.ct, c_, fma(d.bt, b, d.at * a));
-    else
-      return d.at * a + d.bt * b + d.ct * c_;
+  // the weighted tendencies of the three time levels
+  constexpr bool FP64 = std::is_same<R, double>::value;
+  auto ab3 = [&](auto field, double a, double b, double c_) {
+    return ab_sum<ab_alone(decltype(field)::value, NX, G::Y3, FP64)>(d.at, a, d.bt, b, d.ct, c_);
   };
-  auto bc = [&](double b, double c_) {
-    if constexpr (std::is_same<R, double>::value && G::Y3)
-      return fma(d.bt, b, d.ct * c_);
-    else
-      return d.bt * b + d.ct * c_;
-  };
+  std::integral_constant<AbField, AbField::U> fu;
+  std::integral_constant<AbField, AbField::V> fv;
+  std::integral_constant<AbField, AbField::W> fw;
   for (int k0 = w0; k0 < nzm; k0 += RW * PB) {
     double v[PB][12];
 #pragma unroll
@@ -1552,23 +1552,17 @@ __global__ void __launch_bounds__(64 * NW) k_press(DevT<R> d, int na, int nb, in
         pim = s.rot(pk, -1);
       double pkb = P[(k > 0 ? k - 1 : 0) * LD + col];
       double rdz = 1. / (dz * adzw[k]);
-      double du_a = v[q][0] - (pk - pim) * rdx;
-      double dw_a = v[q][1] - (pk - pkb) * rdz;
+      double du_a = fma(-(pk - pim), rdx, v[q][0]);
+      double dw_a = fma(-(pk - pkb), rdz, v[q][1]);
       double uu = v[q][2], ww = v[q][3];
-      double un, wn;
-      if constexpr (NX == 64) {  // the b and c terms first
-        un = uu + dt3 * (d.at * du_a + bc(v[q][4], v[q][5]));
-        wn = ww + dt3 * (d.at * dw_a + bc(v[q][6], v[q][7]));
-      } else {
-        un = uu + dt3 * ab3(du_a, v[q][4], v[q][5]);
-        wn = ww + dt3 * ab3(dw_a, v[q][6], v[q][7]);
-      }
+      double un = fma(dt3, ab3(fu, du_a, v[q][4], v[q][5]), uu);
+      double wn = fma(dt3, ab3(fw, dw_a, v[q][6], v[q][7]), ww);
       double dv_a = 0.0, vn = 0.0, vv = 0.0;
       if constexpr (G::Y3) {  // press_grad.F90:29, adams.F90:29,32
         double pjm = s.roty(pk, -1);
-        dv_a = v[q][8] - (pk - pjm) * rdx;
+        dv_a = fma(-(pk - pjm), rdx, v[q][8]);
         vv = v[q][9];
-        vn = vv + dt3 * ab3(dv_a, v[q][10], v[q][11]);
+        vn = fma(dt3, ab3(fv, dv_a, v[q][10], v[q][11]), vv);
       }
       if (live) {
         uan[o] = du_a;
