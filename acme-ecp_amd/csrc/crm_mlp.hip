@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "../../include/crm_mlp.h"
+#include "crm_index.hpp"
 #include "crm_mlp_dev.hpp"
 
 namespace crm_mlp_ns {
@@ -158,8 +159,8 @@ __global__ void __launch_bounds__(256) k_train(const float* X, const float* T, i
   }
   float gb[3] = {0.f, 0.f, 0.f}, gb4 = 0.f, e2 = 0.f;
   const int row = 16 * wave + r;
-  for (int tile = blockIdx.x; tile * TROWS < n; tile += gridDim.x) {
-    const long m = (long)tile * TROWS + row;
+  for (Strided tile = tiles_of(n, TROWS, blockIdx.x, gridDim.x); tile.more(); tile.next()) {
+    const long m = tile.at * TROWS + row;
     const bool have = m < n;
     // an offset the compiler cannot see through, so that the weight reads stay inside the loop
     // (hoisted out of it, the network would be held in registers and spill)
