@@ -15,6 +15,7 @@
 
 #include "../../include/crm_glue.h"
 #include "crm_engine.hpp"
+#include "crm_index.hpp"
 
 #pragma clang fp contract(off)
 
@@ -33,11 +34,8 @@ struct Cols {
 // Rows of 64 columns: a workgroup covers 64 columns of RPB rows at a time; rows beyond the
 // grid's are reached by striding.
 constexpr int COLS = 64, RPB = 4;
-struct RowRange {
-  int first, step;
-};
-__device__ __forceinline__ RowRange my_rows() {
-  return {(int)(blockIdx.y * RPB + threadIdx.y), (int)(gridDim.y * RPB)};
+__device__ __forceinline__ Strided my_rows(long rows) {
+  return {(long)blockIdx.y * RPB + threadIdx.y, (long)gridDim.y * RPB, rows};
 }
 __device__ __forceinline__ int my_column() { return (int)(blockIdx.x * COLS + threadIdx.x); }
 
@@ -50,19 +48,18 @@ __global__ void __launch_bounds__(COLS* RPB) k_gcm_input(int ncol, int pcols, in
   if (i >= ncol) return;
   const Cols L{pcols};
   auto W = [](const double* p) { return const_cast<double*>(p); };
-  const int nrows = pver + 1 + nrad * crm_nz;
-  const RowRange rr = my_rows();
-  for (int row = rr.first; row < nrows; row += rr.step) {
-    if (row > pver) {
+  for (Strided row = my_rows(pver + 1 + (long)nrad * crm_nz); row.more(); row.next()) {
+    if (row.at > pver) {
       // Q dp -> heating rate on the CRM levels (CRM level m sits on GCM level pver-1-m)
-      const int mr = row - pver - 1, m = mr / nrad;
+      const long mr = row.at - pver - 1;
+      const int m = level_of(mr, nrad);
       const double dp = st.pdel[L.at(i, pver - 1 - m)];
       double* qrad = W(rad.qrad);
       const size_t o = (size_t)i + (size_t)pcols * mr;
       qrad[o] = qrad[o] / dp;
       continue;
     }
-    const int k = row;
+    const int k = (int)row.at;
     const size_t o = L.at(i, k);
     W(in.zint)[o] = st.zi[o];
     W(in.pint)[o] = st.pint[o];
@@ -98,10 +95,9 @@ __global__ void __launch_bounds__(COLS* RPB) k_flux_bypass(int ncol, int pcols, 
                                                            double* pq) {
   const int i = my_column();
   if (i >= ncol) return;
-  const RowRange rr = my_rows();
-  for (int k = rr.first; k < pver; k += rr.step) {
-    const size_t o = (size_t)i + (size_t)pcols * k;
-    if (k < pver - 1) {
+  for (Strided k = my_rows(pver); k.more(); k.next()) {
+    const size_t o = (size_t)i + (size_t)pcols * k.at;
+    if (k.at < pver - 1) {
       ps_[o] = 0.;
       pq[o] = 0.;
     } else {
@@ -130,11 +126,11 @@ __global__ void __launch_bounds__(COLS* SUM_WAVES) k_gcm_tend(int ncol, int pcol
   if ((int)blockIdx.x < nq) {
     // heating rate -> Q dp on the CRM levels (CRM level m sits on GCM level pver-1-m)
     double* qrad = const_cast<double*>(rad.qrad);
-    const int rows = nrad * crm_nz;
-    for (int i = lane; i < ncol; i += COLS)
-      for (int mr = (int)blockIdx.x * SUM_WAVES + wave; mr < rows; mr += nq * SUM_WAVES) {
-        const double dp = pdel[L.at(i, pver - 1 - mr / nrad)];
-        const size_t o = (size_t)i + (size_t)pcols * mr;
+    for (long i = lane; i < ncol; i += COLS)
+      for (Strided mr{(long)blockIdx.x * SUM_WAVES + wave, (long)nq * SUM_WAVES, (long)nrad * crm_nz}; mr.more();
+           mr.next()) {
+        const double dp = pdel[L.at((int)i, pver - 1 - level_of(mr.at, nrad))];
+        const size_t o = (size_t)i + (size_t)pcols * mr.at;
         qrad[o] = qrad[o] * dp;
       }
     return;
@@ -240,11 +236,10 @@ __global__ void __launch_bounds__(COLS* RPB) k_rad_columns(int ncol, int pcols, 
                                                            crm_rad_view rad, crm_rad_column_view out) {
   const int i = my_column();
   if (i >= ncol) return;
-  const RowRange rr = my_rows();
-  for (int row = rr.first; row < nrad * pver; row += rr.step) {
-    const int k = row / nrad, r = row - k * nrad;
+  for (Strided row = my_rows((long)nrad * pver); row.more(); row.next()) {
+    const int k = level_of(row.at, nrad), r = (int)(row.at - (long)k * nrad);
     const size_t g = (size_t)i + (size_t)pcols * k;    // (pcols,pver)
-    const size_t o = (size_t)i + (size_t)pcols * row;  // (pcols,nrad,pver)
+    const size_t o = (size_t)i + (size_t)pcols * row.at;  // (pcols,nrad,pver)
     const int m = pver - 1 - k;  // CRM level on GCM level k
     if (m >= crm_nz) {  // above the CRM: the GCM column's values
       out.t[o] = st.t[g];
@@ -282,9 +277,8 @@ __global__ void __launch_bounds__(COLS* RPB) k_rad_qrad(int ncol, int pcols, lon
                                                         const double* qrl, double* qrad) {
   const int i = my_column();
   if (i >= ncol) return;
-  const RowRange rr = my_rows();
-  for (long row = rr.first; row < rows; row += rr.step) {
-    const size_t o = (size_t)i + (size_t)pcols * row;
+  for (Strided row = my_rows(rows); row.more(); row.next()) {
+    const size_t o = (size_t)i + (size_t)pcols * row.at;
     qrad[o] = qrs[o] + qrl[o];
   }
 }

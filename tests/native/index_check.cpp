@@ -1,11 +1,16 @@
 // Walks of crm_index.hpp on the host: argv rows, tile, blocks; prints how many tiles all blocks
 // take together, the first row of the last tile and whether an index ever fell or went below 0.
+// With four arguments (row nrad 0 0): the level of a row.
 #include <cstdio>
 #include <cstdlib>
 
 #include "crm_index.hpp"
 
-int main(int, char** argv) {
+int main(int argc, char** argv) {
+  if (argc == 5) {
+    std::printf("%d\n", level_of(std::atol(argv[1]), std::atoi(argv[2])));
+    return 0;
+  }
   const long rows = std::atol(argv[1]);
   const int tile = std::atoi(argv[2]);
   const unsigned blocks = (unsigned)std::atol(argv[3]);

@@ -26,6 +26,21 @@ def test_training_tiles(walk, rows, blocks):
     assert (taken, last, wrapped) == (-(-rows // 64), (rows - 1) // 64 * 64, 0)
 
 
+# rows on both sides of 2^31 and 2^32, with the levels of 28-level columns of that many
+@pytest.mark.parametrize("row", [0, 1, 2**31 - 1, 2**31, 2**32 - 1, 2**32, 28 * (2**31 - 1) - 1])
+@pytest.mark.parametrize("nrad", [1, 16, 76695845, 2**31 - 1])
+def test_level_of_a_row(walk, row, nrad):
+    if row // nrad <= INT_MAX:
+        assert walk(row, nrad, 0, 0) == [row // nrad]
+
+
+def test_gcm_kernels_count_rows_with_it():
+    src = open(os.path.join(ROOT, "acme-ecp_amd", "csrc", "crm_glue.hip")).read()
+    assert src.count("(long)nrad * crm_nz") + src.count("(long)nrad * pver") >= 6
+    for product in ("nrad * crm_nz", "nrad * pver"):
+        assert src.count(product) == src.count("(long)" + product)
+
+
 def test_training_kernel_walks_its_tiles_with_it():
     src = open(os.path.join(ROOT, "acme-ecp_amd", "csrc", "crm_mlp.hip")).read()
     body = src[src.index("k_train("):src.index("k_reduce(")]
