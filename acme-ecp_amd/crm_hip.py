@@ -36,7 +36,7 @@ ABI_SYMBOLS = ["crm_hip_init", "crm_hip_run", "crm_hip_run_device", "crm_hip_run
 DEBUG_SYMBOLS = ["crm_hip_debug_run", "crm_hip_debug_get", "crm_hip_fft991_operators",
                  "crm_hip_profile_kernels", "crm_hip_kernel_time", "crm_hip_kernel_name",
                  "crm_hip_graph_launches", "crm_hip_graph_cache_size",
-                 "crm_hip_debug_stop_call_at"]
+                 "crm_hip_debug_stop_call_at", "crm_hip_launch_shape"]
 # Kernel classes of one call (CRM_K_* of include/crm_hip_debug.h), in launch order.
 KERNELS = ["setup", "init", "setperturb", "kurant", "precip_init", "pre", "sgs", "mom", "press",
            "mpdata", "precip", "diffuse", "micro", "stats", "final"]
@@ -102,6 +102,7 @@ def load():
     lib.crm_hip_autotune.argtypes = views + [IA]
     lib.crm_hip_set_graphs.argtypes = [P, C.c_int]
     lib.crm_hip_debug_stop_call_at.argtypes = [P, C.c_int]
+    lib.crm_hip_launch_shape.argtypes = [P, C.POINTER(CrmDims), C.c_int, C.c_int * 4]
     lib.crm_hip_graph_launches.argtypes = [P]
     lib.crm_hip_graph_launches.restype = C.c_longlong
     lib.crm_hip_graph_cache_size.argtypes = [P]
@@ -215,6 +216,8 @@ class CrmHip:
         return dict(zip(KERNELS, list(a)))
 
     def set_schedule(self, sched):
+        """Threads per workgroup of the named classes; the others keep those of schedule().  From
+        then on all of them hold for every batch size."""
         cur = self.schedule()
         cur.update(sched)
         a = (C.c_int * len(KERNELS))(*[cur[k] for k in KERNELS])
@@ -267,6 +270,15 @@ class CrmHip:
         rc = self.lib.crm_hip_debug_stop_call_at(self.ctx, int(nstep))
         if rc:
             raise CrmError(rc, "crm_hip_debug_stop_call_at")
+
+    def launch_shape(self, dims, kernel):
+        """(threads per workgroup, chunks of levels, scalars handed on, variant) of a kernel class
+        in a call of these dimensions."""
+        a = (C.c_int * 4)()
+        rc = self.lib.crm_hip_launch_shape(self.ctx, C.byref(dims), KERNELS.index(kernel), a)
+        if rc:
+            raise CrmError(rc, "crm_hip_launch_shape")
+        return tuple(a)
 
     def debug_run(self, case, dt_gl, phase_stop):
         return self._call(self.lib.crm_hip_debug_run, case.dims(), case.column_info(), dt_gl,

@@ -89,14 +89,18 @@ struct Engine : CrmEngine {
   int acc_use = 0, acc_uv = 0;
   double acc_factor = 0.0;
   // launch schedule: threads per workgroup of each segment-kernel class (a multiple of 64 up
-  // to 256; instances per workgroup = block / columns), set by the autotuner.  k_micro of the
+  // to 256; instances per workgroup = block / columns).  Until the caller or the autotuner sets it
+  // (sized), batches of fewer waves than the device has SIMDs use 64.  k_micro of the
   // FP64 engine starts with 64: its waves end at different times, and a workgroup keeps its
   // registers until the last (4096 x 64 x 58: 588 us with 256, 476 with 128, 454 with 64; 1024 x 64
   // x 58: 150, 127, 126).  Mixed 246, 234, 232, but gathering the next kurant maximum it is
   // slower (a call 431 ms with 256, 437 with 64).  The other sweeps are within 5% of 256 or slower.
   static constexpr int MICRO_BLOCK = sizeof(R) == 8 ? 64 : 256;
-  int block[CRM_K_COUNT] = {256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256, 256, MICRO_BLOCK, 256, 256};
+  static constexpr int DEFAULT_BLOCK[CRM_K_COUNT] = {256, 256, 256, 256, 256, 256, 256,         256,
+                                                     256, 256, 256, 256, MICRO_BLOCK, 256, 256};
+  int block[CRM_K_COUNT];
   static_assert(CRM_K_MICRO == 12, "position of k_micro's default");
+  bool sized = false;
   // launch variant of each kernel class (variants_of), set by the autotuner
   int variant[CRM_K_COUNT] = {};
   // HIP graphs of the steady substep (one subcycle, constant Adams-Bashforth coefficients),
@@ -153,6 +157,7 @@ struct Engine : CrmEngine {
   }
   int graph_cache_size() const override { return (int)graphs.size(); }
 
+  Engine() { std::copy(DEFAULT_BLOCK, DEFAULT_BLOCK + CRM_K_COUNT, block); }
   ~Engine() override;
   int run(const crm_dims* dims, const crm_column_info* col, double dt_gl, const crm_input_view* in,
           crm_state_view* state, crm_rad_view* rad, crm_output_view* out, bool device_views,
@@ -175,6 +180,7 @@ struct Engine : CrmEngine {
     for (int k = 0; k < CRM_K_COUNT; k++)
       if (blk[k] < 64 || blk[k] > 256 || blk[k] % 64) return CRM_ERR_ARG;
     for (int k = 0; k < CRM_K_COUNT; k++) block[k] = blk[k];
+    sized = true;
     drop_graphs();
     return CRM_OK;
   }
@@ -191,6 +197,7 @@ struct Engine : CrmEngine {
   void get_variants(int* v) const override {
     for (int k = 0; k < CRM_K_COUNT; k++) v[k] = variant[k];
   }
+  int launch_shape(const crm_dims* dims, int kid, int shape[4]) const override;
   void set_graphs(int mode) override {
     use_graphs = mode;
     drop_graphs();
@@ -513,23 +520,25 @@ static void launch_press(int nzm, hipStream_t s, const DevT<R>& d, int na, int n
   start_press<NX, R, G, 8, 4>(nzm, s, d, na, nb, nc);
 }
 
+// levels per trip of the other kind than the default, registers bounded for three waves per SIMD,
+// levels dealt to several workgroups
+struct MpdataKind {
+  bool other, w3, split;
+};
+
 // o: where the advected fields go (their own buffers, or the hand-over buffers of split sweeps)
 template <int NX, typename R, typename G>
-static void launch_mpdata(dim3 g, dim3 b, hipStream_t s, const DevT<R>& d, const Scalars<R>& o, bool split,
-                          int variant) {
+static void launch_mpdata(dim3 g, dim3 b, hipStream_t s, const DevT<R>& d, const Scalars<R>& o, MpdataKind kind) {
   constexpr bool PAIR = (NX == 64 && !G::Y3);
-  const bool other = variant == 1 || variant == 3;
   const int nb = (int)g.x;
-  const bool many = PAIR && (size_t)nb * b.x >= (size_t)64 * 2048;
-  const bool w3 = variant == 0 ? many : variant == 2 || variant == 3 || variant == 5;
   g.x *= 3;  // a grid per scalar
-  if (split)
+  if (kind.split)
     k_mpdata<NX, R, G, PAIR, false, true><<<g, b, 0, s>>>(d, nb, o);
-  else if (w3 && other)
+  else if (kind.w3 && kind.other)
     k_mpdata<NX, R, G, !PAIR, true, false><<<g, b, 0, s>>>(d, nb, o);
-  else if (w3)
+  else if (kind.w3)
     k_mpdata<NX, R, G, PAIR, true, false><<<g, b, 0, s>>>(d, nb, o);
-  else if (other)
+  else if (kind.other)
     k_mpdata<NX, R, G, !PAIR, false, false><<<g, b, 0, s>>>(d, nb, o);
   else
     k_mpdata<NX, R, G, PAIR, false, false><<<g, b, 0, s>>>(d, nb, o);
@@ -539,6 +548,7 @@ struct Launcher {
   int nx, nzm, ncrms;
   hipStream_t s;
   const int* block;  // threads per workgroup of each kernel class
+  bool sized;        // block is the caller's or the autotuner's choice
   bool split;        // the scalars are handed on through other buffers (mpdata, precip, diffuse)
   dim3 grid_inst(int b) const { return dim3((unsigned)((ncrms + b - 1) / b)); }
   int waves() const { return (int)(((size_t)ncrms * nx + 63) / 64); }
@@ -574,12 +584,30 @@ struct Launcher {
     return n;
   }
   // From 1024 waves on, MPDATA and the sedimentation are not cut (chunks), and the scalars are
-  // updated in place (k_diffuse at 4096 x 64 x 58: 181 us from one buffer to another, 169 in place)
-  static bool split_batch(int ncrms, int columns) { return (size_t)ncrms * columns < (size_t)64 * 1024; }
+  // updated in place (k_diffuse at 4096 x 64 x 58: 181 us from one buffer to another, 169 in place).
+  // MPDATA's variants other than 0 are sweeps over all levels, in place at every size.
+  static bool split_batch(int ncrms, int columns, int mpdata_variant) {
+    return mpdata_variant == 0 && (size_t)ncrms * columns < (size_t)64 * 1024;
+  }
+  // The instance of k_mpdata that a variant means.  The register bound of variant 0: at 64 columns
+  // in 2D from 2048 waves on (two per SIMD), where a third wave per SIMD has work.
+  MpdataKind mpdata(int variant, bool y3) const {
+    const bool many = nx == 64 && !y3 && waves() >= 2048;
+    return {variant == 1 || variant == 3, variant == 0 ? many : variant == 2 || variant == 3 || variant == 5, split};
+  }
+  // classes whose workgroups are not sized by the schedule: one wave (k_setup, k_setperturb), 128
+  // threads (k_precip_init), the waves of the variant (k_press), a wave per chunk (k_precip_wg)
+  bool takes_size(int kid) const {
+    switch (kid) {
+      case CRM_K_SETUP: case CRM_K_SETPERTURB: case CRM_K_PRECIP_INIT: case CRM_K_PRESS: return false;
+      case CRM_K_PRECIP: return nx != 128 && chunks(kid) == 1;
+      default: return nx != 128;
+    }
+  }
   // threads per workgroup of segment-kernel class kid: 128-column instances span two waves
   // whose exchanges are workgroup barriers, so they run one instance per workgroup; a batch
   // of fewer waves than the device has SIMDs is spread one wave per workgroup
-  int bs(int kid) const { return nx == 128 ? 128 : waves() < 1024 ? 64 : block[kid]; }
+  int bs(int kid) const { return nx == 128 ? 128 : !sized && waves() < 1024 ? 64 : block[kid]; }
   // grid and workgroup of segment-kernel class kid
   dim3 g(int kid) const {
     return dim3((unsigned)(((size_t)ncrms * nx + bs(kid) - 1) / bs(kid)), (unsigned)chunks(kid));
@@ -805,7 +833,8 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
   d.docoriolis = ctx->coriolis;
   host_constants(d);
   // a debug run that stops inside a substep reads the fields in their own buffers
-  Launcher L{nx, nzm, ncrms, s, ctx->block, phase_stop == 0 && Launcher::split_batch(ncrms, nx)};
+  const Launcher L{nx, nzm, ncrms, s, ctx->block, ctx->sized,
+                   phase_stop == 0 && Launcher::split_batch(ncrms, nx, ctx->variant[CRM_K_MPDATA])};
   // the advected scalars after MPDATA and after the sedimentation (Scalars, crm_kernels.hpp)
   auto after_mpdata = [&]() { return L.split ? Scalars<R>{d.qcl, d.qci, d.qpl} : Scalars<R>{d.t, d.qt, d.qp}; };
   auto after_precip = [&]() { return L.split ? Scalars<R>{d.qcl, d.qci, d.qpi} : Scalars<R>{d.t, d.qt, d.qp}; };
@@ -942,6 +971,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
     key.append((const char*)&qrad, sizeof(qrad));
     key.append((const char*)ctx->block, sizeof(ctx->block));
     key.append((const char*)ctx->variant, sizeof(ctx->variant));
+    key.push_back((char)ctx->sized);
     // the call's sequence; with launch false only the host bookkeeping is replayed
     auto sequence = [&](bool launch) {
       for (int n = 1; n <= nstop; n++) {
@@ -965,7 +995,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
           NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
           NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
           NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
-          NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA])));
+          NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.mpdata(ctx->variant[CRM_K_MPDATA], y3))));
           NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp)));
         }
         std::swap(d.u, d.dudt[nc]);
@@ -1085,7 +1115,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
         NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
         NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
         NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS])));
-        NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA])));
+        NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.mpdata(ctx->variant[CRM_K_MPDATA], y3))));
         NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp)));
         std::swap(d.u, d.dudt[nc]);
         std::swap(d.w, d.dwdt[nc]);
@@ -1152,7 +1182,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       if (last && phase_stop == 11) goto stopped;
       TIMED(CRM_K_PRESS, NX_DISPATCH(nx, (launch_press<NXV, R, GEO>(nzm, s, d, na, nb, nc, ctx->variant[CRM_K_PRESS]))));
       if (last && phase_stop == 13) goto stopped;
-      TIMED(CRM_K_MPDATA, NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.split, ctx->variant[CRM_K_MPDATA]))));
+      TIMED(CRM_K_MPDATA, NX_DISPATCH(nx, (launch_mpdata<NXV, R, GEO>(L.g(CRM_K_MPDATA), L.b(CRM_K_MPDATA), s, d, after_mpdata(), L.mpdata(ctx->variant[CRM_K_MPDATA], y3)))));
       TIMED(CRM_K_PRECIP, NX_DISPATCH(nx, (launch_precip<NXV, R>(L, d, after_mpdata().t, after_mpdata().qp, after_precip().qp, L.split ? d.qv : d.qp))));
       if (last && phase_stop == 15) goto stopped;
       std::swap(d.u, d.dudt[nc]);
@@ -1498,28 +1528,58 @@ int Engine<R>::debug_get(const char* name, double* buf) {
 }
 
 
+// What a call of these dimensions launches for a class with the present schedule and variants.
+template <typename R>
+int Engine<R>::launch_shape(const crm_dims* dims, int kid, int shape[4]) const {
+  if (int rc = validate(dims)) return rc;
+  const int nx = dims->nx * dims->ny;
+  const Launcher L{nx, dims->nz, dims->ncrms, nullptr, block, sized,
+                   Launcher::split_batch(dims->ncrms, nx, variant[CRM_K_MPDATA])};
+  const MpdataKind m = L.mpdata(variant[CRM_K_MPDATA], dims->ny > 1);
+  shape[0] = L.takes_size(kid) || nx == 128 ? L.bs(kid) : 0;
+  shape[1] = L.chunks(kid);
+  shape[2] = L.split;
+  shape[3] = kid == CRM_K_MPDATA ? m.other + 2 * m.w3 : variant[kid];
+  return CRM_OK;
+}
+
 // Workgroup sizes per kernel class: one call per candidate size with every class timed on
 // the stream, then the fastest size of each class.  The views are scratch: each call advances
 // them.
 template <typename R>
 int Engine<R>::autotune(const crm_dims* dims, const crm_column_info* col, double dt_gl, const crm_input_view* in,
                         crm_state_view* state, crm_rad_view* rad, crm_output_view* out, int* best) {
-  // every workgroup size (64, 128, 256) with every launch variant; each trial call times
-  // every kernel class
+  // every workgroup size (64, 128, 256) with every launch variant that this batch launches
+  // differently; each trial call times every kernel class
   static const int cand[] = {64, 128, 256};
+  if (int rc = validate(dims)) return rc;
   const unsigned saved_mask = prof_mask;
-  const bool y3 = dims && dims->ny > 1;
-  const int nxc = dims ? dims->nx * dims->ny : 0;
+  const bool y3 = dims->ny > 1;
+  const int nxc = dims->nx * dims->ny;
+  // the default launches of this batch
+  const Launcher L{nxc, dims->nz, dims->ncrms, stream, DEFAULT_BLOCK, false,
+                   Launcher::split_batch(dims->ncrms, nxc, 0)};
+  // MPDATA: variant 5 is 2 again; where the levels are dealt to workgroups the other variants would
+  // take that from the sedimentation and the diffusion as well, which their own time does not show
+  auto variants = [&](int k) { return k != CRM_K_MPDATA ? variants_of(k, nxc, y3) : L.split ? 1 : 5; };
+  auto defsize = [&](int k) {  // position in cand
+    const int threads = L.takes_size(k) ? L.bs(k) : DEFAULT_BLOCK[k];
+    return threads == 64 ? 0 : threads == 128 ? 1 : 2;
+  };
+  auto tried = [&](int k, int c, int v) { return v < variants(k) && (L.takes_size(k) || c == defsize(k)); };
   constexpr int NV = MAX_VARIANTS;
   double t[3][NV][CRM_K_COUNT] = {};
+  int saved_block[CRM_K_COUNT], saved_variant[CRM_K_COUNT];
+  const bool saved_sized = sized;
+  for (int k = 0; k < CRM_K_COUNT; k++) saved_block[k] = block[k], saved_variant[k] = variant[k];
+  sized = true;
   for (int v = 0; v < NV; v++) {
     for (int c = 0; c < 3; c++) {
-      bool any = false;  // a class whose variant v exists
+      bool any = false;  // a class that this trial launches in a new way
       for (int k = 0; k < CRM_K_COUNT; k++) {
-        block[k] = cand[c];
-        const int nv = variants_of(k, nxc, y3);
-        variant[k] = v < nv ? v : 0;
-        any |= v < nv;
+        block[k] = cand[L.takes_size(k) ? c : defsize(k)];
+        variant[k] = v < variants(k) ? v : 0;
+        any |= tried(k, c, v);
       }
       if (!any) continue;
       drop_graphs();
@@ -1527,20 +1587,22 @@ int Engine<R>::autotune(const crm_dims* dims, const crm_column_info* col, double
       int rc = run(dims, col, dt_gl, in, state, rad, out, true, 0);
       if (rc) {
         profile_kernels(saved_mask);
-        for (int k = 0; k < CRM_K_COUNT; k++) variant[k] = 0;
+        for (int k = 0; k < CRM_K_COUNT; k++) block[k] = saved_block[k], variant[k] = saved_variant[k];
+        sized = saved_sized;
+        drop_graphs();
         return rc;
       }
       for (int k = 0; k < CRM_K_COUNT; k++)
-        if (v < variants_of(k, nxc, y3)) t[c][v][k] = kt_n[k] ? kt_ms[k] / (double)kt_n[k] : 0.0;
+        if (tried(k, c, v)) t[c][v][k] = kt_n[k] ? kt_ms[k] / (double)kt_n[k] : 0.0;
     }
   }
   for (int k = 0; k < CRM_K_COUNT; k++) {
     // the default threads and variant unless another measured faster by more than 3% (timing noise
     // of a short trial call is a few percent)
-    const int dc = k == CRM_K_MICRO && MICRO_BLOCK == 64 ? 0 : 2;
+    const int dc = defsize(k);
     int bc = dc, bv = 0;
     double bt = t[dc][0][k];
-    for (int v = 0; v < variants_of(k, nxc, y3); v++)
+    for (int v = 0; v < variants(k); v++)
       for (int c = 0; c < 3; c++)
         if (t[c][v][k] > 0.0 && t[c][v][k] < bt) {
           bc = c;

@@ -67,6 +67,7 @@ struct CrmEngine {
   virtual void get_schedule(int* block) const = 0;
   virtual int set_variants(const int* variant) = 0;
   virtual void get_variants(int* variant) const = 0;
+  virtual int launch_shape(const crm_dims* dims, int kid, int shape[4]) const = 0;
   virtual void set_graphs(int mode) = 0;
   virtual int get_graphs() const = 0;
   virtual void set_debug_stop(int nstep) = 0;

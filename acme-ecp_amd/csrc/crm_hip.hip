@@ -314,6 +314,11 @@ int crm_hip_get_schedule(const crm_hip_ctx* ctx, int block[CRM_HIP_NKERNEL]) {
   return CRM_OK;
 }
 
+int crm_hip_launch_shape(const crm_hip_ctx* ctx, const crm_dims* dims, int kid, int shape[4]) {
+  if (!ctx || !ctx->eng || kid < 0 || kid >= CRM_K_COUNT || !shape) return CRM_ERR_ARG;
+  return ctx->eng->launch_shape(dims, kid, shape);
+}
+
 int crm_hip_set_coriolis(crm_hip_ctx* ctx, int docoriolis) {
   if (!ctx || !ctx->eng) return CRM_ERR_ARG;
   ctx->eng->set_coriolis(docoriolis);

@@ -222,26 +222,31 @@ typedef struct crm_class_desc {
 int crm_hip_run_many(int n, crm_hip_ctx *const *ctxs, const crm_class_desc *classes, double dt_gl,
                      int *status);
 
-/* Workgroup size (64, 128, 192 or 256 threads) of each kernel class of a context. */
+/* Workgroup size (64, 128, 192 or 256 threads) of each kernel class of a context. Until this or
+ * the autotuner sets the sizes, batches of fewer than 1024 waves (columns / 64) use 64 in every
+ * class; afterwards every batch uses the sizes set. Not sized by it: CRM_K_SETUP,
+ * CRM_K_SETPERTURB, CRM_K_PRECIP_INIT, CRM_K_PRESS, CRM_K_PRECIP where its levels are dealt to the
+ * waves of a workgroup (fewer than 1024 waves), and 128-column CRMs (a workgroup per instance). */
 int crm_hip_set_schedule(crm_hip_ctx *ctx, const int block[CRM_HIP_NKERNEL]);
 int crm_hip_get_schedule(const crm_hip_ctx *ctx, int block[CRM_HIP_NKERNEL]);
 
 /* Launch variant ("tile shape") of each kernel class of a context, 0 the default; results are
- * bitwise the same in every variant. CRM_K_PRESS of 2D 64-column CRMs: an
- * instance on a workgroup of 8 waves (0, 1), 4 (2, 3) or 16 (4), with four (0, 2) or two (1, 3, 4)
- * levels of each wave loaded together. CRM_K_MPDATA (each scalar on its own waves): 0 chosen by the batch's size (small batches deal
- * the levels to several workgroups; large ones take 2 at 64 columns in 2D, else 4), 1 the other
- * number of levels per trip of the sweep's steady state than the default (two for 2D 64-column
- * CRMs, else one), 2 and 3 the default and 1 with the registers bounded for three waves per SIMD,
- * 4 the default with unbounded registers, 5 as 2. Other classes have variant 0 only. */
+ * bitwise the same in every variant. CRM_K_PRESS of 2D 64-column CRMs: an instance on a workgroup
+ * of 8 waves (0, 1), 4 (2, 3) or 16 (4), with four (0, 2) or two (1, 3, 4) levels of each wave
+ * loaded together. CRM_K_MPDATA (each scalar on its own waves): 0 chosen by the batch's size: below
+ * 1024 waves the levels are dealt to several workgroups, and with them those of the sedimentation
+ * and the diffusion; above, 2 at 64 columns in 2D from 2048 waves on, else 4. The others sweep all
+ * levels at every size: 2 with registers bounded for three waves per SIMD, 4 unbounded, both with
+ * the default number of levels per trip (two for 2D 64-column CRMs, else one); 3 and 1 the same
+ * with the other number; 5 as 2. Other classes have variant 0 only. */
 int crm_hip_set_variants(crm_hip_ctx *ctx, const int variant[CRM_HIP_NKERNEL]);
 int crm_hip_get_variants(const crm_hip_ctx *ctx, int variant[CRM_HIP_NKERNEL]);
 
 /* Autotuner: runs the call once per candidate workgroup size (64, 128, 256) and launch variant,
- * with every kernel class timed on the context's stream, keeps the fastest (size, variant) of
- * each class (the default threads - 256, for CRM_K_MICRO in FP64 64 - and variant 0
- * unless another is faster by more than 3%)
- * for later calls of this context and writes the sizes to block_out (may be NULL;
+ * that this batch launches differently (below 1024 waves of MPDATA variant 0 only), with every
+ * kernel class timed on the context's stream, keeps the fastest (size, variant) of each class
+ * (the default threads - 256, for CRM_K_MICRO in FP64 64, below 1024 waves 64 - and variant 0
+ * unless another is faster by more than 3%) for later calls of this context and writes the sizes to block_out (may be NULL;
  * crm_hip_get_variants gives the variants). The views are device pointers and are advanced by
  * every trial call: pass scratch copies. */
 int crm_hip_autotune(crm_hip_ctx *ctx, const crm_dims *dims, const crm_column_info *col, double dt_gl,

@@ -77,6 +77,13 @@ long long crm_hip_graph_launches(const crm_hip_ctx *ctx);
 /* Number of captured graphs the context holds (at most 32; least recently used first out). */
 int crm_hip_graph_cache_size(const crm_hip_ctx *ctx);
 
+/* What a call of these dimensions launches for kernel class kid with the context's schedule and
+ * variants: shape[0] threads per workgroup (0 where the schedule does not size the class), shape[1]
+ * chunks its levels are dealt to, shape[2] 1 where MPDATA, the sedimentation and the diffusion
+ * hand the scalars on through other buffers, shape[3] the variant (CRM_K_MPDATA: 1 for the other
+ * number of levels per trip, plus 2 for bounded registers). Launches nothing. */
+int crm_hip_launch_shape(const crm_hip_ctx *ctx, const crm_dims *dims, int kid, int shape[4]);
+
 /* Test hook: a captured call (CRM_GRAPHS_CALL) stops at substep nstep (1-based) as if it needed
  * more subcycles, and the host resumes it there; 0 turns the hook off. */
 int crm_hip_debug_stop_call_at(crm_hip_ctx *ctx, int nstep);
