@@ -12,6 +12,7 @@ cpu_baseline leg of bench.py import this module.
 import ctypes as C
 import os
 import sys
+import unittest
 
 import numpy as np
 
@@ -63,9 +64,17 @@ class _Runner:
         return buf[:n]
 
 
+class ReferenceMissing(FileNotFoundError, unittest.SkipTest):
+    """The reference is not built for a size class (its tree is not there): a test that needs it is
+    skipped, as a missing file elsewhere."""
+
+
 def reference(case):
     """Reference CRM (compiled reference phases + harness) for case's size class."""
-    return _Runner(ref_so_path(case), "ref_crm", "ref_get")
+    path = ref_so_path(case)
+    if not os.path.exists(path):
+        raise ReferenceMissing(path)
+    return _Runner(path, "ref_crm", "ref_get")
 
 
 def reference_set_coriolis(case, on):
