@@ -90,12 +90,13 @@ struct Engine : CrmEngine {
   double acc_factor = 0.0;
   // launch schedule: threads per workgroup of each segment-kernel class (a multiple of 64 up
   // to 256; instances per workgroup = block / columns).  Until the caller or the autotuner sets it
-  // (sized), batches of fewer waves than the device has SIMDs use 64.  k_micro of the
-  // FP64 engine starts with 64: its waves end at different times, and a workgroup keeps its
-  // registers until the last (4096 x 64 x 58: 588 us with 256, 476 with 128, 454 with 64; 1024 x 64
-  // x 58: 150, 127, 126).  Mixed 246, 234, 232, but gathering the next kurant maximum it is
-  // slower (a call 431 ms with 256, 437 with 64).  The other sweeps are within 5% of 256 or slower.
-  static constexpr int MICRO_BLOCK = sizeof(R) == 8 ? 64 : 256;
+  // (sized), batches of fewer waves than the device has SIMDs use 64.  k_micro starts with fewer:
+  // its waves end at different times, and a workgroup keeps its registers until the last.  A call
+  // of 4096 x 64 x 58 with 64, 128 and 256 threads (the gathering k_micro in two pieces, Launcher::
+  // chunks): where a third of the instances convect FP64 766, 771 and 801 ms, mixed 425, 425 and
+  // 429; quiet soundings FP64 731, 731 and 728, mixed 408, 406 and 405.  The other sweeps are
+  // within 5% of 256 or slower.
+  static constexpr int MICRO_BLOCK = sizeof(R) == 8 ? 64 : 128;
   static constexpr int DEFAULT_BLOCK[CRM_K_COUNT] = {256, 256, 256, 256, 256, 256, 256,         256,
                                                      256, 256, 256, 256, MICRO_BLOCK, 256, 256};
   int block[CRM_K_COUNT];
@@ -560,8 +561,12 @@ struct Launcher {
   // idle wave slots: to about `fill` waves in all, measured at 16 to 866 x 32 x 28, 256 x 128 x
   // 58, 500 x 64 x 58, 1024 x 4 x 4 x 28 and 333 x 8 x 8 x 40 for fills of 1024 to 16384.
   // k_micro's levels are independent and uneven (a cloudy level takes a Newton iteration and
-  // powers), so smaller pieces also balance a full device: 4096 x 64 x 58 FP64 568 us in one
-  // piece, 462 in two, 442 in four (mixed 293, 271, 243).
+  // powers), so smaller pieces also balance a full device; but each piece of a queued call adds its
+  // own maximum to the 32 slots of the next kurant number, and where nothing is cloudy only that
+  // shows.  A call of 4096 x 64 x 58 FP64 in 1, 2 and 4 pieces: a third of the instances convecting
+  // 792, 766 and 770 ms, quiet soundings 726, 731 and 738 (mixed, 128 threads: 431, 425 and 426,
+  // quiet 408, 406 and 412); 1024 x 64 x 58 FP64 in 2, 4 and 8: 234, 213 and 209, quiet 197, 197
+  // and 201.
   int chunks(int kid) const {
     int fill, least;  // waves aimed at, fewest levels per chunk
     switch (kid) {
@@ -572,7 +577,7 @@ struct Launcher {
       case CRM_K_MPDATA: fill = 1024, least = 4; break;  // waves per scalar
       case CRM_K_PRECIP: fill = 2048, least = 4; break;
       case CRM_K_DIFFUSE: fill = 4096, least = 2; break;
-      case CRM_K_MICRO: fill = std::max(8192, 4 * waves()), least = 1; break;
+      case CRM_K_MICRO: fill = std::max(8192, 2 * waves()), least = 1; break;
       case CRM_K_STATS: fill = 2048, least = 2; break;
       case CRM_K_FINAL: fill = std::max(8192, 2 * waves()), least = 1; break;
       default: return 1;

@@ -242,11 +242,12 @@ int crm_hip_get_schedule(const crm_hip_ctx *ctx, int block[CRM_HIP_NKERNEL]);
 int crm_hip_set_variants(crm_hip_ctx *ctx, const int variant[CRM_HIP_NKERNEL]);
 int crm_hip_get_variants(const crm_hip_ctx *ctx, int variant[CRM_HIP_NKERNEL]);
 
-/* Autotuner: runs the call once per candidate workgroup size (64, 128, 256) and launch variant,
+/* Autotuner: runs the call once per candidate workgroup size (64, 128, 256) and launch variant
  * that this batch launches differently (below 1024 waves of MPDATA variant 0 only), with every
- * kernel class timed on the context's stream, keeps the fastest (size, variant) of each class
- * (the default threads - 256, for CRM_K_MICRO in FP64 64, below 1024 waves 64 - and variant 0
- * unless another is faster by more than 3%) for later calls of this context and writes the sizes to block_out (may be NULL;
+ * kernel class timed on the context's stream, and keeps the fastest (size, variant) of each class
+ * for later calls of this context. The default stays unless another is faster by more than 3%:
+ * variant 0 and 256 threads, for CRM_K_MICRO 64 in FP64 and 128 in mixed precision, below 1024
+ * waves 64 for every class. The sizes are written to block_out (may be NULL;
  * crm_hip_get_variants gives the variants). The views are device pointers and are advanced by
  * every trial call: pass scratch copies. */
 int crm_hip_autotune(crm_hip_ctx *ctx, const crm_dims *dims, const crm_column_info *col, double dt_gl,

@@ -7,6 +7,7 @@ import pytest
 
 from crm_hip import KERNELS, CrmHip, DeviceCase
 from crm_inputs import add_convection, make_case
+from crm_views import CrmDims
 from test_gpu_chunks import repeated
 
 pytestmark = pytest.mark.gpu
@@ -64,6 +65,14 @@ def test_mpdata_variants_are_the_ones_launched(shape, prec):
             _, chunks, split, got = hip.launch_shape(case.dims(), "mpdata")
             assert got == kind and split == (small and v == 0) and (split or chunks == 1)
             _same(ref, _run(hip, case, 3))
+
+
+def test_pieces_of_the_microphysics():
+    """A full device takes two pieces per wave of columns (each adds an atomic maximum to the queued
+    call), a smaller batch as many as give 8192 waves."""
+    with CrmHip(0) as hip:
+        for n, pieces in ((8192, 2), (4096, 2), (4095, 2), (2048, 4), (1024, 8), (64, 58)):
+            assert hip.launch_shape(CrmDims(n, n, 60, 64, 1, 58, 16, 1, 1000.0, 5.0), "micro")[1] == pieces
 
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
