@@ -36,7 +36,8 @@ ABI_SYMBOLS = ["crm_hip_init", "crm_hip_run", "crm_hip_run_device", "crm_hip_run
 DEBUG_SYMBOLS = ["crm_hip_debug_run", "crm_hip_debug_get", "crm_hip_fft991_operators",
                  "crm_hip_profile_kernels", "crm_hip_kernel_time", "crm_hip_kernel_name",
                  "crm_hip_graph_launches", "crm_hip_graph_cache_size",
-                 "crm_hip_debug_stop_call_at", "crm_hip_launch_shape"]
+                 "crm_hip_debug_stop_call_at", "crm_hip_launch_shape",
+                 "crm_hip_queue_counts"]
 # Kernel classes of one call (CRM_K_* of include/crm_hip_debug.h), in launch order.
 KERNELS = ["setup", "init", "setperturb", "kurant", "precip_init", "pre", "sgs", "mom", "press",
            "mpdata", "precip", "diffuse", "micro", "stats", "final"]
@@ -103,6 +104,7 @@ def load():
     lib.crm_hip_set_graphs.argtypes = [P, C.c_int]
     lib.crm_hip_debug_stop_call_at.argtypes = [P, C.c_int]
     lib.crm_hip_launch_shape.argtypes = [P, C.POINTER(CrmDims), C.c_int, C.c_int * 4]
+    lib.crm_hip_queue_counts.argtypes = [P, C.c_longlong * 2]
     lib.crm_hip_graph_launches.argtypes = [P]
     lib.crm_hip_graph_launches.restype = C.c_longlong
     lib.crm_hip_graph_cache_size.argtypes = [P]
@@ -261,6 +263,12 @@ class CrmHip:
 
     def graph_launches(self):
         return int(self.lib.crm_hip_graph_launches(self.ctx))
+
+    def queue_counts(self):
+        """(launched, run by the device) substeps of accelerated calls queued without the host."""
+        a = (C.c_longlong * 2)()
+        self.lib.crm_hip_queue_counts(self.ctx, a)
+        return a[0], a[1]
 
     def graph_cache_size(self):
         return int(self.lib.crm_hip_graph_cache_size(self.ctx))

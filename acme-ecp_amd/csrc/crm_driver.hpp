@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -17,6 +18,7 @@
 #include <map>
 #include <string>
 #include <type_traits>
+#include <thread>
 #include <vector>
 
 #include "../../include/crm_hip.h"
@@ -45,6 +47,7 @@ struct HostTransform {
 enum { NSCAL = 17 };  // u t qt qp qn tabs qv qcl qci qpl qpi tk tkh tke dudt x3
 enum { NSCAL3 = 4 };  // 3D only: v dvdt x3
 enum { NPOOL = 9 };  // blocks of the field pool (pool_sizes)
+constexpr int QUEUE_AHEAD = 4;   // substeps of an accelerated call queued ahead of the device
 constexpr int MAX_VARIANTS = 6;  // launch variants of a kernel class (variants_of)
 
 }  // namespace
@@ -128,6 +131,10 @@ struct Engine : CrmEngine {
   static constexpr size_t GRAPH_CACHE_MAX = 32;
   std::list<std::string> graph_lru;  // most recently used first
   long long graph_launches = 0;
+  // substeps of accelerated calls that were queued, and that ran from the queue; the substep the
+  // device last decided on in such a call (pinned host memory)
+  long long queue_launched = 0, queue_ran = 0;
+  unsigned long long* progress = nullptr;
   void drop_graphs() {
     if (!graphs.empty() && stream) (void)hipStreamSynchronize(stream);
     for (auto& kv : graphs) (void)hipGraphExecDestroy(kv.second);
@@ -210,6 +217,7 @@ struct Engine : CrmEngine {
     drop_graphs();
   }
   long long graph_count() const override { return graph_launches; }
+  void queue_counts(long long counts[2]) const override { counts[0] = queue_launched, counts[1] = queue_ran; }
   hipStream_t get_stream() const override { return stream; }
   int set_mlp(const crm_mlp* m) override {
     if (m && crm_mlp_ns::mlp_device(m) != device) return CRM_ERR_ARG;
@@ -956,6 +964,9 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
   // of its bookkeeping before it (slot rotation, buffer swaps, Adams-Bashforth history).  A call
   // with mean-state acceleration queues the same sequence launch by launch: the host's read of
   // the maximum and the flag every substep left the device idle for 45 us of 600 (500 x 64 x 58).
+  // The host then stays QUEUE_AHEAD substeps ahead of the device, so that a call that stops leaves
+  // few empty launches behind: queued to its end, one that stopped at its first substep took 0.5 to
+  // 1 ms of 3 to 6 longer at 16 x 32 x 28, 1.6 to 5 of 35 to 70 at 500 x 64 x 58.
   if (ctx->use_graphs >= CRM_GRAPHS_CALL && !sc && !net_inputs && ctx->prof_mask == 0 && phase_stop == 0 &&
       nstop <= 2048) {
     struct Snap {
@@ -977,9 +988,23 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
     key.append((const char*)ctx->block, sizeof(ctx->block));
     key.append((const char*)ctx->variant, sizeof(ctx->variant));
     key.push_back((char)ctx->sized);
+    // Waits until the device has decided on substep n; false when it has stopped the call.  The
+    // wait ends by itself (a device that no longer answers is found at the call's next
+    // synchronization).
+    auto decided = [&](int n) {
+      const volatile unsigned long long* p = ctx->progress;
+      const auto t0 = std::chrono::steady_clock::now();
+      while (!(*p & QUEUE_STOPPED) && *p < (unsigned long long)n) {
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1)) break;
+        std::this_thread::yield();
+      }
+      return !(*p & QUEUE_STOPPED);
+    };
     // the call's sequence; with launch false only the host bookkeeping is replayed
     auto sequence = [&](bool launch) {
       for (int n = 1; n <= nstop; n++) {
+        if (acc && n > QUEUE_AHEAD && !decided(n - QUEUE_AHEAD)) break;
+        if (acc) ctx->queue_launched++;
         snap[n] = Snap{na, nb, nc, d, {dt3[0], dt3[1], dt3[2]}};
         d.nstep = n;
         d.icycle = 1;
@@ -995,7 +1020,8 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
           // slots for the next (the last substep's maximum is not read)
           if (n == 1) k_clear_u64<<<1, 64, 0, s>>>(gmax + GMAX_FLAGS, d.stop);
           if (n == 1 || acc) NX_DISPATCH(nx, (k_kurant<NXV, R><<<L.g(CRM_K_KURANT), L.b(CRM_K_KURANT), 0, s>>>(d)));
-          k_precip_init<R, true><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128) + 1), dim3(128), 0, s>>>(d, ctx->debug_stop);
+          k_precip_init<R, true><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128) + 1), dim3(128), 0, s>>>(
+              d, ctx->debug_stop, acc ? ctx->progress : nullptr);
           NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad)));
           NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
           NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
@@ -1028,6 +1054,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
     if (acc) {
       rc = arrival.alone();
       if (rc) return rc;
+      *(volatile unsigned long long*)ctx->progress = 0;
       sequence(true);
       HIPCHECK(hipGetLastError());
     } else if (jc) {  // one graph with the other classes of crm_hip_run_many
@@ -1067,6 +1094,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       nstep = (int)stopped_at - 1;
       if (!acc) ctx->graph_launches -= nstop - nstep;
     }
+    if (acc) ctx->queue_ran += nstep;
     if (nstep >= 1) ctx->stats.ncycle_max = std::max(ctx->stats.ncycle_max, 1);
     d.stop = nullptr;
   }
@@ -1115,7 +1143,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       d.dt3na = dt3[na];
       const double* qrad = qrad_buf;
       auto body = [&]() {
-        k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d, 0);
+        k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d, 0, nullptr);
         NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad)));
         NX_DISPATCH(nx, (k_sgs<NXV, R, GEO><<<L.g(CRM_K_SGS), L.b(CRM_K_SGS), 0, s>>>(d)));
         NX_DISPATCH(nx, (k_mom<NXV, R, GEO><<<L.g(CRM_K_MOM), L.b(CRM_K_MOM), 0, s>>>(d, na)));
@@ -1177,7 +1205,7 @@ static int run_core(Engine<R>* ctx, const crm_dims* dm, const crm_column_info* c
       d.dt3na = dt3[na];
       if (icyc == 1)
         TIMED(CRM_K_PRECIP_INIT,
-              (k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d, 0)));
+              (k_precip_init<R><<<dim3((unsigned)(((size_t)ncrms * nzm + 127) / 128)), dim3(128), 0, s>>>(d, 0, nullptr)));
       const double* qrad = qrad_buf;
       TIMED(CRM_K_PRE, NX_DISPATCH(nx, (launch_pre<NXV, R>(L, d, na, qrad))));
       if (last && phase_stop == 7) goto stopped;
@@ -1394,6 +1422,7 @@ Engine<R>::~Engine() {
   if (lat_dev) (void)hipFree(lat_dev);
   for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
   if (ev0) (void)hipEventDestroy(ev0);
+  if (progress) (void)hipHostFree(progress);
   if (ev_ready) (void)hipEventDestroy(ev_ready);
   if (ev1) (void)hipEventDestroy(ev1);
   if (stream) (void)hipStreamDestroy(stream);
@@ -1633,7 +1662,8 @@ static CrmEngine* make_engine(int device, int* rc) {
   e->device = device;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&e->stream) != hipSuccess ||
       hipEventCreate(&e->ev0) != hipSuccess || hipEventCreate(&e->ev1) != hipSuccess ||
-      hipMalloc(&e->gmax, GMAX_WORDS * sizeof(unsigned long long)) != hipSuccess) {
+      hipMalloc(&e->gmax, GMAX_WORDS * sizeof(unsigned long long)) != hipSuccess ||
+      hipHostMalloc(&e->progress, sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
     delete e;
     *rc = CRM_ERR_DEVICE;
     return nullptr;

@@ -314,6 +314,12 @@ int crm_hip_get_schedule(const crm_hip_ctx* ctx, int block[CRM_HIP_NKERNEL]) {
   return CRM_OK;
 }
 
+int crm_hip_queue_counts(const crm_hip_ctx* ctx, long long counts[2]) {
+  if (!ctx || !ctx->eng || !counts) return CRM_ERR_ARG;
+  ctx->eng->queue_counts(counts);
+  return CRM_OK;
+}
+
 int crm_hip_launch_shape(const crm_hip_ctx* ctx, const crm_dims* dims, int kid, int shape[4]) {
   if (!ctx || !ctx->eng || kid < 0 || kid >= CRM_K_COUNT || !shape) return CRM_ERR_ARG;
   return ctx->eng->launch_shape(dims, kid, shape);

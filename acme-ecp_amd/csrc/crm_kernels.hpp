@@ -57,8 +57,11 @@ __global__ void k_zero_u64(unsigned long long* __restrict__ p, size_t n) {
 // of substep nstep's first kernel: one subcycle when cfl / 0.7 <= 1; anything else (more
 // subcycles, the reference's abort, a non-finite value) stops the queued call at this substep for
 // the host to take over; so does the acceleration's 5 K flag (gmax[3]), and nstep == stop_at (a
-// test hook, 0 when off).  The maximum's slots are cleared for the next one gathered.
-__device__ __forceinline__ void decide(unsigned long long* gmax, int nstep, int stop_at) {
+// test hook, 0 when off).  The maximum's slots are cleared for the next one gathered.  progress
+// (host memory, may be null): the substep decided on, with QUEUE_STOPPED where it stops the call.
+constexpr unsigned long long QUEUE_STOPPED = 1ull << 63;
+__device__ __forceinline__ void decide(unsigned long long* gmax, int nstep, int stop_at,
+                                       unsigned long long* progress) {
   const int l = threadIdx.x & 63;
   unsigned long long* slot = gmax + GMAX_FLAGS + (l & (KURANT_SLOTS - 1)) * KURANT_STRIDE;
   unsigned long long cbits = *slot;
@@ -67,11 +70,15 @@ __device__ __forceinline__ void decide(unsigned long long* gmax, int nstep, int 
     cbits = o > cbits ? o : cbits;
   }
   const double q = __longlong_as_double((long long)cbits) / (double)0.7f;
-  if (!(q <= 1.0) || nstep == stop_at || gmax[3]) {
+  const bool stops = !(q <= 1.0) || nstep == stop_at || gmax[3];
+  if (stops) {
     if (l == 0) gmax[GMAX_STOP] = (unsigned long long)nstep;
   } else if (l < KURANT_SLOTS) {
     *slot = 0ull;
   }
+  if (progress && l == 0)
+    __hip_atomic_store(progress, (unsigned long long)nstep | (stops ? QUEUE_STOPPED : 0ull), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2327,11 +2334,11 @@ __global__ void CRM_LB k_diffuse(DevT<R> d, Scalars<R> src) {
 // these coefficients with it.
 // ------------------------------------------------------------------------------------------
 template <typename R, bool DECIDE = false>
-__global__ void k_precip_init(DevT<R> d, int stop_at) {
+__global__ void k_precip_init(DevT<R> d, int stop_at, unsigned long long* progress) {
   CRM_STOP_CHECK(d);
   if constexpr (DECIDE) {
     if (blockIdx.x == gridDim.x - 1) {
-      if (threadIdx.x < 64) decide(d.gmax, d.nstep, stop_at);
+      if (threadIdx.x < 64) decide(d.gmax, d.nstep, stop_at, progress);
       return;
     }
   }

@@ -74,6 +74,11 @@ const char *crm_hip_kernel_name(int kid);
 /* Number of substeps replayed from captured graphs since the context was created. */
 long long crm_hip_graph_launches(const crm_hip_ctx *ctx);
 
+/* Substeps of calls with mean-state acceleration since the context was created: counts[0] launched
+ * without the host's decision, counts[1] of those that the device ran. The others were launched
+ * behind the substep at which the device stopped the call, and returned at entry. */
+int crm_hip_queue_counts(const crm_hip_ctx *ctx, long long counts[2]);
+
 /* Number of captured graphs the context holds (at most 32; least recently used first out). */
 int crm_hip_graph_cache_size(const crm_hip_ctx *ctx);
 
