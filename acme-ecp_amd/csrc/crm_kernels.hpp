@@ -2493,18 +2493,13 @@ __device__ __forceinline__ void diagnose_level(const DevT<R>& d, const S_& s, in
   }
 }
 
-// The instance's cloud-ice level range from this workgroup's levels.  The chunks of an instance
-// extend the range that k_diffuse emptied: kmin is not negative, so it orders as its bits, and so
-// does kmax >= -1 as signed bits.
+// The instance's cloud-ice level range from this workgroup's levels.  The chunks of an instance (at
+// least two, Launcher::chunks) extend the range that k_diffuse emptied: kmin is not negative, so it
+// orders as its bits, and so does kmax >= -1 as signed bits.
 template <typename R>
 __device__ __forceinline__ void ice_range(const DevT<R>& d, int c, int kmin, int kmax) {
-  if (gridDim.y == 1) {
-    inst(d, I_KMIN, c) = kmin;
-    inst(d, I_KMAX, c) = kmax;
-  } else {
-    atomicMin((unsigned long long*)&inst(d, I_KMIN, c), (unsigned long long)__double_as_longlong((double)kmin));
-    atomicMax((long long*)&inst(d, I_KMAX, c), __double_as_longlong((double)kmax));
-  }
+  atomicMin((unsigned long long*)&inst(d, I_KMIN, c), (unsigned long long)__double_as_longlong((double)kmin));
+  atomicMax((long long*)&inst(d, I_KMAX, c), __double_as_longlong((double)kmax));
 }
 
 // The level means of accelerate_crm.F90:196-250 after micro_proc, minus those of the last

@@ -136,7 +136,7 @@ __device__ __forceinline__ void blocks(const bf16* W, const s4 (&in)[KB], f4 (&a
 // tiles, and the four waves share the 144 16 x 16 gradient blocks, whose accumulators stay in
 // registers over the workgroup's tiles.  109 KB of LDS: one workgroup per CU, and a grid of at
 // most one per CU.  Bound by latency: 424 MFMAs per wave and tile are 3 us at the matrix rate; the
-// shares (142 KB per workgroup, written here and read by k_reduce) are 73 MB at 256 workgroups.
+// shares (141 KB per workgroup) are 36 MB at 256 workgroups, written here and read by k_reduce.
 __global__ void __launch_bounds__(256) k_train(const float* X, const float* T, int n, Weights w, const float* norm,
                                                float* part) {
   __shared__ __attribute__((aligned(16))) bf16 sX[KP][TLD], sH[3][NH][TLD], sY[NP][TLD], sD[3][NH][TLD];
