@@ -1278,7 +1278,7 @@ __global__ void CRM_LB k_mom(DevT<R> d, int na) {
 // 1024 x 4x4 x 28 36 -> 24, 500 x 64 x 58 75 -> 65, 4096 x 64 x 58 535 -> 508 and mixed 345 -> 295.
 // Bound: memory, in phases.  The registers of the batched loads allow two workgroups of a CU, so
 // the transforms and the sweep of one are covered by the loads and stores of one other; at 4096
-// instances a launch moves 22 words per cell (8 of them again, for the gradient) at 2.5 TB/s.
+// instances a launch moves 22 words per cell (8 of them again, for the gradient) at 5.4 TB/s.
 //
 // The Thomas sweep runs on one wave (128 columns: two), lane = slot, its factors in LDS.  The
 // level coefficients do not depend on the recurrence: all waves compute them before it, and the
