@@ -61,6 +61,8 @@ CrmOutputView = _struct("CrmOutputView", OUT_ORDER)
 def _ptr(a):
     if a is None:
         return c_dp()
+    if isinstance(a, int):        # a raw address
+        return C.cast(C.c_void_p(a), c_dp)
     assert a.dtype == np.float64 and a.flags["F_CONTIGUOUS"]
     return a.ctypes.data_as(c_dp)
 
@@ -120,11 +122,16 @@ class CrmCase:
 def _struct_at(cls, order, addr):
     """A view struct over raw addresses (integers, None for a null pointer).  The struct is made
     of its bytes: converting some 90 addresses of a call to pointer objects one by one took 90 us,
-    more than most of the kernels it is made for."""
-    return cls.from_buffer_copy(struct.pack("%dP" % len(order), *[addr[f] or 0 for f in order]))
+    more than most of the kernels it is made for.  Where a member is an array it is done so all the
+    same."""
+    values = [addr[f] for f in order]
+    try:
+        return cls.from_buffer_copy(struct.pack("%dP" % len(order), *[0 if v is None else v for v in values]))
+    except (struct.error, TypeError):
+        return cls(*[_ptr(v) for v in values])
 
 
 def views_from_addresses(inp, state, rad, out):
-    """Views over device arrays given as dicts name -> integer address."""
+    """Views over arrays given as dicts name -> integer address (or host array, or None)."""
     return (_struct_at(CrmInputView, INPUT_ORDER, inp), _struct_at(CrmStateView, STATE_ORDER, state),
             _struct_at(CrmRadView, RAD_ORDER, rad), _struct_at(CrmOutputView, OUT_ORDER, out))
